@@ -69,11 +69,16 @@ namespace g16 {
 namespace {
 
 constexpr int kGroupM = 8;
+// Direct A runs few tile columns (direct_route): with 8 tile rows to a group, a group of 3 columns is
+// not a divisor of an XCD's 32 workgroups, and rows of x are read again in the next round (65536 x
+// 3072 x 768: 377 us; 339 with 1 or 2 rows to a group, 348 with 4; packed A within 2 % either way).
+constexpr int kDirectGroupM = 2;
 constexpr int kSplitAlign = 64;  // split-K slices start on a multiple of every tile's K step
 // The planner's rule (M <= 64) splits no K below this: two slices of 256 cost more than they save
 // (graph-timed: 16 x 8192 x 512 (M x N x K) 6.0 us unsplit, 7.1 split twice; 48 x 2048 x 512 6.2
 // vs 7.2); at K = 1024 four slices win (64 x 1024^2 7.7 -> 7.1).
 constexpr int kMinSplitK = 1024;
+constexpr float kHalfMax = 65504.f;  // largest finite fp16
 constexpr uint32_t kOob = 0x80000000u;  // buffer offset past every descriptor's range: reads 0
 
 typedef short short4v __attribute__((ext_vector_type(4)));
@@ -241,8 +246,11 @@ __device__ inline void phase_barrier() { asm volatile("s_barrier" ::: "memory");
 // workgroup; split, by the slice that arrives last, over every slice in slice order. A split
 // slice that saw such a value publishes its rows' |max| in place of its partial tile. A tile that
 // is computed again stores 1 into *spec_miss (when not NULL; pinned host memory).
+// DIRECT: A is unused; the kernel streams the fp32 activations X through registers, casts them on the
+// way into the A stages and rescales a row as soon as a value of it leaves fp16's range (the 256x256
+// tile, unsplit).
 template <class Cfg, bool OUT_F16, bool SPLITK, bool PACKED_A = false, bool PACKED_B = false, bool RESIDENT = false,
-          bool SPEC = false>
+          bool SPEC = false, bool DIRECT = false>
 __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                                                          void* __restrict__ Cv, const float* __restrict__ bias,
                                                          const float* __restrict__ rscale, float* __restrict__ part,
@@ -256,11 +264,19 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
                 "resident A: the unsplit 32x128 tile");
   static_assert(!SPEC || (Cfg::WAVES == 4 && !Cfg::MF16 && !PACKED_A && !PACKED_B && !RESIDENT),
                 "speculative A: the 4-wavefront tiles, 32x32x16 blocks (lane l's A rows are l % 32)");
+  static_assert(!DIRECT || (Cfg::WAVES == 8 && Cfg::BK == 32 && Cfg::MF16 && !SPLITK && !PACKED_A && !RESIDENT && !SPEC),
+                "direct A: the unsplit 8-wavefront tiles");
   constexpr int A_STAGES = RESIDENT ? kResidentSteps : NSTAGE;
   __shared__ __attribute__((aligned(1024))) unsigned char sA[A_STAGES][Cfg::A_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char sB[NSTAGE][Cfg::B_BYTES];
   __shared__ float s_scale[(RESIDENT || SPEC) ? BM : 1];
   __shared__ float s_rowmax[SPEC ? BM : 1];  // speculative recomputation: the rows' |max|, then 2^-e
+  // direct A: the factors 2^-e of the rows' exponents so far (0 for an infinite row); per ring stage
+  // and staging wavefront, the K step whose A raised an exponent, and that step's factors for the
+  // wavefront's rows
+  __shared__ float s_fac[DIRECT ? BM : 1];
+  __shared__ int s_evt[DIRECT ? NSTAGE : 1][DIRECT ? Cfg::WAVES : 1];
+  __shared__ __attribute__((aligned(16))) float s_delta[DIRECT ? NSTAGE : 1][DIRECT ? BM : 4];
   const uint32_t sA_lds = lds_base(&sA[0][0]), sB_lds = lds_base(&sB[0][0]);
 
   // ---- tile assignment (XCD-aware, grouped) ----
@@ -284,9 +300,10 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       const int xcd = lin % 8, q8 = ntiles / 8, r8 = ntiles % 8;
       lin = xcd * q8 + min(xcd, r8) + lin / 8;  // XCD x holds q8 + (x < r8) workgroups
     }
-    const int per_group = kGroupM * ntn;
-    const int first_m = (lin / per_group) * kGroupM;
-    const int gsz = min(ntm - first_m, kGroupM);
+    constexpr int kGroup = DIRECT ? kDirectGroupM : kGroupM;
+    const int per_group = kGroup * ntn;
+    const int first_m = (lin / per_group) * kGroup;
+    const int gsz = min(ntm - first_m, kGroup);
     const int tm = first_m + (lin % per_group) % gsz;
     const int tn = (lin % per_group) / gsz;
     const int tile = tm * ntn + tn;
@@ -334,7 +351,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
         // whole 16 KB blocks; a 128-column tile streams one half of each: rows 0-127 of a block are
         // its first 8 KB (chunks q < 8), rows 128-255 the second, each already the 128-row stage
         // image (the row swizzle repeats every 8 rows). Step k0 adds k0/BK blocks (16 KB) either way.
-        static_assert(PACKED_A && (Cfg::BN == 256 || Cfg::BN == 128), "packed weight: the 256-row tiles");
+        static_assert((PACKED_A || DIRECT) && (Cfg::BN == 256 || Cfg::BN == 128), "packed weight: the 256-row tiles");
         constexpr int kHalves = 256 / Cfg::BN;
         return __builtin_amdgcn_make_buffer_rsrc(
             const_cast<_Float16*>(B) + static_cast<size_t>(tn / kHalves) * ceil_div(K, BK) * 8192 + (tn % kHalves) * 4096, 0,
@@ -679,41 +696,282 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       // that phase publishes it to the group that reads next.
       constexpr int D = NSTAGE - 2;
       const int grp = wave >> 2;
-      if (nk > 0) {
+      if constexpr (DIRECT) {
+        // Direct A. Per K step a wavefront stages 32 rows x 32 fp32 values: load i of a lane is 16 bytes
+        // of row 8 i + lane / 8 (8 lanes cover one row's 128 bytes, a cache line; 16-byte pieces 32
+        // bytes apart, which would make the LDS writes 16 bytes wide, took 365 us where this takes 340,
+        // at 65536 x 3072 x 768). Two register sets alternate, so a step's loads have two steps to land: M_j casts the set of step j + 2 into its stage (whose
+        // last readers finished before M_j, as for the DMA above) and then refills the set with step
+        // j + 4. The compiler places the loads' waits; it does not count the asm DMA of B, so B's DMA
+        // of step j + 2 is issued between the cast and the refill: then only the 4 loads of step j + 3
+        // are younger than B's DMA of step j + 1, and the wait for step j + 2's loads (at most those 4
+        // outstanding) covers that DMA too, which every wavefront needs before the barrier that ends
+        // M_j. The LDS writes are complete before the barrier that ends C_j, which precedes M_{j+2} of
+        // either group.
+        //   Rescaling. The cast of a value past fp16's range is infinite; M_j takes the largest |x| it
+        // casts along, and C_j begins by looking at it. If a row has such a value, the wavefront reads
+        // its 8-row group of the step's values again, raises the row's exponent so that the largest lands at most at the
+        // threshold (the rowscale cast's rule, on what the row has shown so far), writes the scaled
+        // values over the stage, and leaves the factor for the accumulators, which every wavefront
+        // applies before its MFMAs of that step. Later steps of the row are scaled as they are cast.
+        //   M_j has little room: with ~100 instructions (address arithmetic mostly) it set the pace, 1570
+        // shader cycles per step at 4096^3 against 1054 with packed A. So the loop is unrolled over the
+        // ring (every LDS address is an immediate) and the descriptors' ranges and the scalar offset,
+        // which the range check includes, replace per-step masks and pointers.
+        constexpr int NL = BM * BK * 4 / 16 / Cfg::THREADS;
+        static_assert(NL == 4 && BM / Cfg::WAVES == 32 && Cfg::B_INSTR == 2 && NSTAGE == 4,
+                      "4 loads of 8 rows and two DMA instructions per wavefront and step");
+        const int dr0 = wave * 32 + (lane >> 3), dc = lane & 7;  // this lane's first row, its 4-value chunk
+        // X from this tile's first row on; loads past its last row give 0. A step past K reads what
+        // follows (the next row): its stage is never multiplied. Columns past K in the last step of a
+        // K that is no multiple of BK are masked by the lane's offset.
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(static_cast<const float*>(X) + static_cast<size_t>(m0) * K), 0,
+            static_cast<int>(min(static_cast<long>(M - m0), static_cast<long>(BM)) * K * 4), kRawBufferDword3);
+        const uint32_t voff = static_cast<uint32_t>((dr0 * K + dc * 4) * 4);
+        const uint32_t tail = (nk - 1) * BK + dc * 4 < K ? 0u : kOob;
+        // this lane's 8 bytes in the stage for load 0; load i is 8 i rows (512 i bytes) further, with
+        // the same swizzle (8 i / 2 is a multiple of 4)
+        unsigned char* const wbase =
+            &sA[0][0] + dr0 * (BK * 2) + (((dc >> 1) ^ pack_swz(dr0)) << 4) + ((dc & 1) << 3);
+        float4v xs[2][NL];
+        int scaled = 0;  // 1: some row this wavefront stages has a factor < 1
+        auto load_op = [&](int s, int l) __attribute__((always_inline)) {
+          const uint32_t last = s == nk - 1 ? 0xffffffffu : 0u;
+          return __builtin_bit_cast(
+              float4v, __builtin_amdgcn_raw_buffer_load_b128(
+                           rx, static_cast<int>(((tail & last) | voff) + static_cast<uint32_t>(l * 32 * K)), s * (BK * 4), 0));
+        };
+        auto load_x = [&](auto hc, int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int s = 0; s < D; ++s) dma(s, kbeg + s * BK);
-      }
-      wait_dma_le<(D - 1) * NDMA>();  // step 0 has landed
-      b_run = B + static_cast<size_t>(kbeg + D * BK) * N + n0;
-      phase_barrier();
-      if (grp == 1) phase_barrier();
-      for (int j = 0; j < nk; ++j) {
-        __builtin_amdgcn_sched_barrier(0);
-        {
-          // The memory phase interleaves its fragment reads (LDS) and its DMA issue (texture path):
-          // NFRAG / NDMA reads, then one DMA instruction, NDMA times, then any reads left over. On
-          // the 256x256 tile at 4096^3 (12 reads, 4 DMA) this ran 0.4-0.6 % faster than all reads
-          // before all DMA, with the same result bits; every form that issues a DMA before the
-          // first reads ran 1.5-3 % slower.
-          const int kd = kbeg + (j + D) * BK;
-          const __amdgpu_buffer_rsrc_t ra = rsrc_a(kd), rb = rsrc_b_next(kd);
-          constexpr int PER = NFRAG / NDMA;
+          for (int l = 0; l < NL; ++l) xs[decltype(hc)::value][l] = load_op(s, l);
+        };
+        auto absmax4 = [](float m, float4v v) __attribute__((always_inline)) {
+          m = fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y));
+          return fmaxf(fmaxf(m, fabsf(v.z)), fabsf(v.w));
+        };
+        auto write_op = [&](int st, int l, float4v v) __attribute__((always_inline)) {
+          *reinterpret_cast<half4*>(wbase + st * Cfg::A_BYTES + l * 8 * (BK * 2)) = __builtin_convertvector(v, half4);
+        };
+        // The lane number anew, for the rarely taken branches: an address kept across the loop for them
+        // would be spilled, and a reload from scratch waits for every load in flight.
+        auto lane_id = []() __attribute__((always_inline)) {
+          int ln;
+          asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+          return ln;
+        };
+        auto apply_factors = [&](float4v (&v)[NL]) __attribute__((always_inline)) {
+          if (__builtin_expect(__builtin_amdgcn_readfirstlane(scaled), 0)) {
+            const float* const fac = s_fac + wave * 32 + (lane_id() >> 3);
 #pragma unroll
-          for (int d = 0; d < NDMA; ++d) {
-#pragma unroll
-            for (int f = d * PER; f < (d + 1) * PER; ++f) frag_op(0, j % NSTAGE, f);
-            dma_op((j + D) % NSTAGE, kd, ra, rb, d);
+            for (int l = 0; l < NL; ++l) v[l] *= fac[8 * l];
           }
+        };
+        // step s has a value past fp16's range in a row of this wavefront (see above)
+        auto raise = [&](int s) __attribute__((always_inline)) {
+          const int st = s % NSTAGE, ln = lane_id();
+          const int c = ln & 7;
+#pragma unroll 1
+          for (int l = 0; l < NL; ++l) {
+            const int r = wave * 32 + 8 * l + (ln >> 3);
+            half4* const staged =
+                reinterpret_cast<half4*>(&sA[st][r * (BK * 2) + (((c >> 1) ^ pack_swz(r)) << 4) + ((c & 1) << 3)]);
+            const half4 h = *staged;
+            if (!__any(fmaxf(fmaxf(fabsf(h.x), fabsf(h.y)), fmaxf(fabsf(h.z), fabsf(h.w))) > kHalfMax)) {
+              s_delta[st][r] = 1.f;
+              continue;
+            }
+            float4v v = __builtin_bit_cast(
+                float4v, __builtin_amdgcn_raw_buffer_load_b128(
+                             rx, s * BK + c * 4 < K ? static_cast<int>((r * K + c * 4) * 4) : static_cast<int>(kOob),
+                             s * (BK * 4), 0));
+            float f = s_fac[r];
+            v *= f;
+            float rm = absmax4(0.f, v);
 #pragma unroll
-          for (int f = NDMA * PER; f < NFRAG; ++f) frag_op(0, j % NSTAGE, f);
+            for (int d = 1; d < 8; d *= 2)
+              rm = fmaxf(rm, __int_as_float(__builtin_amdgcn_ds_bpermute((ln ^ d) * 4, __float_as_int(rm))));
+            float g = 1.f;
+            if (rm > kHalfMax) {
+              int e;
+              float sc;
+              row_exponent(rm, texp, e, sc);
+              g = e == kInfExp ? 0.f : ldexpf(1.f, -e);
+            }
+            *staged = __builtin_convertvector(v * g, half4);
+            s_delta[st][r] = g;  // the row's 8 lanes write the same values
+            s_fac[r] = f * g;
+          }
+          s_evt[st][wave] = s;
+          scaled = 1;
+        };
+        // largest |x| of a load so far; asm, so that it stays in front of the register's next load
+        auto absmax_asm = [](float& m, float4v v) __attribute__((always_inline)) {
+          asm volatile("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|"
+                       : "+v"(m)
+                       : "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
+        };
+        auto stage_x = [&](auto hc, int s) __attribute__((always_inline)) {
+          constexpr int H = decltype(hc)::value;
+          apply_factors(xs[H]);
+          float m = 0.f;
+#pragma unroll
+          for (int l = 0; l < NL; ++l) {
+            m = absmax4(m, xs[H][l]);
+            write_op(s % NSTAGE, l, xs[H][l]);
+          }
+          if (__any(m > kHalfMax)) raise(s);
+        };
+        // B's DMA, in step order. Packed: the step's 16 KB block is a scalar offset, the range ends with
+        // the last block, and the two instructions differ by 1 KB in memory as in LDS, which the
+        // instruction's offset adds to both. Row-major: a running pointer, the range ends with the
+        // matrix (rows past K), and lanes past N are masked.
+        const uint32_t bst = sB_lds + wave * Cfg::B_INSTR * 1024;
+        const __amdgpu_buffer_rsrc_t rbp = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<_Float16*>(B) + static_cast<size_t>(tn) * nk * 8192, 0, nk * 16384, kRawBufferDword3);
+        uint32_t bvo[2];
+        int kleft = K;
+        const _Float16* bcur = B + n0;
+        if constexpr (PACKED_B) {
+          bvo[0] = bvo[1] = static_cast<uint32_t>(wave * Cfg::B_INSTR * 1024 + lane * 16);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int row = b_row0 + i * Cfg::B_ROWS_PER_INSTR, c = b_phys ^ Cfg::swz_b(row);
+            bvo[i] = n0 + c * 8 < N ? static_cast<uint32_t>((row * N + c * 8) * 2) : kOob;
+          }
         }
-        wait_dma_le<(D - 1) * NDMA>();  // step j+1 has landed (this wavefront's part)
+        auto dma_b = [&](int st, int s) __attribute__((always_inline)) {
+          const uint32_t at = bst + st * Cfg::B_BYTES;
+          if constexpr (PACKED_B) {
+            asm volatile(
+                "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+                "buffer_load_dwordx4 %1, %2, %3 offen offset:1024 lds"
+                :
+                : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(bvo[0]), "s"(rbp), "s"(s * 16384)
+                : "memory", "m0");
+          } else {
+            const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<_Float16*>(bcur), 0, kleft >= BK ? 0x7fffffff : (kleft > 0 ? (kleft * N - n0) * 2 : 0),
+                kRawBufferDword3);
+            bcur += static_cast<size_t>(BK) * N;
+            kleft -= BK;
+            dma16(rb, at, bvo[0]);
+            dma16(rb, at + 1024, bvo[1]);
+          }
+        };
+        constexpr std::integral_constant<int, 0> c0{};
+        constexpr std::integral_constant<int, 1> c1{};
+        // each wavefront resets what it alone writes; the others read it past the barrier below
+        if (lane < NSTAGE) s_evt[lane][wave] = -1;
+        if (lane < 32) s_fac[wave * 32 + lane] = 1.f;
+        load_x(c0, 0);
+        load_x(c1, 1);
+        dma_b(0, 0);
+        dma_b(1, 1);
+        stage_x(c0, 0);
+        load_x(c0, 2);
+        stage_x(c1, 1);
+        load_x(c1, 3);
+        wait_dma_le<2 * NL>();  // B's steps 0 and 1 have landed
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         phase_barrier();
-        __builtin_amdgcn_sched_barrier(0);
+        if (grp == 1) phase_barrier();
+        auto step = [&](auto hc, int j) __attribute__((always_inline)) {
+          constexpr int H = decltype(hc)::value;
+          const int st = j % NSTAGE, stw = (j + D) % NSTAGE;
+          __builtin_amdgcn_sched_barrier(0);
+          const int evt = s_evt[st][wm0 / 32 + (lane & 3)];  // the 4 wavefronts that stage its 128 rows
+          constexpr int PER = NFRAG / 4;
 #pragma unroll
-        for (int m = 0; m < NMFMA; ++m) mfma_op(0, m);
-        __builtin_amdgcn_sched_barrier(0);
+          for (int f = 0; f < PER; ++f) frag_op(0, st, f);
+          __builtin_amdgcn_sched_barrier(0);
+          // step j + 2's activations are in registers, B's step j + 1 has landed (the builtin, so that
+          // the compiler knows it and adds no wait of its own past the DMA below)
+          __builtin_amdgcn_s_waitcnt(kWaitVmcnt0 + NL);
+          __builtin_amdgcn_sched_barrier(0);
+          dma_b(stw, j + D);
+          apply_factors(xs[H]);
+          float m = 0.f;
+#pragma unroll
+          for (int l = 0; l < NL; ++l) {
+            __builtin_amdgcn_sched_barrier(0);
+            write_op(stw, l, xs[H][l]);
+            absmax_asm(m, xs[H][l]);
+            __builtin_amdgcn_sched_barrier(0);
+            xs[H][l] = load_op(j + D + 2, l);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int f = (l + 1) * PER; f < (l + 2 < NL ? (l + 2) * PER : (l + 1 < NL ? NFRAG : 0)); ++f) frag_op(0, st, f);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          phase_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+          if (__builtin_expect(__any((m > kHalfMax) | (evt == j)), 0)) {
+            if (__any(m > kHalfMax)) raise(j + D);
+            // rows whose exponent was raised at this step: their sums so far follow
+            if (__any(evt == j)) {
+              const float* const del = &s_delta[st][wm0 + 4 * (lane_id() >> 4)];
+#pragma unroll
+              for (int i = 0; i < TM; ++i) {
+                if (__builtin_amdgcn_readlane(evt, i / 2) == j) {
+                  const float4v f = *reinterpret_cast<const float4v*>(del + 16 * i);
+#pragma unroll
+                  for (int jj = 0; jj < TN; ++jj) acc[i][jj] *= f;
+                }
+              }
+            }
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = 0; q < NMFMA; ++q) mfma_op(0, q);
+          __builtin_amdgcn_sched_barrier(0);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wavefront's part of stage j + 2 is in LDS
+          phase_barrier();
+        };
+        int j = 0;
+        for (; j + 1 < nk; j += 2) {
+          step(c0, j);
+          step(c1, j + 1);
+        }
+        if (j < nk) step(c0, j);
+      } else {
+        if (nk > 0) {
+#pragma unroll
+          for (int s = 0; s < D; ++s) dma(s, kbeg + s * BK);
+        }
+        wait_dma_le<(D - 1) * NDMA>();  // step 0 has landed
+        b_run = B + static_cast<size_t>(kbeg + D * BK) * N + n0;
         phase_barrier();
+        if (grp == 1) phase_barrier();
+        for (int j = 0; j < nk; ++j) {
+          __builtin_amdgcn_sched_barrier(0);
+          {
+            // The memory phase interleaves its fragment reads (LDS) and its DMA issue (texture path):
+            // NFRAG / NDMA reads, then one DMA instruction, NDMA times, then any reads left over. On
+            // the 256x256 tile at 4096^3 (12 reads, 4 DMA) this ran 0.4-0.6 % faster than all reads
+            // before all DMA, with the same result bits; every form that issues a DMA before the
+            // first reads ran 1.5-3 % slower.
+            const int kd = kbeg + (j + D) * BK;
+            const __amdgpu_buffer_rsrc_t ra = rsrc_a(kd), rb = rsrc_b_next(kd);
+            constexpr int PER = NFRAG / NDMA;
+#pragma unroll
+            for (int d = 0; d < NDMA; ++d) {
+#pragma unroll
+              for (int f = d * PER; f < (d + 1) * PER; ++f) frag_op(0, j % NSTAGE, f);
+              dma_op((j + D) % NSTAGE, kd, ra, rb, d);
+            }
+#pragma unroll
+            for (int f = NDMA * PER; f < NFRAG; ++f) frag_op(0, j % NSTAGE, f);
+          }
+          wait_dma_le<(D - 1) * NDMA>();  // step j+1 has landed (this wavefront's part)
+          phase_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int m = 0; m < NMFMA; ++m) mfma_op(0, m);
+          __builtin_amdgcn_sched_barrier(0);
+          phase_barrier();
+        }
       }
       if (grp == 0) phase_barrier();  // every wavefront passes the same number of barriers
     } else {
@@ -974,8 +1232,14 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int grow = m0 + wm0 + 32 * ri + (lane >> 3) + 8 * q;
-        erow[ri][q] = (RESIDENT || respec) ? s_scale[grow - m0]
-                                           : (SPEC ? 1.f : (rscale != nullptr && grow < M ? rscale[grow] : 1.f));
+        if constexpr (DIRECT) {
+          // 1 / factor: a power of two's exponent negated, infinity for a row's factor 0
+          const uint32_t f = __float_as_uint(s_fac[grow - m0]);
+          erow[ri][q] = __uint_as_float(f == 0u ? 0x7f800000u : 0x7f000000u - f);
+        } else {
+          erow[ri][q] = (RESIDENT || respec) ? s_scale[grow - m0]
+                                             : (SPEC ? 1.f : (rscale != nullptr && grow < M ? rscale[grow] : 1.f));
+        }
       }
 #pragma unroll
     for (int rj = 0; rj < ERJ; ++rj) {
@@ -1233,7 +1497,11 @@ using GemmFn = void (*)(const _Float16*, const _Float16*, void*, const float*, c
                         int, int, int, int, int, int, const void*, int, int, int, uint32_t*);
 
 template <bool OUT_F16>
-GemmFn<OUT_F16> gemm_fn(Tile t, bool splitk, bool packed, bool packed_b, bool resident = false, bool spec = false) {
+GemmFn<OUT_F16> gemm_fn(Tile t, bool splitk, bool packed, bool packed_b, bool resident = false, bool spec = false,
+                        bool direct = false) {
+  if (direct)
+    return packed_b ? hgemm_kernel<Cfg256, OUT_F16, false, false, true, false, false, true>
+                    : hgemm_kernel<Cfg256, OUT_F16, false, false, false, false, false, true>;
   if (spec) {
     // speculative fp16 A on the 4-wavefront tiles
     if (splitk) {
@@ -1303,6 +1571,27 @@ bool resident_route(const Plan& p, int ksplit, int K) {
   return p.tile == Tile::T32 && ksplit == 1 && K > 0 && ceil_div(K, Cfg32::BK) <= kResidentSteps;
 }
 
+// fp32 activations run as one direct launch (cast in registers on the way into the GEMM's A stages)
+// where the plan is the unsplit 256x256 tile, at most 4 tile columns read each row, the grid fills
+// three quarters of the CUs, and a tile row of x stays within a descriptor's range. It saves the cast
+// pass over x (6 bytes per value at ~6 TB/s), and costs the GEMM 32 KB of fp32 A per K step and CU
+// instead of 16 KB, and the cast's instructions, once per tile column. Event-timed on one box, cast +
+// packed GEMM -> direct (us, M x K x N, prepacked weight): 65536 x 768 x 768 134 -> 99, 65536 x 3072 x
+// 768 456 -> 349, 65536 x 256 x 256 52 -> 28, 65536 x 768 x 1024 158 -> 128, 16384 x 4096 x 1024 178 ->
+// 141; with more columns the gain ends: 65536 x 768 x 2048 261 -> 246, 65536 x 768 x 3072 364 -> 376,
+// 4096^3 117 -> 140. With 1 % of the rows past fp16's range: 65536 x 768 x 768 135 -> 113, 20000 x 768
+// x 768 47 -> 42, 20000 x 768 x 1280 (not taken) 73 -> 74; a half-empty grid has nothing to hide the
+// rescaling behind, 11000 x 768 x 768 (129 tiles, not taken) 34 -> 38 (29 without such rows).
+constexpr int kDirectMaxK = 1 << 20;
+constexpr int kDirectMaxN = 1024;
+bool direct_route(const Plan& p, int N, int K, int ksplit, int num_cus) {
+  return p.tile == Tile::T256 && ksplit == 1 && K > 0 && K <= kDirectMaxK && N <= kDirectMaxN &&
+         4L * p.ntm * p.ntn >= 3L * num_cus;
+}
+// Thresholds the direct launch takes: up to 2^15, so that every value of a row within the threshold
+// has a finite cast (it rescales only rows that leave fp16's range).
+constexpr int kDirectMaxTexp = 15;
+
 // A speculative launch (mm_t's GEMM path in one launch for fp16 x on the 4-wavefront tiles): log2
 // of the threshold (>= kSpecMinTexp), the largest fp16 bit pattern not above it, and the weight's
 // history slot (or NULL).
@@ -1326,7 +1615,7 @@ int fp16_bits_at_most(int texp) {
 int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, const float* bias, const float* rscale,
                 int M, int N, int K, int ksplit, int num_cus, void* ws, size_t ws_bytes, uint32_t* counters_in,
                 size_t counter_bytes_in, void* stream, bool packed = false, bool packed_b = false,
-                const ResidentCast* rc = nullptr, const SpecA* sp = nullptr) {
+                const ResidentCast* rc = nullptr, const SpecA* sp = nullptr, bool direct = false) {
   if (M < 0 || N < 0 || K < 0 || K % 8 != 0 || N % 8 != 0 || K > kMaxK || N > kMaxN) return G16_E_SHAPE;
   if (M == 0 || N == 0) return G16_OK;
   if (ksplit < 1 || ksplit > 256) return G16_E_SPLIT;
@@ -1335,7 +1624,7 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   const KSplit ks = ksplit_for(K, ksplit);
   if (num_cus <= 0) num_cus = stream_cus(static_cast<hipStream_t>(stream));
   Plan p = choose_tile(M, N, K, num_cus);
-  if (rc != nullptr && !resident_route(p, ks.ksplit, K)) return G16_E_SHAPE;
+  if (direct ? !direct_route(p, N, K, ks.ksplit, num_cus) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
   const bool spec = sp != nullptr;
   if (spec && (!four_wave(p.tile) || packed ||
                ks.ksplit > kSpecMaxSplit || sp->texp < kSpecMinTexp))
@@ -1365,16 +1654,16 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   const auto* b = reinterpret_cast<const _Float16*>(B);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool sk = ks.ksplit > 1;
-  const bool res = rc != nullptr;
-  const void* x = res ? rc->x : nullptr;
-  const int x_f32 = res ? rc->x_f32 : 0;
-  const int texp = res ? rc->texp : (spec ? sp->texp : 0);
+  const bool res = rc != nullptr && !direct;
+  const void* x = rc != nullptr ? rc->x : nullptr;
+  const int x_f32 = rc != nullptr ? rc->x_f32 : 0;
+  const int texp = rc != nullptr ? rc->texp : (spec ? sp->texp : 0);
   const int tbits = spec ? sp->tbits : 0;
   uint32_t* miss = spec ? sp->miss : nullptr;
   if (out_f16)
-    return launch(gemm_fn<true>(p.tile, sk, packed, packed_b, res, spec), grid, block, s, a, b, C, bias, rscale, part,
+    return launch(gemm_fn<true>(p.tile, sk, packed, packed_b, res, spec, direct), grid, block, s, a, b, C, bias, rscale, part,
                   counters, M, N, K, ks.kchunk, ks.ksplit, p.ntm, p.ntn, x, x_f32, texp, tbits, miss);
-  return launch(gemm_fn<false>(p.tile, sk, packed, packed_b, res, spec), grid, block, s, a, b, C, bias, rscale, part,
+  return launch(gemm_fn<false>(p.tile, sk, packed, packed_b, res, spec, direct), grid, block, s, a, b, C, bias, rscale, part,
                 counters, M, N, K, ks.kchunk, ks.ksplit, p.ntm, p.ntn, x, x_f32, texp, tbits, miss);
 }
 
@@ -1615,6 +1904,8 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   if (scratch == nullptr) return G16_E_NULL;
   if (!g16::aligned16(scratch)) return G16_E_ALIGN;
   if (scratch_bytes < g16_mm_t_scratch_bytes(M, N, K, num_cus)) return G16_E_WORKSPACE;
+  if (x_is_f32 && texp <= g16::kDirectMaxTexp && g16_mm_t_direct_route(M, N, K, num_cus) == 1)
+    return g16_mm_t_direct(static_cast<const float*>(x), w_t, 0, out, out_is_f16, bias, thresh, M, N, K, num_cus, stream);
   const bool packed = g16_hgemm_use_packed(M, N, K, num_cus) == 1;
   auto* y = static_cast<uint16_t*>(scratch);
   auto* s = reinterpret_cast<float*>(static_cast<unsigned char*>(scratch) + g16::round256(g16::cast_bytes(M, K, packed)));
@@ -1632,6 +1923,24 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   const int ks = g16_hgemm_plan(M, N, K, num_cus);
   return g16::gemm_launch(y, w_t, out, out_is_f16 != 0, bias, s, M, N, K, ks, num_cus, workspace, workspace_bytes,
                           counters, counter_bytes, stream);
+}
+
+extern "C" int g16_mm_t_direct_route(int M, int N, int K, int num_cus) {
+  if (M <= 0 || N <= 0 || K <= 0 || num_cus <= 0) return 0;
+  return g16::direct_route(g16::choose_tile(M, N, K, num_cus), N, K, g16_hgemm_plan(M, N, K, num_cus), num_cus) ? 1 : 0;
+}
+
+extern "C" int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,
+                               const float* bias, float thresh, int M, int N, int K, int num_cus, void* stream) {
+  if (M < 0 || N < 0 || K < 0 || K % 8 != 0 || N % 8 != 0 || num_cus <= 0) return G16_E_SHAPE;
+  if (M == 0 || N == 0) return G16_OK;
+  if (out == nullptr || x == nullptr || w == nullptr) return G16_E_NULL;
+  const int texp = g16::thresh_exponent(thresh);
+  if (texp == -1000 || texp > g16::kDirectMaxTexp || g16_mm_t_direct_route(M, N, K, num_cus) == 0) return G16_E_SHAPE;
+  if (!g16::aligned16(x)) return G16_E_ALIGN;
+  const g16::ResidentCast rc{x, 1, texp};
+  return g16::gemm_launch(nullptr, w, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus, nullptr, 0, nullptr, 0,
+                          stream, false, w_packed != 0, &rc, nullptr, true);
 }
 
 extern "C" int g16_mm_t_spec_history(void* stream) {

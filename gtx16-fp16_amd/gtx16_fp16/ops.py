@@ -88,29 +88,29 @@ def skinny_config(N: int, K: int, sms: int) -> tuple[tuple[int, int, int], int]:
     return ((N + cols - 1) // cols * ksplit, 1, 1), rows
 
 
-# (M, N, K, device index) -> the GEMM route mm_t takes for that shape, computed once per shape:
-# ("packed", packed-activation bytes) | ("splitk", ksplit, partial bytes, counter bytes) | ("plain",);
-# skinny shapes are keyed (-M, N, K, device index) -> (ksplit, partial bytes, counter bytes).
+# (M, N, K, device index) -> the GEMM route mm_t takes for that shape (_gemm_route), computed once per
+# shape; skinny shapes are keyed (-M, N, K, device index) -> (ksplit, partial bytes, counter bytes).
 _routes: dict[tuple[int, int, int, int], tuple] = {}
 
 
 def _gemm_route(lib, M: int, N: int, K: int, dev: torch.device) -> tuple:
-    """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes) of the GEMM path
-    for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count."""
+    """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes, direct) of the GEMM
+    path for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count; direct:
+    fp32 activations run as one launch that casts them itself (g16_mm_t_direct)."""
     key = (M, N, K, dev.index or 0)
     r = _routes.get(key)
     if r is None:
         cus = _sm_count(dev)
         scratch = lib.g16_mm_t_scratch_bytes(M, N, K, cus)
         if lib.g16_hgemm_use_packed(M, N, K, cus):
-            r = ("packed", scratch, 1, 0, 0)
+            r = ("packed", scratch, 1, 0, 0, lib.g16_mm_t_direct_route(M, N, K, cus) == 1)
         else:
             ksplit = lib.g16_hgemm_plan(M, N, K, cus)
             if ksplit > 1:
                 r = ("splitk", scratch, ksplit, lib.g16_hgemm_splitk_workspace_bytes(M, N, K, ksplit, cus),
-                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus))
+                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False)
             else:
-                r = ("plain", scratch, 1, 0, 0)
+                r = ("plain", scratch, 1, 0, 0, False)
         _remember(key, r)
     return r
 
@@ -165,7 +165,9 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     x2d fp16 or fp32; w_t fp16; bias fp32 (or None); out fp32 or fp16. Check supported() first.
     M <= 8: fp32 math on the unquantised x (skinny path). M > 8: rows with |max| > 1024 are scaled
     by a power of two, cast to fp16, multiplied on the matrix cores with fp32 accumulation and
-    scaled back; shapes with too few output tiles split K with a deterministic reduction."""
+    scaled back; shapes with too few output tiles split K with a deterministic reduction. (Large fp32
+    batches into at most 1024 columns scale only the rows that leave fp16's range, 65504: the GEMM
+    casts x itself, and every value is rounded at least as finely.)"""
     if out_dtype not in (torch.float32, torch.float16):
         raise ValueError(f"out_dtype must be float32 or float16, got {out_dtype}")
     _check_operands(x2d, w_t, bias)
@@ -206,8 +208,11 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     if x2d.dtype == torch.float16 and dev.index not in _spec_history:
         if lib.g16_mm_t_spec_history(stream) == 0:
             _spec_history.add(dev.index)
-    kind, scratch_bytes, _ks, ws_bytes, cnt_bytes = _gemm_route(lib, M, N, K, dev)
+    kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct = _gemm_route(lib, M, N, K, dev)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
+    if direct and x2d.dtype == torch.float32:
+        _direct(lib, x2d, w_t, 0, out, bptr, M, N, K, dev, stream)
+        return out
     # no scratch where the GEMM casts its own rows into LDS (one launch, the unsplit small tile)
     scratch = scratch_buffer(dev, stream, scratch_bytes) if scratch_bytes else None
     bufs = split_buffers(dev, stream, ws_bytes, cnt_bytes) if kind == "splitk" else (None, 0, None, 0)
@@ -216,6 +221,14 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
                                   M, N, K, _sm_count(dev), None if scratch is None else scratch.data_ptr(),
                                   scratch_bytes, *bufs, stream), "GEMM")
     return out
+
+
+def _direct(lib, x2d: torch.Tensor, w: torch.Tensor, packed: int, out: torch.Tensor, bptr, M: int, N: int, K: int,
+            dev: torch.device, stream: int) -> None:
+    # fp32 activations into few columns (N <= 1024): the GEMM reads and casts x itself, no scratch
+    _clib.check(lib.g16_mm_t_direct(x2d.data_ptr(), w.data_ptr(), packed, out.data_ptr(),
+                                    1 if out.dtype == torch.float16 else 0, bptr, ROW_SCALE_THRESHOLD, M, N, K,
+                                    _sm_count(dev), stream), "GEMM")
 
 
 def prepacked_route(M: int, N: int, K: int, device: torch.device) -> bool:
@@ -347,6 +360,9 @@ def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias:
     b = None if bias is None else bias.float().contiguous()
     x2d = _aligned(x2d)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
+    if _cast_source is None and x2d.dtype == torch.float32 and _gemm_route(lib, M, N, K, dev)[5]:
+        _direct(lib, x2d, wp, 1, out, None if b is None else b.data_ptr(), M, N, K, dev, stream)
+        return out
     _scratch, xp, rscale = _packed_cast(lib, x2d, M, K, dev, stream, _cast_source)
     fn = lib.g16_hgemm_packed_ab_f32out if out_dtype == torch.float32 else lib.g16_hgemm_packed_ab_f16out
     _clib.check(fn(xp, wp.data_ptr(), out.data_ptr(), None if b is None else b.data_ptr(), rscale, M, N, K, stream),

@@ -232,6 +232,27 @@ def test_one_launch_route_needs_no_scratch(lib):
         assert lib.g16_mm_t_scratch_bytes(M, N, K, 256) > 0, (M, N, K)
 
 
+def test_direct_route_rule_and_refusals(lib):
+    # fp32 activations cast by the GEMM itself: unsplit 256x256 tiles, N <= 1024, three quarters of the
+    # CUs busy; where the rule says 0 the entry point refuses before any launch
+    r, A = lib.g16_mm_t_direct_route, 0x1000
+    assert r(65536, 768, 768, 256) == 1 and r(65536, 768, 3072, 256) == 1 and r(65536, 256, 8, 256) == 1
+    assert r(65536, 3072, 768, 256) == 0 and r(4096, 4096, 4096, 256) == 0 and r(11000, 768, 768, 256) == 0
+    assert r(64, 1024, 1024, 256) == 0 and r(0, 768, 768, 256) == 0 and r(65536, 768, 768, 0) == 0
+    assert r(65536, 256, (1 << 20) + 8, 256) == 0 and r(65536, 256, 1 << 20, 256) == 1
+    d = lib.g16_mm_t_direct
+    assert d(A, A, 0, A, 0, None, 1024.0, 4096, 4096, 4096, 256, None) == -1
+    assert d(A, A, 0, A, 0, None, 65536.0, 65536, 768, 768, 256, None) == -1    # threshold past 2^15
+    assert d(A, A, 0, A, 0, None, 1000.0, 65536, 768, 768, 256, None) == -1     # not a power of two
+    assert d(A + 4, A, 0, A, 0, None, 1024.0, 65536, 768, 768, 256, None) == -2
+    assert d(A, A + 8, 1, A, 0, None, 1024.0, 65536, 768, 768, 256, None) == -2
+    assert d(None, A, 0, A, 0, None, 1024.0, 65536, 768, 768, 256, None) == -3
+    assert d(A, A, 0, A, 0, None, 1024.0, 0, 768, 768, 256, None) == 0
+    # g16_mm_t_gemm asks for its scratch on these shapes as on every other
+    need = lib.g16_mm_t_scratch_bytes(65536, 768, 768, 256)
+    assert lib.g16_mm_t_gemm(A, 1, A, A, 0, None, 1024.0, 65536, 768, 768, 256, A, need - 1, None, 0, None, 0, None) == -4
+
+
 def test_fast_extension_matches_the_c_entry_points(lib):
     # _g16fast forwards its arguments unchanged: the same rejected calls give the same statuses
     fast = _clib.fast()
