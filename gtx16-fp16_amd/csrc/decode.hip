@@ -50,8 +50,9 @@ __device__ inline float act(const _Float16* __restrict__ A, long i) { return sta
 
 template <typename TX, int MM, int U>
 __global__ __launch_bounds__(kStripThreads) void strips_kernel(const TX* __restrict__ A, const _Float16* __restrict__ D,
-                                                               float* __restrict__ C, const float* __restrict__ bias,
-                                                               int N, int K, int rows_per_wave) {
+                                                               void* __restrict__ Cv, int c_f16,
+                                                               const float* __restrict__ bias, int N, int K,
+                                                               int rows_per_wave) {
   const int s = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -143,7 +144,10 @@ __global__ __launch_bounds__(kStripThreads) void strips_kernel(const TX* __restr
 #pragma unroll
     for (int w = 1; w < kStripWaves; ++w) sum += red[w][m][c];
     const int n = s * kStripCols + c;
-    C[static_cast<long>(m) * N + n] = sum + (bias != nullptr ? bias[n] : 0.f);
+    sum += bias != nullptr ? bias[n] : 0.f;
+    // an fp16 output is the fp32 sum rounded once
+    if (c_f16) static_cast<_Float16*>(Cv)[static_cast<long>(m) * N + n] = static_cast<_Float16>(sum);
+    else static_cast<float*>(Cv)[static_cast<long>(m) * N + n] = sum;
   }
 }
 
@@ -161,7 +165,7 @@ auto strips_fn_u(int M) {
 }
 
 template <typename TX>
-int strips_launch(const TX* A, const uint16_t* D, float* C, const float* bias, int M, int N, int K, void* stream) {
+int strips_launch(const TX* A, const uint16_t* D, void* C, int c_f16, const float* bias, int M, int N, int K, void* stream) {
   if (M < 0 || N < 0 || K < 0 || M > G16_STRIPS_MAX_M || K % 8 != 0 || N % 8 != 0) return G16_E_SHAPE;
   if (M == 0 || N == 0) return G16_OK;
   if (C == nullptr || (K > 0 && (A == nullptr || D == nullptr))) return G16_E_NULL;
@@ -170,7 +174,7 @@ int strips_launch(const TX* A, const uint16_t* D, float* C, const float* bias, i
   // Eight row loads per lane in flight when a wavefront has that many rows; K <= 2040 takes two.
   auto fn = rows >= 4 * kWave ? strips_fn_u<TX, 8>(M) : strips_fn_u<TX, 2>(M);
   return launch(fn, dim3(static_cast<unsigned>(N / kStripCols)), dim3(kStripThreads), static_cast<hipStream_t>(stream),
-                A, reinterpret_cast<const _Float16*>(D), C, bias, N, K, rows);
+                A, reinterpret_cast<const _Float16*>(D), C, c_f16, bias, N, K, rows);
 }
 
 }  // namespace
@@ -189,12 +193,19 @@ extern "C" int g16_pack_decode_weight(const uint16_t* w_t, uint16_t* wd, int K, 
 
 extern "C" int g16_skinny_strips_f32in(const float* A, const uint16_t* wd, float* C, const float* bias, int M, int N,
                                        int K, void* stream) {
-  return g16::strips_launch<float>(A, wd, C, bias, M, N, K, stream);
+  return g16::strips_launch<float>(A, wd, C, 0, bias, M, N, K, stream);
 }
 
 extern "C" int g16_skinny_strips_f16in(const uint16_t* A, const uint16_t* wd, float* C, const float* bias, int M, int N,
                                        int K, void* stream) {
-  return g16::strips_launch<_Float16>(reinterpret_cast<const _Float16*>(A), wd, C, bias, M, N, K, stream);
+  return g16::strips_launch<_Float16>(reinterpret_cast<const _Float16*>(A), wd, C, 0, bias, M, N, K, stream);
+}
+
+extern "C" int g16_skinny_strips(const void* A, int a_is_f32, const uint16_t* wd, void* C, int c_is_f16, const float* bias,
+                                 int M, int N, int K, void* stream) {
+  const int f16 = c_is_f16 != 0 ? 1 : 0;
+  return a_is_f32 ? g16::strips_launch<float>(static_cast<const float*>(A), wd, C, f16, bias, M, N, K, stream)
+                  : g16::strips_launch<_Float16>(static_cast<const _Float16*>(A), wd, C, f16, bias, M, N, K, stream);
 }
 
 extern "C" int g16_skinny_strips_route(int M, int N, int K, int x_f32) {

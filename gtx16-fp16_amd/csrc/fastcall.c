@@ -1,10 +1,10 @@
 /* _g16fast: a CPython extension that calls the per-call entry points of libg16.so that sit on
- * latency-bound paths -- g16_skinny_f32in and g16_skinny_strips_f32in (the FastLinear decode
+ * latency-bound paths -- g16_skinny, g16_skinny_strips and their fp32 forms (mm_t at M <= 8 and the FastLinear decode
  * shortcut, the counterpart of the reference's PreparedLaunch, src/gtx16_fp16/kernels.py:324-338)
  * and g16_mm_t_gemm (mm_t's GEMM path, ops.py:86-108) -- with METH_FASTCALL argument parsing. Through ctypes the same calls spend
  * ~0.1 us per argument converting them; here the conversion is a few ns per argument.
  *
- * The module does not link libg16.so: bind() receives the addresses of the three functions from the
+ * The module does not link libg16.so: bind() receives the addresses of the functions from the
  * library the ctypes binding already loaded, so both bindings call into the same instance. Pointer
  * arguments are Python ints or None (NULL); every call returns the entry point's int status. The
  * GIL is released around the call, as ctypes does.
@@ -20,6 +20,11 @@ typedef int (*mm_t_gemm_fn)(const void*, int, const void*, void*, int, const voi
                             size_t, void*, size_t, void*, size_t, void*);
 
 typedef int (*strips_fn)(const void*, const void*, void*, const void*, int, int, int, void*);
+typedef int (*skinny_any_fn)(const void*, int, const void*, void*, int, const void*, int, int, int, int, void*, size_t,
+                             void*, size_t, void*);
+typedef int (*strips_any_fn)(const void*, int, const void*, void*, int, const void*, int, int, int, void*);
+static skinny_any_fn g_skinny = NULL;
+static strips_any_fn g_strips = NULL;
 static skinny_fn g_skinny_f32in = NULL;
 static strips_fn g_strips_f32in = NULL;
 static mm_t_gemm_fn g_mm_t_gemm = NULL;
@@ -57,17 +62,19 @@ static int check_nargs(const char* name, Py_ssize_t nargs, Py_ssize_t want) {
 
 static PyObject* fast_bind(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
   (void)self;
-  void *skinny, *gemm, *strips;
-  if (check_nargs("bind", nargs, 3) || as_ptr(args[0], &skinny) || as_ptr(args[1], &gemm) ||
-      as_ptr(args[2], &strips))
+  void *skinny, *gemm, *strips, *skinny_any, *strips_any;
+  if (check_nargs("bind", nargs, 5) || as_ptr(args[0], &skinny) || as_ptr(args[1], &gemm) ||
+      as_ptr(args[2], &strips) || as_ptr(args[3], &skinny_any) || as_ptr(args[4], &strips_any))
     return NULL;
-  if (skinny == NULL || gemm == NULL || strips == NULL) {
-    PyErr_SetString(PyExc_ValueError, "bind() needs three non-NULL function addresses");
+  if (skinny == NULL || gemm == NULL || strips == NULL || skinny_any == NULL || strips_any == NULL) {
+    PyErr_SetString(PyExc_ValueError, "bind() needs five non-NULL function addresses");
     return NULL;
   }
   g_skinny_f32in = (skinny_fn)skinny;
   g_mm_t_gemm = (mm_t_gemm_fn)gemm;
   g_strips_f32in = (strips_fn)strips;
+  g_skinny = (skinny_any_fn)skinny_any;
+  g_strips = (strips_any_fn)strips_any;
   Py_RETURN_NONE;
 }
 
@@ -111,6 +118,41 @@ static PyObject* fast_strips_f32in(PyObject* self, PyObject* const* args, Py_ssi
   return PyLong_FromLong(st);
 }
 
+/* skinny(x, x_is_f32, w_t, out, out_is_f16, bias, M, N, K, ksplit, partials, partial_bytes, counters,
+ * counter_bytes, stream) -> status of g16_skinny */
+static PyObject* fast_skinny(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  void *x, *w, *out, *bias, *part, *cnt, *stream;
+  int x_is_f32, out_is_f16, M, N, K, ksplit, st;
+  size_t part_bytes, cnt_bytes;
+  if (check_bound((const void*)g_skinny) || check_nargs("skinny", nargs, 15)) return NULL;
+  if (as_ptr(args[0], &x) || as_int(args[1], &x_is_f32) || as_ptr(args[2], &w) || as_ptr(args[3], &out) ||
+      as_int(args[4], &out_is_f16) || as_ptr(args[5], &bias) || as_int(args[6], &M) || as_int(args[7], &N) ||
+      as_int(args[8], &K) || as_int(args[9], &ksplit) || as_ptr(args[10], &part) || as_size(args[11], &part_bytes) ||
+      as_ptr(args[12], &cnt) || as_size(args[13], &cnt_bytes) || as_ptr(args[14], &stream))
+    return NULL;
+  Py_BEGIN_ALLOW_THREADS
+  st = g_skinny(x, x_is_f32, w, out, out_is_f16, bias, M, N, K, ksplit, part, part_bytes, cnt, cnt_bytes, stream);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(st);
+}
+
+/* skinny_strips(x, x_is_f32, wd, out, out_is_f16, bias, M, N, K, stream) -> status of g16_skinny_strips */
+static PyObject* fast_strips(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
+  (void)self;
+  void *x, *wd, *out, *bias, *stream;
+  int x_is_f32, out_is_f16, M, N, K, st;
+  if (check_bound((const void*)g_strips) || check_nargs("skinny_strips", nargs, 10)) return NULL;
+  if (as_ptr(args[0], &x) || as_int(args[1], &x_is_f32) || as_ptr(args[2], &wd) || as_ptr(args[3], &out) ||
+      as_int(args[4], &out_is_f16) || as_ptr(args[5], &bias) || as_int(args[6], &M) || as_int(args[7], &N) ||
+      as_int(args[8], &K) || as_ptr(args[9], &stream))
+    return NULL;
+  Py_BEGIN_ALLOW_THREADS
+  st = g_strips(x, x_is_f32, wd, out, out_is_f16, bias, M, N, K, stream);
+  Py_END_ALLOW_THREADS
+  return PyLong_FromLong(st);
+}
+
 /* mm_t_gemm(x, x_is_f32, w_t, out, out_is_f16, bias, thresh, M, N, K, num_cus, scratch, scratch_bytes,
  * workspace, workspace_bytes, counters, counter_bytes, stream) -> status of g16_mm_t_gemm */
 static PyObject* fast_mm_t_gemm(PyObject* self, PyObject* const* args, Py_ssize_t nargs) {
@@ -139,7 +181,11 @@ static PyObject* fast_mm_t_gemm(PyObject* self, PyObject* const* args, Py_ssize_
 
 static PyMethodDef fast_methods[] = {
     {"bind", (PyCFunction)(void (*)(void))fast_bind, METH_FASTCALL,
-     "bind(skinny_f32in_addr, mm_t_gemm_addr, skinny_strips_f32in_addr)"},
+     "bind(skinny_f32in_addr, mm_t_gemm_addr, skinny_strips_f32in_addr, skinny_addr, skinny_strips_addr)"},
+    {"skinny", (PyCFunction)(void (*)(void))fast_skinny, METH_FASTCALL,
+     "g16_skinny with fast argument parsing; returns its status"},
+    {"skinny_strips", (PyCFunction)(void (*)(void))fast_strips, METH_FASTCALL,
+     "g16_skinny_strips with fast argument parsing; returns its status"},
     {"skinny_strips_f32in", (PyCFunction)(void (*)(void))fast_strips_f32in, METH_FASTCALL,
      "g16_skinny_strips_f32in with fast argument parsing; returns its status"},
     {"skinny_f32in", (PyCFunction)(void (*)(void))fast_skinny_f32in, METH_FASTCALL,

@@ -2,7 +2,7 @@
 //
 // Semantics (reference: src/gtx16_fp16/kernels.py:153-219, ops.py:45-51,78-84): fp32 math on the
 // unquantised activations (fp32 or fp16 used as is), fp16 weights widened to fp32, bias added once,
-// fp32 output.
+// fp32 output, or an fp16 one rounded once from it as it is stored.
 //
 // The path is HBM-bound for small M (arithmetic intensity <= 8 flop/byte): B is streamed exactly
 // once and the design follows from B's layout ([K,N], N contiguous):
@@ -25,7 +25,8 @@
 //     strip, and the last arriver reads slices x M x width partial sums back through one CU.
 //     Up to N = 8192 the strips are 256 columns (half the slices of 512-column strips and a 4x
 //     smaller read-back; 128-column strips stream worse: 1 x 4096^2 in 8.58-8.62 us, against
-//     9.11-9.16 with 512 columns and 8.91-8.98 with 128), above that 512 (strip_cols).
+//     9.11-9.16 with 512 columns and 8.91-8.98 with 128), above that 512, except at M >= 7
+//     (strip_cols).
 #include <mutex>
 #include <type_traits>
 
@@ -45,7 +46,7 @@ constexpr int kWaves = 8;        // wavefronts per workgroup
 constexpr int kThreads = kWaves * kWave;
 constexpr int kMinRows = 8;      // the plan gives every wavefront at least this many rows
 constexpr int kMfBatch = 32;     // K rows per batch of the matrix-core form
-constexpr int kMfMaxBatches = 4; // ... its activations held in registers: up to 128 rows per wavefront
+constexpr int kMfGroup = 4;      // ... whose activations are held in registers at a time: 128 rows per wavefront
 
 // Launch schedule of the kernel:
 //   cols   -- columns of the strip a workgroup owns: 512 (one 1 KB row per load instruction) or
@@ -111,12 +112,12 @@ __device__ inline void split_hi_lo(float x, _Float16& hi, _Float16& lo) {
   lo = __builtin_bit_cast(_Float16, hz ? (xz ? static_cast<uint16_t>(0u) : tiny) : ((lb & 0x7fffu) == 0 ? tiny : lb));
 }
 
-// MF (launched by use_mf: M = 8, 256-column strips, 32..128 K rows per wavefront): a wavefront
+// MF (launched by use_mf: larger M on 256-column strips, enough K rows per wavefront): a wavefront
 // whose activations are all finite multiplies on the matrix cores (below); one with an inf or NaN
 // among them takes the fp32 FMA loop.
 template <typename TX, int MM, class S, bool MF = false>
 __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__ A, const _Float16* __restrict__ B,
-                                                          float* __restrict__ C, const float* __restrict__ bias,
+                                                          void* __restrict__ Cv, int c_f16, const float* __restrict__ bias,
                                                           float* __restrict__ part, uint32_t* __restrict__ counters,
                                                           int N, int K, int rows_per_wave, int ksplit, int nstrips) {
   constexpr int kStripCols = S::cols, kLanesPerRow = S::lanes_per_row, kRowsPerLoad = S::rows_per_load;
@@ -139,10 +140,27 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[m][j] = 0.f;
 
-  // A[m, r] for row r = k + sub of a load instruction that starts at row k: the instruction's
+  // A[m, r] for row r = k + sub of load instruction u of a batch, which starts at row k: the instruction's
   // kRowsPerLoad activations are wavefront-uniform (scalar loads), each lane keeps its own. Rows at
   // or past k1 are not read (tail of the slice) and give 0.
-  auto act = [&](int k, bool whole, float (&a)[MM]) {
+  //   fp16 activations of an even row and the next share an aligned dword (K is even): with EVEN (the
+  // wavefront's rows start at an even one) it is loaded once and each lane shifts its half down, one
+  // VALU instruction per load and row of A; the half-by-half form below loads it twice, converts both
+  // halves and selects (4 x 4096^2: 14.1 us, 10.4 with EVEN). The odd half past the slice belongs to
+  // a row the caller skips.
+  auto act = [&](auto evenc, int kb, int u, bool whole, float (&a)[MM]) __attribute__((always_inline)) {
+    const int k = kb + u * kRowsPerLoad;
+    if constexpr (std::is_same_v<TX, _Float16> && decltype(evenc)::value) {
+#pragma unroll
+      for (int m = 0; m < MM; ++m) {
+        const uint32_t* row = reinterpret_cast<const uint32_t*>(A + static_cast<size_t>(m) * K);
+        const int pair = u * kRowsPerLoad / 2;  // kb is even
+        const int odd = kRowsPerLoad == 2 ? sub : u & 1;
+        const uint32_t d = (whole || kb + 2 * pair < k1) ? row[(kb >> 1) + pair] : 0u;
+        a[m] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(d >> (16 * odd))));
+      }
+      return;
+    }
 #pragma unroll
     for (int m = 0; m < MM; ++m) {
       float v[kRowsPerLoad];
@@ -189,75 +207,111 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
         w[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(bp + static_cast<size_t>(min(row, k1 - 1)) * N));
       }
     };
-    float xr[kMfMaxBatches][8];
-    float amax = 0.f;
-    if (nb <= kMfMaxBatches && rows_per_wave >= kMfBatch) {
-      // The first batch's weights stream while the activations come in (a wavefront that falls
-      // back to the FMA loop drops them). Every activation this lane's A fragments need is then
-      // loaded: rows past the wavefront's range (and rows am >= M) are 0.
-      load_batch(k0);
-#pragma unroll
-      for (int bt = 0; bt < kMfMaxBatches; ++bt)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const int row = k0 + kMfBatch * bt + 4 * t + sig;
-          xr[bt][t] = (bt < nb && am < MM && row < k1) ? x_at(A, static_cast<size_t>(am) * K + row) : 0.f;
-        }
-      // |x| of row am over the wavefront's rows (the 4 lanes of each row combined); an inf or NaN
-      // sends the wavefront to the FMA loop
-      bool bad = false;
-#pragma unroll
-      for (int bt = 0; bt < kMfMaxBatches; ++bt)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          const float v = fabsf(xr[bt][t]);
-          bad = bad || !(v <= 3.402823466e38f);
-          amax = fmaxf(amax, v);
-        }
-      amax = fmaxf(amax, __shfl_xor(amax, 16));
-      amax = fmaxf(amax, __shfl_xor(amax, 32));
-      fma_loop = __any(bad);
-    }
-    if (!fma_loop) {
-      const int e = amax > 0.f ? __builtin_amdgcn_frexp_expf(amax) - 15 : 0;  // amax * 2^-e in [2^14, 2^15)
-      float4v acc2[2][8];
+    constexpr bool XF16 = std::is_same_v<TX, _Float16>;
+    // fp16 activations are their own A fragments: no scale, no lo parts (A rows 8-15 are 0 and their
+    // sums, which an infinite weight makes NaN, are not used), and infinities and NaN multiply as in
+    // the FMA loop.
+    //   The activations are held kMfGroup batches at a time. Their row exponents only rise: a group
+    // with a larger |x| in row m scales the row's sums down to the new exponent (exact) and goes on in
+    // it, so the parts of every x are exact to 2^-38 of the row's largest |x| so far.
+    std::conditional_t<XF16, _Float16, float> xr[kMfGroup][8];
+    float4v acc2[2][8];
+    constexpr int kNoExp = -1000;  // no nonzero activation in the row yet
+    int e = kNoExp;
+    if (rows_per_wave >= kMfBatch) {
+      fma_loop = false;
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc2[s][j] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int g0 = 0; g0 < nb; g0 += kMfGroup) {
+        // The group's first weights stream while its activations come in (a wavefront that falls
+        // back to the FMA loop drops them). Rows past the wavefront's range (and rows am >= M) are 0.
+        load_batch(k0 + kMfBatch * g0);
 #pragma unroll
-      for (int bt = 0; bt < kMfMaxBatches; ++bt) {
-        if (bt >= nb) break;
-        const int r = k0 + kMfBatch * bt;
-        if (bt > 0) load_batch(r);
+        for (int bt = 0; bt < kMfGroup; ++bt)
 #pragma unroll
-        for (int u = 0; u < 16; ++u)
-          if (!col_ok || r + 2 * u + sub >= k1) w[u] = u32x4{0u, 0u, 0u, 0u};
-        half8 af;
+          for (int t = 0; t < 8; ++t) {
+            const int row = k0 + kMfBatch * (g0 + bt) + 4 * t + sig;
+            if constexpr (XF16)
+              xr[bt][t] = (am < MM && !alo && row < k1) ? A[static_cast<size_t>(am) * K + row] : static_cast<_Float16>(0.f);
+            else
+              xr[bt][t] = (am < MM && row < k1) ? x_at(A, static_cast<size_t>(am) * K + row) : 0.f;
+          }
+        if constexpr (!XF16) {
+          // |x| of row am over the group's rows (the 4 lanes of each row combined); an inf or NaN sends
+          // the wavefront to the FMA loop
+          bool bad = false;
+          float amax = 0.f;
 #pragma unroll
-        for (int t = 0; t < 8; ++t) {
-          _Float16 hi, lo;
-          split_hi_lo(__builtin_ldexpf(xr[bt][t], -e), hi, lo);
-          af[t] = alo ? lo : hi;
+          for (int bt = 0; bt < kMfGroup; ++bt)
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+              const float v = fabsf(xr[bt][t]);
+              bad = bad || !(v <= 3.402823466e38f);
+              amax = fmaxf(amax, v);
+            }
+          if (__any(bad)) {
+            fma_loop = true;
+            break;
+          }
+          amax = fmaxf(amax, __shfl_xor(amax, 16));
+          amax = fmaxf(amax, __shfl_xor(amax, 32));
+          // amax * 2^-e in [2^14, 2^15)
+          const int en = amax > 0.f ? max(e, __builtin_amdgcn_frexp_expf(amax) - 15) : e;
+          if (g0 > 0 && __any(en != e)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int d = __shfl(e - en, 4 * (g & 1) + i);
+#pragma unroll
+              for (int s = 0; s < 2; ++s)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc2[s][j][i] = __builtin_ldexpf(acc2[s][j][i], d);
+            }
+          }
+          e = en;
         }
 #pragma unroll
-        for (int p = 0; p < 8; ++p)
+        for (int bt = 0; bt < kMfGroup; ++bt) {
+          if (g0 + bt >= nb) break;
+          const int r = k0 + kMfBatch * (g0 + bt);
+          if (bt > 0) load_batch(r);
 #pragma unroll
-          for (int d = 0; d < 4; ++d) {
-            const auto sw = __builtin_amdgcn_permlane16_swap(w[2 * p][d], w[2 * p + 1][d], false, false);
-            w[2 * p][d] = sw[0];
-            w[2 * p + 1][d] = sw[1];
+          for (int u = 0; u < 16; ++u)
+            if (!col_ok || r + 2 * u + sub >= k1) w[u] = u32x4{0u, 0u, 0u, 0u};
+          half8 af;
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            if constexpr (XF16) {
+              af[t] = xr[bt][t];
+            } else {
+              _Float16 hi, lo;
+              split_hi_lo(__builtin_ldexpf(xr[bt][t], -e), hi, lo);
+              af[t] = alo ? lo : hi;
+            }
           }
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+          for (int p = 0; p < 8; ++p)
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            half8 bf;
+            for (int d = 0; d < 4; ++d) {
+              const auto sw = __builtin_amdgcn_permlane16_swap(w[2 * p][d], w[2 * p + 1][d], false, false);
+              w[2 * p][d] = sw[0];
+              w[2 * p + 1][d] = sw[1];
+            }
 #pragma unroll
-            for (int t = 0; t < 8; ++t) bf[t] = __builtin_bit_cast(half8, w[2 * t + s])[j];
-            acc2[s][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf, acc2[s][j], 0, 0, 0);
-          }
+          for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              half8 bf;
+#pragma unroll
+              for (int t = 0; t < 8; ++t) bf[t] = __builtin_bit_cast(half8, w[2 * t + s])[j];
+              acc2[s][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf, acc2[s][j], 0, 0, 0);
+            }
+        }
       }
+    }
+    if (!fma_loop) {
       // Lane l, register i of acc2[s][j]: A row 4 (l / 16) + i, column 8 (16 s + l % 16) + j, i.e. the
       // hi part of activation row m = 4 (l / 16 % 2) + i in lanes 0-31 and its lo part in lanes
       // 32-63. Each lane writes its 8 consecutive columns as two 16-byte writes, scaled back by
@@ -267,7 +321,15 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
       const int mrow = 4 * (g & 1);
       int er[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) er[i] = __shfl(e, mrow + i);
+      for (int i = 0; i < 4; ++i) er[i] = XF16 ? 0 : __shfl(e, mrow + i);
+      if constexpr (XF16) {
+        if (g >= 2) {
+#pragma unroll
+          for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc2[s][j] = float4v{0.f, 0.f, 0.f, 0.f};
+        }
+      }
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -282,7 +344,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
         }
     }
   }
-  if (fma_loop && col < N) {
+  auto fma_rows = [&](auto evenc) __attribute__((always_inline)) {
     constexpr int U = S::loads;
     constexpr int RB = U * kRowsPerLoad;  // rows of a batch
     const _Float16* bp = B + col + static_cast<size_t>(sub) * N;
@@ -297,7 +359,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         float a[MM];
-        act(k + u * kRowsPerLoad, true, a);
+        act(evenc, k, u, true, a);
         fma_row<MM>(acc, a, w[u]);
       }
     }
@@ -314,11 +376,21 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         float a[MM];
-        act(k + u * kRowsPerLoad, false, a);
+        act(evenc, k, u, false, a);
         if (k + u * kRowsPerLoad + sub < k1) fma_row<MM>(acc, a, w[u]);
       }
     }
+  };
+  if (fma_loop && col < N) {
+    if (std::is_same_v<TX, _Float16> && k0 % 2 == 0) fma_rows(std::true_type{});
+    else fma_rows(std::false_type{});
   }
+
+  // an fp16 output is the fp32 sum rounded once, as a cast of an fp32 output would
+  auto put = [&](size_t i, float v) {
+    if (c_f16) static_cast<_Float16*>(Cv)[i] = static_cast<_Float16>(v);
+    else static_cast<float*>(Cv)[i] = v;
+  };
 
   const int part_row = wave * kRowsPerLoad + sub;
   if constexpr (MM == 1) {
@@ -340,7 +412,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
       for (int w = 1; w < kParts; ++w) mine += red[w][0][t];
     }
     if (ksplit == 1) {
-      if (live) C[c] = mine + (bias != nullptr ? bias[c] : 0.f);
+      if (live) put(c, mine + (bias != nullptr ? bias[c] : 0.f));
       return;
     }
     if (live) store_coherent(part + static_cast<size_t>(kpart) * N + c, mine);
@@ -357,7 +429,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
         for (int b = 0; b < kZBatch; ++b)
           if (z0 + b < ksplit) sum += v[b];
       }
-      if (live) C[c] = sum + (bias != nullptr ? bias[c] : 0.f);
+      if (live) put(c, sum + (bias != nullptr ? bias[c] : 0.f));
     }
     reset_counter(counters + strip * kCounterStride);
     return;
@@ -405,12 +477,13 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
   }
   auto store_out = [&](int i, V v) {
     const int c = group_col(i);
-    float* o = C + static_cast<size_t>(group_row(i)) * N + c;
+    const size_t o = static_cast<size_t>(group_row(i)) * N + c;
     if constexpr (kGW == 4) {
       if (bias != nullptr) v += float4v{bias[c], bias[c + 1], bias[c + 2], bias[c + 3]};
-      *reinterpret_cast<float4v*>(o) = v;
+      if (c_f16) *reinterpret_cast<half4*>(static_cast<_Float16*>(Cv) + o) = __builtin_convertvector(v, half4);
+      else *reinterpret_cast<float4v*>(static_cast<float*>(Cv) + o) = v;
     } else {
-      *o = v + (bias != nullptr ? bias[c] : 0.f);
+      put(o, v + (bias != nullptr ? bias[c] : 0.f));
     }
   };
 
@@ -482,7 +555,7 @@ Split split_for(int K, int ksplit) {
 }
 
 template <typename TX>
-using SkinnyFn = void (*)(const TX*, const _Float16*, float*, const float*, float*, uint32_t*, int, int, int, int, int);
+using SkinnyFn = void (*)(const TX*, const _Float16*, void*, int, const float*, float*, uint32_t*, int, int, int, int, int);
 
 // The schedule of each M and strip width: graph-timed sweeps on MI355X of 2-16 loads per batch,
 // with and without the issue barrier, over M = 1..8 and K x N in {4096^2, 1024 x 3072,
@@ -506,11 +579,12 @@ template <int MM> struct SchedFor<MM, 512> {
 // last arriver's read-back (slices x M x strip width) dominates the exchange, which the narrow
 // strips cut 4x (1 x 4096^2: 9.16 -> 8.63 us; 6 x 4096^2: 14.87 -> 10.98); with many strips the
 // split is shallow already and the 1 KB rows stream slightly better (1 x 4096 x 11008: 16.77 us
-// with 512 columns, 16.90 with 256; 8 x 4096 x 14336: 27.3 vs 31.9).
-int strip_cols(int M, int N) {
-  (void)M;
-  return N <= 8192 ? 256 : 512;
-}
+// with 512 columns, 16.90 with 256). M = 7 and 8 take 256 columns throughout: the matrix-core form
+// needs them, and gains more than the wide rows (fp32 x, 512-column FMA loop -> 256-column matrix
+// cores: 7 x 4096 x 11008 23.8 -> 21.9 us, 8 x 4096 x 11008 25.6 -> 22.1, 8 x 8192 x 9216 42.2 -> 37.7,
+// 7 x 512 x 9000 9.9 -> 7.7, 8 x 8192 x 28672 84.3 -> 82.3, 7 x 8192 x 28672 80.4 -> 81.5); M = 5 and 6
+// do not (5 x 8192 x 9216 34.5 vs 38.9, 6 x 4096 x 14336 24.6 vs 25.5).
+int strip_cols(int M, int N) { return N <= 8192 || M >= 7 ? 256 : 512; }
 
 template <typename TX, int COLS>
 SkinnyFn<TX> skinny_fn_w(int M) {
@@ -525,18 +599,28 @@ SkinnyFn<TX> skinny_fn_w(int M) {
     default: return skinny_kernel<TX, 8, typename SchedFor<8, COLS>::type>;
   }
 }
-// The matrix-core form (skinny_kernel's MF) runs where it pays: M = 8 on 256-column strips with
-// 32..128 K rows per wavefront. Graph-timed against the FMA loop, weights rotated past the
-// Infinity Cache, us (K x N): 4096 x 4096 12.69 vs 12.95, 11008 x 4096 20.50 vs 25.52, 14336 x 4096
-// 24.80 vs 29.29, 4096 x 8192 16.52 vs 19.18. Smaller M lose: one batch per wavefront leaves the
-// matrix-core work and the hi/lo split exposed next to the FMAs they replace (M = 7, 4096^2:
-// 12.62 vs 11.24; M = 2..6: 1.5-3 us slower); so do wavefronts with fewer rows than a batch.
-bool use_mf(int M, int cols, int rows_per_wave) {
-  return M == 8 && cols == 256 && rows_per_wave >= kMfBatch && rows_per_wave <= kMfBatch * kMfMaxBatches;
+// The matrix-core form (skinny_kernel's MF) runs where it pays: 256-column strips and enough K rows
+// per wavefront to hide its work (permutes, hi/lo split) behind the weights' loads, more at smaller M.
+// Graph-timed against the FMA loop, weights rotated past the Infinity Cache, us (K x N, rows per
+// wavefront), fp32 activations: M = 8 4096 x 4096 (32) 12.69 vs 12.95, 11008 x 4096 (86) 20.50 vs
+// 25.52; M = 7 4096 x 8192 (64) 16.36 vs 17.29, 11008 x 4096 21.0 vs 23.5, but 4096 x 4096 12.4 vs
+// 11.3; M = 6 11008 x 4096 21.0 vs 22.2, but 4096 x 8192 16.7 vs 16.3; M = 5 11008 x 4096 21.5 vs
+// 21.8. fp16: M = 8 4096 x 4096 11.7 vs 12.6, 11008 x 4096 20.3 vs 24.0; M = 5 19.8 vs 20.8. With
+// one batch per wavefront and few slices (N > 8192) the FMA loop is the faster and more accurate one
+// at M = 8 too (7 x 1536 x 10240, 32 rows: 10.7 us against 11.9 on the matrix cores).
+bool use_mf(int M, int N, int cols, int rows_per_wave) {
+  return cols == 256 && M >= 5 && rows_per_wave >= (M == 8 && N <= 8192 ? kMfBatch : (M >= 7 ? 64 : 80));
 }
 template <typename TX>
 SkinnyFn<TX> skinny_fn(int M, int cols, bool mf) {
-  if (mf) return skinny_kernel<TX, 8, typename SchedFor<8, 256>::type, true>;
+  if (mf) {
+    switch (M) {
+      case 5: return skinny_kernel<TX, 5, typename SchedFor<5, 256>::type, true>;
+      case 6: return skinny_kernel<TX, 6, typename SchedFor<6, 256>::type, true>;
+      case 7: return skinny_kernel<TX, 7, typename SchedFor<7, 256>::type, true>;
+      default: return skinny_kernel<TX, 8, typename SchedFor<8, 256>::type, true>;
+    }
+  }
   return cols == 256 ? skinny_fn_w<TX, 256>(M) : skinny_fn_w<TX, 512>(M);
 }
 
@@ -575,7 +659,7 @@ int plan_with(int M, int N, int K, int num_cus, int cols) {
 }
 
 template <typename TX>
-int skinny_launch(const TX* A, const uint16_t* B, float* C, const float* bias, int M, int N, int K, int ksplit,
+int skinny_launch(const TX* A, const uint16_t* B, void* C, int c_f16, const float* bias, int M, int N, int K, int ksplit,
                   void* ws, size_t ws_bytes, uint32_t* counters_in, size_t counter_bytes_in, void* stream) {
   if (M < 0 || N < 0 || K < 0 || M > G16_SKINNY_MAX_M || K % 8 != 0 || N % 8 != 0) return G16_E_SHAPE;
   if (M == 0 || N == 0) return G16_OK;
@@ -597,8 +681,8 @@ int skinny_launch(const TX* A, const uint16_t* B, float* C, const float* bias, i
     part = static_cast<float*>(ws);
   }
   const dim3 grid(static_cast<unsigned>(nstrips) * static_cast<unsigned>(sp.ksplit)), block(kThreads);
-  return launch(skinny_fn<TX>(M, cols, use_mf(M, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
-                reinterpret_cast<const _Float16*>(B), C, bias, part, counters, N, K, sp.rows_per_wave, sp.ksplit,
+  return launch(skinny_fn<TX>(M, cols, use_mf(M, N, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
+                reinterpret_cast<const _Float16*>(B), C, c_f16, bias, part, counters, N, K, sp.rows_per_wave, sp.ksplit,
                 nstrips);
 }
 
@@ -665,7 +749,7 @@ extern "C" int g16_skinny_f32in_noalloc(const float* A, const uint16_t* B, float
     const int rc = g16::launch(g16::clear_words, dim3((kWords + 255) / 256), dim3(256), st, counters, kWords);
     if (rc != 0) return rc;
   }
-  return g16::skinny_launch<float>(A, B, C, bias, M, N, K, ksplit, base + G16_NOALLOC_COUNTER_BYTES,
+  return g16::skinny_launch<float>(A, B, C, 0, bias, M, N, K, ksplit, base + G16_NOALLOC_COUNTER_BYTES,
                                    G16_NOALLOC_PARTIAL_BYTES, counters, G16_NOALLOC_COUNTER_BYTES, stream);
 }
 
@@ -688,13 +772,23 @@ extern "C" size_t g16_skinny_counter_bytes(int M, int N, int K, int ksplit) {
 extern "C" int g16_skinny_f32in(const float* A, const uint16_t* B, float* C, const float* bias, int M, int N, int K,
                                 int ksplit, void* workspace, size_t workspace_bytes, uint32_t* counters,
                                 size_t counter_bytes, void* stream) {
-  return g16::skinny_launch<float>(A, B, C, bias, M, N, K, ksplit, workspace, workspace_bytes, counters, counter_bytes,
+  return g16::skinny_launch<float>(A, B, C, 0, bias, M, N, K, ksplit, workspace, workspace_bytes, counters, counter_bytes,
                                    stream);
 }
 
 extern "C" int g16_skinny_f16in(const uint16_t* A, const uint16_t* B, float* C, const float* bias, int M, int N,
                                 int K, int ksplit, void* workspace, size_t workspace_bytes, uint32_t* counters,
                                 size_t counter_bytes, void* stream) {
-  return g16::skinny_launch<_Float16>(reinterpret_cast<const _Float16*>(A), B, C, bias, M, N, K, ksplit, workspace,
+  return g16::skinny_launch<_Float16>(reinterpret_cast<const _Float16*>(A), B, C, 0, bias, M, N, K, ksplit, workspace,
                                       workspace_bytes, counters, counter_bytes, stream);
+}
+
+extern "C" int g16_skinny(const void* A, int a_is_f32, const uint16_t* B, void* C, int c_is_f16, const float* bias, int M,
+                          int N, int K, int ksplit, void* workspace, size_t workspace_bytes, uint32_t* counters,
+                          size_t counter_bytes, void* stream) {
+  const int f16 = c_is_f16 != 0 ? 1 : 0;
+  return a_is_f32 ? g16::skinny_launch<float>(static_cast<const float*>(A), B, C, f16, bias, M, N, K, ksplit, workspace,
+                                              workspace_bytes, counters, counter_bytes, stream)
+                  : g16::skinny_launch<_Float16>(static_cast<const _Float16*>(A), B, C, f16, bias, M, N, K, ksplit,
+                                                 workspace, workspace_bytes, counters, counter_bytes, stream);
 }

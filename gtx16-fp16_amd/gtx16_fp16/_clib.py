@@ -63,6 +63,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "g16_pack_decode_weight": (_I, [_P, _P, _I, _I, _P]),
     "g16_skinny_strips_f32in": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
     "g16_skinny_strips_f16in": (_I, [_P, _P, _P, _P, _I, _I, _I, _P]),
+    "g16_skinny": (_I, [_P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _SZ, _P, _SZ, _P]),
+    "g16_skinny_strips": (_I, [_P, _I, _P, _P, _I, _P, _I, _I, _I, _P]),
     "g16_skinny_strips_route": (_I, [_I, _I, _I, _I]),
     "g16_gemm_clock": (_I, [_P, _P]),
     "g16_peak_flops_per_lane_iter": (ctypes.c_double, [_I]),
@@ -107,8 +109,8 @@ _fast = None
 
 def fast():
     """The CPython extension ``_g16fast`` (built next to the library from ``csrc/fastcall.c``), bound
-    to the loaded library: ``skinny_f32in``, ``skinny_strips_f32in`` and ``mm_t_gemm`` take the same arguments as the C
-    entry points (pointers as ints or None) and return their status, with argument conversion
+    to the loaded library: ``skinny``, ``skinny_f32in``, ``skinny_strips``, ``skinny_strips_f32in`` and
+    ``mm_t_gemm`` take the same arguments as the C entry points (pointers as ints or None) and return their status, with argument conversion
     that costs a few ns per argument instead of ctypes' ~0.1 us. Missing -> ``RuntimeError``."""
     global _fast
     if _fast is not None:
@@ -126,7 +128,9 @@ def fast():
             spec.loader.exec_module(mod)
             mod.bind(ctypes.cast(lib.g16_skinny_f32in, ctypes.c_void_p).value,
                      ctypes.cast(lib.g16_mm_t_gemm, ctypes.c_void_p).value,
-                     ctypes.cast(lib.g16_skinny_strips_f32in, ctypes.c_void_p).value)
+                     ctypes.cast(lib.g16_skinny_strips_f32in, ctypes.c_void_p).value,
+                     ctypes.cast(lib.g16_skinny, ctypes.c_void_p).value,
+                     ctypes.cast(lib.g16_skinny_strips, ctypes.c_void_p).value)
             _fast = mod
     return _fast
 

@@ -72,7 +72,7 @@ class FastLinear(nn.Module):
     def __init__(self, in_features: int, out_features: int, bias: bool = True, device=None):
         super().__init__()
         self.in_features, self.out_features = in_features, out_features
-        # (M, device index, prepack_decode) -> (PreparedCall of the split kernel or None, ksplit,
+        # (M, device index, prepack_decode, fp32 activations) -> (PreparedCall of the split kernel or None, ksplit,
         # (partial, counter) bytes, weight pointer, bias pointer, PreparedCall of the decode-layout
         # kernel or None) for the token-by-token fast path; None in the first field when the weight or
         # bias the pointers name cannot be handed to the kernel (the call then takes the general
@@ -107,8 +107,8 @@ class FastLinear(nn.Module):
         layer's ``.weight`` (its shape, device or dtype) as they would on nn.Linear."""
         return self.weight_t.t()
 
-    def _decode_entry(self, M: int, dev: torch.device):
-        key = (M, dev.index, self.prepack_decode)
+    def _decode_entry(self, M: int, dev: torch.device, f32: int = 1):
+        key = (M, dev.index, self.prepack_decode, f32)
         w, b = self.weight_t, self.bias
         bptr = None if b is None else b.data_ptr()
         entry = self._skinny.get(key)
@@ -126,11 +126,11 @@ class FastLinear(nn.Module):
                 # the split kernel on weight_t always (also the decode layout's stand-in while its copy
                 # cannot be built: under graph capture)
                 ksplit = lib.g16_skinny_plan(M, N, K, _sm_count(dev))
-                pl = PreparedCall(_clib.fast().skinny_f32in, "skinny GEMM")
+                pl = PreparedCall(_clib.fast().skinny, "skinny GEMM")
                 sizes = (lib.g16_skinny_workspace_bytes(M, N, K, ksplit),
                          lib.g16_skinny_counter_bytes(M, N, K, ksplit))
-                if self.prepack_decode and lib.g16_skinny_strips_route(M, N, K, 1):
-                    pls = PreparedCall(_clib.fast().skinny_strips_f32in, "skinny GEMM (decode layout)")
+                if self.prepack_decode and lib.g16_skinny_strips_route(M, N, K, f32):
+                    pls = PreparedCall(_clib.fast().skinny_strips, "skinny GEMM (decode layout)")
             entry = (pl, ksplit, sizes, w.data_ptr(), bptr, pls)
             self._skinny[key] = entry
         return entry
@@ -190,24 +190,25 @@ class FastLinear(nn.Module):
         # Fast path for small batches (generation): minimal Python per call (linear.py:49-64).
         # Unlike the reference, the weight's support is checked (once per layer and M), so a
         # FastLinear built directly with K or N not a multiple of 8 still takes the fallback.
-        if x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0:
+        if x.is_cuda and x.dtype in (torch.float32, torch.float16) and x.is_contiguous() and x.data_ptr() % 16 == 0:
             K, N = self.in_features, self.out_features
             M = x.numel() // K if shape[-1] == K else -1
             if 0 < M <= SKINNY_MAX_M:
                 dev = x.device
-                pl, ksplit, sizes, wptr, bptr, pls = self._decode_entry(M, dev)
+                f32 = 1 if x.dtype == torch.float32 else 0
+                pl, ksplit, sizes, wptr, bptr, pls = self._decode_entry(M, dev, f32)
                 if pl is not None:
                     stream = stream_handle(dev.index or 0)
-                    out = torch.empty(*shape[:-1], N, device=dev, dtype=torch.float32)
+                    out = torch.empty(*shape[:-1], N, device=dev, dtype=x.dtype)
                     wd = 0
                     if pls is not None:
                         w = self.weight_t
                         wd = self._wd_ptr if self._wd_key == (wptr, tensor_version(w), w.device) else self._decode_weight()
                     if wd:
-                        pls(x.data_ptr(), wd, out.data_ptr(), bptr, M, N, K, stream)
+                        pls(x.data_ptr(), f32, wd, out.data_ptr(), 1 - f32, bptr, M, N, K, stream)
                     else:
                         bufs = split_buffers(dev, stream, *sizes)
-                        pl(x.data_ptr(), wptr, out.data_ptr(), bptr, M, N, K, ksplit, *bufs, stream)
+                        pl(x.data_ptr(), f32, wptr, out.data_ptr(), 1 - f32, bptr, M, N, K, ksplit, *bufs, stream)
                     return out
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype not in (torch.float16, torch.float32):
@@ -231,7 +232,7 @@ class FastLinear(nn.Module):
                   and _clib.load().g16_skinny_strips_route(M, self.out_features, self.in_features,
                                                            int(x2.dtype == torch.float32))
                   and self._decode_weight()):
-                # token-by-token calls the fast path above does not take (fp16 activations, views):
+                # token-by-token calls the fast path above does not take (views, other dtypes):
                 # the decode layout where the library's rule expects a gain
                 y = skinny_strips(x2, self._wd, b)
             else:

@@ -181,7 +181,7 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
 
     x2d = _aligned(x2d)
     if M <= SKINNY_MAX_M:  # memory-bound path, fp32 math
-        out = torch.empty(M, N, device=dev, dtype=torch.float32)
+        out = torch.empty(M, N, device=dev, dtype=out_dtype)
         key = (-M, N, K, dev.index or 0)
         plan = _routes.get(key)
         if plan is None:
@@ -191,10 +191,10 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
             _remember(key, plan)
         ksplit = plan[0]
         bufs = split_buffers(dev, stream, plan[1], plan[2])
-        fn = _clib.fast().skinny_f32in if x2d.dtype == torch.float32 else lib.g16_skinny_f16in
-        _clib.check(fn(x2d.data_ptr(), w_t.data_ptr(), out.data_ptr(), bptr, M, N, K, ksplit, *bufs, stream),
-                    "skinny GEMM")
-        return out if out_dtype == torch.float32 else out.to(out_dtype)
+        _clib.check(_clib.fast().skinny(x2d.data_ptr(), 1 if x2d.dtype == torch.float32 else 0, w_t.data_ptr(),
+                                        out.data_ptr(), 1 if out_dtype == torch.float16 else 0, bptr, M, N, K, ksplit,
+                                        *bufs, stream), "skinny GEMM")
+        return out
 
     # GEMM path: fp16 inputs, with per-row power-of-two scaling for rows that would overflow. One
     # library call runs the rowscale cast into `scratch` and the GEMM on the planned route: the

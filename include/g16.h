@@ -224,7 +224,7 @@ int g16_hgemm_tile(int M, int N, int K, int num_cus, int* rows, int* cols);
  * configuration skinny_config (src/gtx16_fp16/ops.py:45-51,78-84; src/gtx16_fp16/linear.py:49-64).
  * A is read with 16-byte alignment (A must be 16-byte aligned, like B).
  * The kernel streams B once with 16-byte loads; K is split over ksplit workgroups per strip of
- * g16_skinny_strip_cols(M, N) columns (256 up to N = 8192, 512 above) and reduced
+ * g16_skinny_strip_cols(M, N) columns (256 up to N = 8192 and for M >= 7, else 512) and reduced
  * deterministically (last arriving workgroup, slice order). C needs no zero-fill.
  * The split workspace (ksplit * M * N * 4 bytes) must stay below 2 GiB (G16_E_SPLIT otherwise).
  * g16_skinny_plan() returns the ksplit this library would choose for num_cus compute units; the
@@ -236,6 +236,11 @@ int g16_skinny_f32in(const float* A, const uint16_t* B, float* C, const float* b
 int g16_skinny_f16in(const uint16_t* A, const uint16_t* B, float* C, const float* bias, int M,
                      int N, int K, int ksplit, void* workspace, size_t workspace_bytes,
                      uint32_t* counters, size_t counter_bytes, void* stream);
+/* Either activation type with an fp32 or fp16 output: c_is_f16 != 0 rounds each fp32 result once
+ * (nearest-even) as it is stored, the bits a cast of the fp32 output would give. */
+int g16_skinny(const void* A, int a_is_f32, const uint16_t* B, void* C, int c_is_f16,
+               const float* bias, int M, int N, int K, int ksplit, void* workspace,
+               size_t workspace_bytes, uint32_t* counters, size_t counter_bytes, void* stream);
 size_t g16_skinny_workspace_bytes(int M, int N, int K, int ksplit);
 size_t g16_skinny_counter_bytes(int M, int N, int K, int ksplit);
 int g16_skinny_plan(int M, int N, int K, int num_cus);
@@ -275,6 +280,9 @@ int g16_skinny_strips_f32in(const float* A, const uint16_t* wd, float* C, const 
                             int N, int K, void* stream);
 int g16_skinny_strips_f16in(const uint16_t* A, const uint16_t* wd, float* C, const float* bias,
                             int M, int N, int K, void* stream);
+/* Either activation type with an fp32 or fp16 output, as g16_skinny. */
+int g16_skinny_strips(const void* A, int a_is_f32, const uint16_t* wd, void* C, int c_is_f16,
+                      const float* bias, int M, int N, int K, void* stream);
 /* 1 where g16_skinny_strips_* is expected to be faster than g16_skinny_* for this product (a
  * measured rule: M <= 2, or small weights, or fp16 activations at M = 3 and at M = 4 up to
  * N = 8192); 0 otherwise or for sizes out of range. x_f32: 1 for fp32 activations, 0 for fp16. */
