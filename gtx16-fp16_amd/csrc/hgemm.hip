@@ -44,6 +44,11 @@
 //     row's scale (rowscale_math.hpp, the rowscale kernel's arithmetic) and writes the scaled fp16
 //     rows into LDS as the stage images of every K step, which then stay resident; only B streams
 //     through the ring. No fp16 copy of A goes to HBM and no separate rowscale launch runs.
+//   * Direct fp32 A (mm_t's GEMM path in one launch, no fp16 copy of x in HBM): the tiles read x
+//     themselves and cast it on the way into their A stages, through registers on the unsplit 256x256
+//     tile with few columns (direct_route), through a ring of fp32 LDS stages on the 4-wavefront tiles
+//     (stream_route). A row is rescaled as soon as a value of it leaves fp16's range, its sums so far
+//     with it (exact), so no pass over the row has to come first and no slice waits for another.
 //   * Speculative fp16 A (the 4-wavefront tiles with fp16 activations, mm_t's GEMM path in one
 //     launch): a row whose |max| does not exceed the threshold has scale 1, and its rowscale cast is
 //     the activation itself. So the GEMM streams x as A and tracks the largest |x| it multiplies
@@ -171,6 +176,8 @@ struct TileCfg {
 
 // K steps the resident-A tile keeps in LDS: 20 x 4 KB of A plus the 64 KB B ring (K <= 1280).
 constexpr int kResidentSteps = 20;
+// fp32 stages of the 4-wavefront tiles' direct A: the step being cast and three in flight.
+constexpr int kXStages = 4;
 
 using Cfg256 = TileCfg<256, 256, 32, 2, 4, 4, true>;  // 8 wavefronts (two per SIMD), 4-stage ring, 128 KB
 using Cfg256n = TileCfg<256, 128, 32, 2, 4, 4, true>;  // the same schedule on half the columns, 96 KB
@@ -246,9 +253,10 @@ __device__ inline void phase_barrier() { asm volatile("s_barrier" ::: "memory");
 // workgroup; split, by the slice that arrives last, over every slice in slice order. A split
 // slice that saw such a value publishes its rows' |max| in place of its partial tile. A tile that
 // is computed again stores 1 into *spec_miss (when not NULL; pinned host memory).
-// DIRECT: A is unused; the kernel streams the fp32 activations X through registers, casts them on the
-// way into the A stages and rescales a row as soon as a value of it leaves fp16's range (the 256x256
-// tile, unsplit).
+// DIRECT: A is unused; the kernel streams the fp32 activations X itself, casts them on the way into the
+// A stages and rescales a row as soon as a value of it leaves fp16's range: the unsplit 256x256 tile
+// (through registers), and the 4-wavefront tiles with 64-deep K steps, split or not (through a ring of
+// fp32 stages in LDS; a slice rescales by what it has seen, and publishes its sums in units of 1).
 template <class Cfg, bool OUT_F16, bool SPLITK, bool PACKED_A = false, bool PACKED_B = false, bool RESIDENT = false,
           bool SPEC = false, bool DIRECT = false>
 __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
@@ -264,17 +272,20 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
                 "resident A: the unsplit 32x128 tile");
   static_assert(!SPEC || (Cfg::WAVES == 4 && !Cfg::MF16 && !PACKED_A && !PACKED_B && !RESIDENT),
                 "speculative A: the 4-wavefront tiles, 32x32x16 blocks (lane l's A rows are l % 32)");
-  static_assert(!DIRECT || (Cfg::WAVES == 8 && Cfg::BK == 32 && Cfg::MF16 && !SPLITK && !PACKED_A && !RESIDENT && !SPEC),
-                "direct A: the unsplit 8-wavefront tiles");
-  constexpr int A_STAGES = RESIDENT ? kResidentSteps : NSTAGE;
+  constexpr bool STREAM = DIRECT && Cfg::WAVES == 4;  // direct A on the 4-wavefront tiles
+  static_assert(!DIRECT || (Cfg::WAVES == 8 && Cfg::BK == 32 && Cfg::MF16 && !SPLITK && !PACKED_A && !RESIDENT && !SPEC) ||
+                    (STREAM && Cfg::BK == 64 && !Cfg::MF16 && NSTAGE == 4 && !PACKED_A && !PACKED_B && !RESIDENT && !SPEC),
+                "direct A: the unsplit 256x256 tile, the 4-wavefront tiles with 64-deep K steps");
+  constexpr int A_STAGES = RESIDENT ? kResidentSteps : (STREAM ? 2 : NSTAGE);
   __shared__ __attribute__((aligned(1024))) unsigned char sA[A_STAGES][Cfg::A_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char sB[NSTAGE][Cfg::B_BYTES];
+  __shared__ __attribute__((aligned(1024))) unsigned char sX[STREAM ? kXStages : 1][STREAM ? BM * BK * 4 : 16];
   __shared__ float s_scale[(RESIDENT || SPEC) ? BM : 1];
   __shared__ float s_rowmax[SPEC ? BM : 1];  // speculative recomputation: the rows' |max|, then 2^-e
   // direct A: the factors 2^-e of the rows' exponents so far (0 for an infinite row); per ring stage
   // and staging wavefront, the K step whose A raised an exponent, and that step's factors for the
   // wavefront's rows
-  __shared__ float s_fac[DIRECT ? BM : 1];
+  __shared__ __attribute__((aligned(16))) float s_fac[DIRECT ? BM : 4];
   __shared__ int s_evt[DIRECT ? NSTAGE : 1][DIRECT ? Cfg::WAVES : 1];
   __shared__ __attribute__((aligned(16))) float s_delta[DIRECT ? NSTAGE : 1][DIRECT ? BM : 4];
   const uint32_t sA_lds = lds_base(&sA[0][0]), sB_lds = lds_base(&sB[0][0]);
@@ -676,6 +687,174 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       }
       if (it < nk) step(std::integral_constant<int, 0>{}, it);
     };
+    // Direct A on the 4-wavefront tiles. As in kloop4, step j runs the MFMAs of step j on fragments
+    // already in registers, reads step j+1's fragments and issues step j+NSTAGE's B. Of A, each
+    // wavefront moves its own BM/4 rows: DMA of the fp32 values of step j+5 into a ring of kXStages
+    // stages, which no other wavefront reads, and the cast of step j+2 from there (read at the step's
+    // start, written at its end, the MFMAs between) into the fp16 stage that step j's fragments came
+    // from. The wait that ends a step leaves the DMA of two steps in flight: A's step j+3 (cast next)
+    // and B's step j+2 (read next) have then landed.
+    //   These tiles are bound by launches and by the memory's latency, not by their LDS or VALU: the
+    // rowscale launch goes (5 us at 64 x 4096), the cast rides in the K loop's idle issue slots.
+    //   Rescaling as on the 256x256 tile: a step with a value past fp16's range raises its row's
+    // exponent, scales its values, and leaves the factor for the accumulators, which every wavefront
+    // applies before its MFMAs of that step; the row's later steps are scaled as they are cast.
+    auto stream_loop = [&]() __attribute__((always_inline)) {
+      constexpr int RW = BM / 4;              // rows per wavefront
+      constexpr int AI = RW / 4;              // its DMA instructions per step (4 rows of 256 bytes each)
+      constexpr int H = RW / 8;               // 8-row groups: lane l casts 8 values of row 8 h + l / 8
+      constexpr int PARTS = AI + Cfg::B_INSTR;
+      static_assert(!STREAM || (RW % 8 == 0 && 2 * PARTS <= 63), "whole groups, vmcnt range");
+      const float* const xb = static_cast<const float*>(X) + static_cast<size_t>(m0) * K;
+      const uint32_t sX_lds = lds_base(&sX[0][0]);
+      const int xrow = wave * RW + (lane >> 4), xpiece = lane & 15;  // DMA: this lane's first row, its 16 bytes
+      auto dma_x = [&](int s, int d) __attribute__((always_inline)) {
+        const int k0 = kbeg + s * BK, row = xrow + 4 * d;
+        const __amdgpu_buffer_rsrc_t rx =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xb + k0), 0, 0x7fffffff, kRawBufferDword3);
+        const bool ok = m0 + row < M && k0 + xpiece * 4 < kend;
+        dma16(rx, sX_lds + (s % kXStages) * (BM * BK * 4) + (wave * RW + 4 * d) * (BK * 4),
+              ok ? static_cast<uint32_t>((row * K + xpiece * 4) * 4) : kOob);
+      };
+      auto dma_b = [&](int s, int d, __amdgpu_buffer_rsrc_t rb) __attribute__((always_inline)) {
+        dma_op(s % NSTAGE, kbeg + s * BK, rb, rb, Cfg::A_INSTR + d);
+      };
+      const int crow = wave * RW + (lane >> 3), cc = lane & 7;  // cast: this lane's first row, its 8 values
+      int scaled = 0;    // 1: some row this wavefront casts has a factor < 1
+      float fac[H];      // this lane's rows' factors (s_fac)
+#pragma unroll
+      for (int h = 0; h < H; ++h) fac[h] = 1.f;
+      float4v v[H][2];
+      auto read_x = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const float4v* p = reinterpret_cast<const float4v*>(&sX[s % kXStages][(crow + 8 * h) * (BK * 4) + cc * 32]);
+          v[h][0] = p[0];
+          v[h][1] = p[1];
+        }
+      };
+      auto absmax4 = [](float m, float4v x) __attribute__((always_inline)) {
+        m = fmaxf(fmaxf(m, fabsf(x.x)), fabsf(x.y));
+        return fmaxf(fmaxf(m, fabsf(x.z)), fabsf(x.w));
+      };
+      auto cast_x = [&](int s) __attribute__((always_inline)) {
+        if (__builtin_expect(__builtin_amdgcn_readfirstlane(scaled), 0)) {
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            v[h][0] *= fac[h];
+            v[h][1] *= fac[h];
+          }
+        }
+        float m = 0.f;
+#pragma unroll
+        for (int h = 0; h < H; ++h) m = absmax4(absmax4(m, v[h][0]), v[h][1]);
+        if (__builtin_expect(__any(m > kHalfMax), 0)) {
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            const int r = crow + 8 * h;
+            float rm = absmax4(absmax4(0.f, v[h][0]), v[h][1]);
+            rm = fmaxf(rm, __shfl_xor(rm, 1));
+            rm = fmaxf(rm, __shfl_xor(rm, 2));
+            rm = fmaxf(rm, __shfl_xor(rm, 4));
+            float f = 1.f;
+            if (rm > kHalfMax) {
+              int e;
+              float sc;
+              row_exponent(rm, texp, e, sc);
+              f = e == kInfExp ? 0.f : ldexpf(1.f, -e);
+            }
+            v[h][0] *= f;
+            v[h][1] *= f;
+            fac[h] *= f;
+            s_delta[s % NSTAGE][r] = f;  // the row's 8 lanes write the same values
+            s_fac[r] = fac[h];
+          }
+          s_evt[s % NSTAGE][wave] = s;
+          scaled = 1;
+        }
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+          const int r = crow + 8 * h;
+          const half4 lo = __builtin_convertvector(v[h][0], half4), hi = __builtin_convertvector(v[h][1], half4);
+          *reinterpret_cast<half8*>(&sA[s & 1][r * (BK * 2) + ((cc ^ Cfg::swz_a(r)) << 4)]) =
+              __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+      };
+      // each wavefront resets what it alone writes; the others read it past the barriers below
+      if (lane < NSTAGE) s_evt[lane][wave] = -1;
+      if (lane < RW) s_fac[wave * RW + lane] = 1.f;
+      if (nk > 0) {
+#pragma unroll
+        for (int s = 0; s < NSTAGE; ++s) {
+          const __amdgpu_buffer_rsrc_t rb = rsrc_b(kbeg + s * BK);
+#pragma unroll
+          for (int d = 0; d < AI; ++d) dma_x(s, d);
+#pragma unroll
+          for (int d = 0; d < Cfg::B_INSTR; ++d) dma_b(s, d, rb);
+        }
+      }
+      wait_dma_le<2 * PARTS + Cfg::B_INSTR>();  // A's steps 0 and 1
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        read_x(s);
+        cast_x(s);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the fp32 stage 0 has been read
+      if (nk > 0) {
+#pragma unroll
+        for (int d = 0; d < AI; ++d) dma_x(4, d);
+      }
+      wait_dma_le<2 * PARTS>();  // A's step 2, B's steps 0 and 1
+      __syncthreads();
+      if (nk > 0) read_frags(0, 0, 0);
+      int evt = s_evt[0][lane & 3];
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __syncthreads();  // every wavefront holds step 0 in registers: its stages may be refilled
+      b_run = B + static_cast<size_t>(kbeg + NSTAGE * BK) * N + n0;
+      auto step = [&](auto hc, int j) __attribute__((always_inline)) {
+        constexpr int FB = decltype(hc)::value;
+        const __amdgpu_buffer_rsrc_t rb = rsrc_b_next(0);
+        if (__builtin_expect(__any(evt == j), 0)) {
+          // rows whose exponent was raised at this step: their sums so far follow
+#pragma unroll
+          for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const int r0 = wm0 + 32 * i + 8 * q;
+              if (__builtin_amdgcn_readlane(evt, r0 / RW) == j) {
+                const float4v f = *reinterpret_cast<const float4v*>(&s_delta[j % NSTAGE][r0 + 4 * fk]);
+#pragma unroll
+                for (int jj = 0; jj < TN; ++jj)
+#pragma unroll
+                  for (int r = 0; r < 4; ++r) acc[i][jj][4 * q + r] *= f[r];
+              }
+            }
+        }
+        evt = s_evt[(j + 1) % NSTAGE][lane & 3];
+        read_x(j + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+          if (p < AI) dma_x(j + 5, p);
+          else dma_b(j + NSTAGE, p - AI, rb);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = p * NMFMA / PARTS; q < (p + 1) * NMFMA / PARTS; ++q) mfma_op(FB, q);
+#pragma unroll
+          for (int f = p * NFRAG / PARTS; f < (p + 1) * NFRAG / PARTS; ++f) frag_op(FB ^ 1, (j + 1) % NSTAGE, f, (j + 1) & 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        cast_x(j + 2);
+        wait_dma_le<2 * PARTS>();  // A's step j+3, B's step j+2 (this wavefront's part)
+        __syncthreads();
+      };
+      int it = 0;
+      for (; it + 1 < nk; it += 2) {
+        step(std::integral_constant<int, 0>{}, it);
+        step(std::integral_constant<int, 1>{}, it + 1);
+      }
+      if (it < nk) step(std::integral_constant<int, 0>{}, it);
+    };
     if constexpr (Cfg::WAVES == 8) {
       // Ping-pong schedule for two wavefronts per SIMD. Wavefronts 0-3 (group 0) and 4-7 (group 1)
       // land one of each on every SIMD. Each wavefront alternates a memory phase M_j (fragment reads
@@ -975,7 +1154,8 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       }
       if (grp == 0) phase_barrier();  // every wavefront passes the same number of barriers
     } else {
-      if constexpr (RESIDENT) kloop4(std::true_type{}, std::false_type{});
+      if constexpr (STREAM) stream_loop();
+      else if constexpr (RESIDENT) kloop4(std::true_type{}, std::false_type{});
       else kloop4(std::false_type{}, std::false_type{});
     }
     wait_dma_le<0>();  // no DMA may still be writing LDS past this point
@@ -1067,7 +1247,22 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       }
     }
 
+    // 1 / factor: a power of two's exponent negated, infinity for a row's factor 0
+    auto inv_factor = [](float f) { return __uint_as_float(f == 0.f ? 0x7f800000u : 0x7f000000u - __float_as_uint(f)); };
     // ---- split-K: publish this slice, let the last slice reduce ----
+    if constexpr (SPLITK && STREAM) {
+      // the slice's rows have factors of their own: its sums leave in units of 1
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float4v f = *reinterpret_cast<const float4v*>(&s_fac[wm0 + 32 * i + 8 * q + 4 * fk]);
+#pragma unroll
+          for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] *= inv_factor(f[r]);
+        }
+    }
     if constexpr (SPLITK) {
       constexpr uint32_t TILE_BYTES = BM * BN * 4;
       // Each wavefront stores its accumulators in its own register order: slot s of the wavefront is
@@ -1233,9 +1428,15 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       for (int q = 0; q < 4; ++q) {
         const int grow = m0 + wm0 + 32 * ri + (lane >> 3) + 8 * q;
         if constexpr (DIRECT) {
-          // 1 / factor: a power of two's exponent negated, infinity for a row's factor 0
-          const uint32_t f = __float_as_uint(s_fac[grow - m0]);
-          erow[ri][q] = __uint_as_float(f == 0u ? 0x7f800000u : 0x7f000000u - f);
+          if constexpr (SPLITK) {
+            // 1, but not a constant to the compiler: the other routes' scale, bias and fp16 cast are one
+            // fused instruction with one rounding, and without a multiply it would add, then cast
+            float one = 1.f;
+            asm volatile("" : "+v"(one));
+            erow[ri][q] = one;
+          } else {
+            erow[ri][q] = inv_factor(s_fac[grow - m0]);
+          }
         } else {
           erow[ri][q] = (RESIDENT || respec) ? s_scale[grow - m0]
                                              : (SPEC ? 1.f : (rscale != nullptr && grow < M ? rscale[grow] : 1.f));
@@ -1499,9 +1700,16 @@ using GemmFn = void (*)(const _Float16*, const _Float16*, void*, const float*, c
 template <bool OUT_F16>
 GemmFn<OUT_F16> gemm_fn(Tile t, bool splitk, bool packed, bool packed_b, bool resident = false, bool spec = false,
                         bool direct = false) {
-  if (direct)
-    return packed_b ? hgemm_kernel<Cfg256, OUT_F16, false, false, true, false, false, true>
-                    : hgemm_kernel<Cfg256, OUT_F16, false, false, false, false, false, true>;
+  if (direct) {
+    switch (t) {
+      case Tile::T32: return splitk ? hgemm_kernel<Cfg32, OUT_F16, true, false, false, false, false, true> : hgemm_kernel<Cfg32, OUT_F16, false, false, false, false, false, true>;
+      case Tile::T64: return splitk ? hgemm_kernel<Cfg64, OUT_F16, true, false, false, false, false, true> : hgemm_kernel<Cfg64, OUT_F16, false, false, false, false, false, true>;
+      case Tile::T64x64: return splitk ? hgemm_kernel<Cfg64x64, OUT_F16, true, false, false, false, false, true> : hgemm_kernel<Cfg64x64, OUT_F16, false, false, false, false, false, true>;
+      default:
+        return packed_b ? hgemm_kernel<Cfg256, OUT_F16, false, false, true, false, false, true>
+                        : hgemm_kernel<Cfg256, OUT_F16, false, false, false, false, false, true>;
+    }
+  }
   if (spec) {
     // speculative fp16 A on the 4-wavefront tiles
     if (splitk) {
@@ -1592,6 +1800,22 @@ bool direct_route(const Plan& p, int N, int K, int ksplit, int num_cus) {
 // has a finite cast (it rescales only rows that leave fp16's range).
 constexpr int kDirectMaxTexp = 15;
 
+// fp32 activations also run as one direct launch on the 4-wavefront tiles with 64-deep K steps, where
+// the cast's launch costs more than streaming A at 4 bytes instead of 2: for up to 64 rows always; above,
+// past K = 4096 (the cast reads such rows twice), and on short slices of split grids or of many rows.
+// Graph-timed, rotated operands, cast + GEMM -> direct (us, M x K x N): 32x128 tiles 64 x 1024^2 10.4 ->
+// 9.4, 64 x 4096 x 1024 14.5 -> 11.5, 16 x 4096^2 19.6 -> 14.7, 40 x 11008 x 5120 59.2 -> 37.1, 9 x
+// 14336 x 512 37.0 -> 17.5; 64x128 tiles 64 x 4096 x 11008 34.2 -> 33.6, 128 x 6144 x 8192 47.9 -> 41.7;
+// 64x64 tiles 256 x 4096 x 1024 18.1 -> 15.3, 1024^3 13.5 -> 11.9, 160 x 11008 x 1536 49.8 -> 32.4. Not
+// taken: 256 x 1024^2 11.3 -> 11.3 (11.4 -> 12.3 with a row past fp16's range), 256 x 2048 x 4096 16.5
+// -> 18.2, 333 x 4096^2 (64x128) 37.5 -> 39.7.
+bool stream_route(const Plan& p, int M, int K, const KSplit& ks) {
+  if (K <= 0) return false;
+  if (p.tile == Tile::T32) return true;
+  if (p.tile != Tile::T64 && p.tile != Tile::T64x64) return false;
+  return M <= 64 || K > 4096 || (ks.kchunk <= 1024 && (ks.ksplit > 1 || M >= 512 || K <= 768));
+}
+
 // A speculative launch (mm_t's GEMM path in one launch for fp16 x on the 4-wavefront tiles): log2
 // of the threshold (>= kSpecMinTexp), the largest fp16 bit pattern not above it, and the weight's
 // history slot (or NULL).
@@ -1624,7 +1848,7 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   const KSplit ks = ksplit_for(K, ksplit);
   if (num_cus <= 0) num_cus = stream_cus(static_cast<hipStream_t>(stream));
   Plan p = choose_tile(M, N, K, num_cus);
-  if (direct ? !direct_route(p, N, K, ks.ksplit, num_cus) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
+  if (direct ? !direct_route(p, N, K, ks.ksplit, num_cus) && !stream_route(p, M, K, ks) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
   const bool spec = sp != nullptr;
   if (spec && (!four_wave(p.tile) || packed ||
                ks.ksplit > kSpecMaxSplit || sp->texp < kSpecMinTexp))
@@ -1906,6 +2130,16 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   if (scratch_bytes < g16_mm_t_scratch_bytes(M, N, K, num_cus)) return G16_E_WORKSPACE;
   if (x_is_f32 && texp <= g16::kDirectMaxTexp && g16_mm_t_direct_route(M, N, K, num_cus) == 1)
     return g16_mm_t_direct(static_cast<const float*>(x), w_t, 0, out, out_is_f16, bias, thresh, M, N, K, num_cus, stream);
+  if (x_is_f32 && texp <= g16::kDirectMaxTexp) {
+    // one launch: the tiles stream x and cast it themselves (the scratch stays unused)
+    const int ks = g16_hgemm_plan(M, N, K, num_cus);
+    if (g16::stream_route(g16::choose_tile(M, N, K, num_cus), M, K, g16::ksplit_for(K, ks))) {
+      if (!g16::aligned16(x)) return G16_E_ALIGN;
+      const g16::ResidentCast rc{x, 1, texp};
+      return g16::gemm_launch(nullptr, w_t, out, out_is_f16 != 0, bias, nullptr, M, N, K, ks, num_cus, workspace,
+                              workspace_bytes, counters, counter_bytes, stream, false, false, &rc, nullptr, true);
+    }
+  }
   const bool packed = g16_hgemm_use_packed(M, N, K, num_cus) == 1;
   auto* y = static_cast<uint16_t*>(scratch);
   auto* s = reinterpret_cast<float*>(static_cast<unsigned char*>(scratch) + g16::round256(g16::cast_bytes(M, K, packed)));
