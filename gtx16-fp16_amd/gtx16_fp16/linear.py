@@ -9,9 +9,10 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _clib
-from .kernels import SKINNY_MAX_M, PreparedCall, split_buffers, stream_handle
-from .ops import (STRIPS_MAX_M, _is_target, _sm_count, is_affected, mm_t, mm_t_prepacked, pack_decode_weight,
-                  pack_weight, prepacked_route, skinny_strips, supported, tensor_version)
+from .kernels import SKINNY_MAX_M, PreparedCall, scratch_buffer, split_buffers, stream_handle
+from .ops import (ROW_SCALE_THRESHOLD, STRIPS_MAX_M, _gemm_route, _is_target, _sm_count, _spec_history, is_affected, mm_t,
+                  mm_t_prepacked, pack_decode_weight, pack_weight, prepacked_route, skinny_strips, supported,
+                  tensor_version)
 
 
 class FastLinear(nn.Module):
@@ -174,6 +175,34 @@ class FastLinear(nn.Module):
             self._wd_ptr = self._wd.data_ptr()
         return self._wd_ptr
 
+    def _small_gemm(self, x: torch.Tensor, M: int) -> torch.Tensor | None:
+        # mm_t's GEMM call for a contiguous, aligned fp32 or fp16 x of M > 8 rows where the plan is one
+        # of the smaller tiles, whose calls are bound by host time: the same checks as supported() and
+        # mm_t, once, and no reshapes (64 x 4096 x 1024: 15.7 us per call through the general path).
+        # None: not that case (the general path then decides).
+        w, b, dev = self.weight_t, self.bias, x.device
+        K, N = self.in_features, self.out_features
+        if not (w.dtype == torch.float16 and w.device == dev and w.shape == (K, N) and w.is_contiguous()
+                and K % 8 == 0 and N % 8 == 0 and w.data_ptr() % 16 == 0 and _is_target(dev.index or 0)):
+            return None
+        if b is not None and not (b.dtype == torch.float32 and b.device == dev and b.is_contiguous() and b.numel() == N):
+            return None
+        f32 = 1 if x.dtype == torch.float32 else 0
+        if not f32 and dev.index not in _spec_history:
+            return None  # mm_t enables the speculation history first
+        kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, _direct = _gemm_route(_clib.load(), M, N, K, dev)
+        if kind == "packed":
+            return None
+        stream = stream_handle(dev.index or 0)
+        out = torch.empty(*x.shape[:-1], N, device=dev, dtype=x.dtype)
+        scratch = scratch_buffer(dev, stream, scratch_bytes) if scratch_bytes else None
+        bufs = split_buffers(dev, stream, ws_bytes, cnt_bytes) if kind == "splitk" else (None, 0, None, 0)
+        _clib.check(_clib.fast().mm_t_gemm(x.data_ptr(), f32, w.data_ptr(), out.data_ptr(), 1 - f32,
+                                           None if b is None else b.data_ptr(), ROW_SCALE_THRESHOLD, M, N, K,
+                                           _sm_count(dev), None if scratch is None else scratch.data_ptr(),
+                                           scratch_bytes, *bufs, stream), "GEMM")
+        return out
+
     def release_copies(self) -> None:
         """Free the prepacked and decode-layout copies of the weight (rebuilt on demand)."""
         if self._wp is not None or self._wd is not None:
@@ -209,6 +238,10 @@ class FastLinear(nn.Module):
                     else:
                         bufs = split_buffers(dev, stream, *sizes)
                         pl(x.data_ptr(), f32, wptr, out.data_ptr(), 1 - f32, bptr, M, N, K, ksplit, *bufs, stream)
+                    return out
+            elif M > SKINNY_MAX_M:
+                out = self._small_gemm(x, M)
+                if out is not None:
                     return out
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype not in (torch.float16, torch.float32):

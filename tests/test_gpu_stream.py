@@ -129,3 +129,31 @@ def test_stream_replays_in_a_graph(cuda):
         torch.cuda.synchronize()
         for o, e, x, w in zip(outs, eager, xs, ws):
             assert torch.equal(o, e) and torch.equal(g.mm_t(x, w), e)
+
+
+@pytest.mark.parametrize("shape,K,N", [((64,), 1024, 1024), ((3, 37), 1000, 264), ((2, 2, 40), 768, 3072)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("bias", [True, False])
+def test_fast_linear_small_batches_are_mm_t(cuda, shape, K, N, dt, bias):
+    # FastLinear's short path for M > 8 gives mm_t's bits; what it does not take (views, another bias
+    # dtype, a replaced weight) still goes through the general path
+    import torch.nn as nn
+
+    import gtx16_fp16 as g
+
+    torch.manual_seed(0)
+    fl = g.FastLinear.from_linear(nn.Linear(K, N, bias=bias).to(cuda))
+    x = torch.randn(*shape, K, device=cuda).to(dt)
+    want = g.mm_t(x.reshape(-1, K), fl.weight_t, fl.bias, dt).reshape(*shape, N)
+    assert fl._small_gemm(x, x.numel() // K) is not None
+    y = fl(x)
+    assert y.shape == want.shape and y.dtype == dt and torch.equal(y, want)
+    strided = torch.randn(*shape, 2 * K, device=cuda).to(dt)[..., ::2]
+    assert torch.equal(fl(strided), fl(strided.contiguous()))
+    fl.weight_t = (fl.weight_t * 2).contiguous()
+    want = g.mm_t(x.reshape(-1, K), fl.weight_t, fl.bias, dt).reshape(*shape, N)
+    assert torch.equal(fl(x), want)
+    if bias:
+        fl.bias = fl.bias.half()
+        assert fl._small_gemm(x, x.numel() // K) is None
+        assert torch.equal(fl(x), g.mm_t(x.reshape(-1, K), fl.weight_t, fl.bias.float(), dt).reshape(*shape, N))
