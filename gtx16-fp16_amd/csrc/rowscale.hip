@@ -6,8 +6,8 @@
 //
 // Layout: one 64-lane wavefront per row, 4 rows per 256-thread workgroup. Each lane keeps up to
 // CH 16-byte chunks of its row in registers, so the row is read from HBM once: max-reduce across
-// the wavefront (no LDS, no barrier), then scale, convert and store from the registers. Rows longer
-// than 64*CH chunks stream the remainder twice (the second read hits L2).
+// the wavefront (no LDS, no barrier), then scale, convert and store from the registers. Longer rows
+// (K > 4096), and the rows of small batches, get a workgroup each.
 //
 // Output layouts: row-major y[M,K], or the tile-packed layout the 256x256 GEMM streams (see
 // packed_offset in g16_common.hpp): every 256-row x 32-column block of y is one contiguous 16 KB
@@ -19,6 +19,7 @@ namespace g16 {
 namespace {
 
 constexpr int kRowsPerBlock = 4;
+constexpr int kWideMaxM = 512;  // rows up to which every row gets a workgroup (rowscale_launch)
 
 __device__ inline void store_scaled(_Float16* y, u32x4 v, int e, float) {
   *reinterpret_cast<u32x2*>(y) = cast_scaled(v, e, float{});
@@ -75,7 +76,6 @@ __global__ __launch_bounds__(256) void rowscale_kernel(const TX* __restrict__ X,
   }
 #pragma unroll
   for (int c = 0; c < CH; ++c) amax = chunk_absmax(amax, buf[c], TX{});
-  for (int idx = lane + CH * kWave; idx < nch; idx += kWave) amax = chunk_absmax(amax, xr[idx], TX{});
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
 
@@ -88,8 +88,6 @@ __global__ __launch_bounds__(256) void rowscale_kernel(const TX* __restrict__ X,
     const int idx = lane + c * kWave;
     if (idx < nch) store_scaled(out_at<TX, PACK>(Y, row, K, idx, nks), buf[c], e, TX{});
   }
-  for (int idx = lane + CH * kWave; idx < nch; idx += kWave)
-    store_scaled(out_at<TX, PACK>(Y, row, K, idx, nks), xr[idx], e, TX{});
   if (lane == 0) S[row] = sc;
 }
 
@@ -129,6 +127,53 @@ __global__ __launch_bounds__(256) void rowscale_rows2_kernel(const TX* X, _Float
   finish(r0 + half, b);
 }
 
+// One row per workgroup: 4 wavefronts share it, the maxima meet in LDS. Rows up to 4 * 64 * CH chunks
+// (K = 16384 at the launch's CH) are read once, longer ones stream the remainder twice (from L2). Same arithmetic and stores as above, so the same bits.
+template <typename TX, int CH, bool PACK>
+__global__ __launch_bounds__(256) void rowscale_wide_kernel(const TX* __restrict__ X, _Float16* __restrict__ Y,
+                                                            float* __restrict__ S, int M, int K, int texp) {
+  constexpr int EPC = 16 / static_cast<int>(sizeof(TX)), T = 256;
+  __shared__ float s_max[T / kWave];
+  const int row = blockIdx.x, t = threadIdx.x;
+  const int nks = packed_ksteps(K);
+  if constexpr (PACK) {
+    // zeros: a padding row of the last 256-row block, or a real row's columns past K
+    for (int oc = (row >= M ? 0 : K / 8) + t; oc < nks * 4; oc += T)
+      *reinterpret_cast<u32x4*>(reinterpret_cast<unsigned char*>(Y) + packed_offset(row, oc, nks)) =
+          u32x4{0u, 0u, 0u, 0u};
+  }
+  if (row >= M) return;  // the whole workgroup
+  const int nch = K / EPC;
+  const u32x4* xr = reinterpret_cast<const u32x4*>(X + static_cast<size_t>(row) * K);
+  u32x4 buf[CH];
+  float amax = 0.f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int idx = t + c * T;
+    buf[c] = idx < nch ? xr[idx] : u32x4{0u, 0u, 0u, 0u};
+  }
+#pragma unroll
+  for (int c = 0; c < CH; ++c) amax = chunk_absmax(amax, buf[c], TX{});
+  for (int idx = t + CH * T; idx < nch; idx += T) amax = chunk_absmax(amax, xr[idx], TX{});
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+  if ((t & (kWave - 1)) == 0) s_max[t >> 6] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < T / kWave; ++w) amax = fmaxf(amax, s_max[w]);
+  int e;
+  float sc;
+  row_exponent(amax, texp, e, sc);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int idx = t + c * T;
+    if (idx < nch) store_scaled(out_at<TX, PACK>(Y, row, K, idx, nks), buf[c], e, TX{});
+  }
+  for (int idx = t + CH * T; idx < nch; idx += T)
+    store_scaled(out_at<TX, PACK>(Y, row, K, idx, nks), xr[idx], e, TX{});
+  if (t == 0) S[row] = sc;
+}
+
 template <typename TX, int CH, bool PACK>
 int rowscale_launch(const void* X, void* Y, float* S, int M, int K, float thresh, void* stream) {
   if (M < 0 || K < 0 || K % 8 != 0) return G16_E_SHAPE;
@@ -138,13 +183,23 @@ int rowscale_launch(const void* X, void* Y, float* S, int M, int K, float thresh
   const int texp = thresh_exponent(thresh);
   if (texp == -1000) return G16_E_SHAPE;
   constexpr int EPC = 16 / static_cast<int>(sizeof(TX));
+  const int rows = PACK ? ceil_div(M, kPackRows) * kPackRows : M;
+  // A workgroup per row: past K = 4096, where a wavefront would read its row twice, and for so few
+  // rows that a wavefront each leaves CUs idle. Graph-timed, wavefront -> workgroup per row (us, M x K,
+  // fp32): 80 x 2048 3.06 -> 2.58, 333 x 4096 4.39 -> 3.86, 80 x 11008 16.9 -> 3.6, 777 x 8192 14.8 -> 8.3,
+  // 8192 x 8192 99 -> 74 (fp16 62 -> 42; packed 103 -> 89 and 71 -> 52); with more short rows the
+  // wavefronts are the faster ones (2048 x 256 3.0 vs 3.3, 8192 x 1024 10.6 vs 11.5).
+  if (K > kWave * CH * EPC || M <= kWideMaxM) {
+    auto fn = K > kWave * CH * EPC ? rowscale_wide_kernel<TX, CH, PACK> : rowscale_wide_kernel<TX, CH / 4, PACK>;
+    return launch(fn, dim3(rows), dim3(256), static_cast<hipStream_t>(stream), static_cast<const TX*>(X),
+                  static_cast<_Float16*>(Y), S, M, K, texp);
+  }
   if (K == kWave * CH * EPC && M % (2 * kRowsPerBlock) == 0 && (!PACK || M % kPackRows == 0)) {
     // whole rows, an even number of workgroup row sets, no padding rows: the two-row form
     return launch(rowscale_rows2_kernel<TX, CH, PACK>, dim3(M / (2 * kRowsPerBlock)), dim3(256),
                   static_cast<hipStream_t>(stream), static_cast<const TX*>(X), static_cast<_Float16*>(Y), S, M, K,
                   texp);
   }
-  const int rows = PACK ? ceil_div(M, kPackRows) * kPackRows : M;
   const dim3 grid(ceil_div(rows, kRowsPerBlock)), block(256);
   return launch(rowscale_kernel<TX, CH, PACK>, grid, block, static_cast<hipStream_t>(stream),
                 static_cast<const TX*>(X), static_cast<_Float16*>(Y), S, M, K, texp);
