@@ -10,9 +10,11 @@ import torch.nn.functional as F
 
 from . import _clib
 from .kernels import SKINNY_MAX_M, PreparedCall, scratch_buffer, split_buffers, stream_handle
-from .ops import (ROW_SCALE_THRESHOLD, STRIPS_MAX_M, _gemm_route, _is_target, _sm_count, _spec_history, is_affected, mm_t,
+from .ops import (ROW_SCALE_THRESHOLD, STRIPS_MAX_M, _gemm_route, _is_target, _sm_count, is_affected, mm_t,
                   mm_t_prepacked, pack_decode_weight, pack_weight, prepacked_route, skinny_strips, supported,
                   tensor_version)
+
+_F32, _F16 = torch.float32, torch.float16  # forward's type checks cost more with the attribute lookups
 
 
 class FastLinear(nn.Module):
@@ -108,7 +110,7 @@ class FastLinear(nn.Module):
         layer's ``.weight`` (its shape, device or dtype) as they would on nn.Linear."""
         return self.weight_t.t()
 
-    def _decode_entry(self, M: int, dev: torch.device, f32: int = 1):
+    def _decode_entry(self, M: int, dev: torch.device, f32: bool = True):
         key = (M, dev.index, self.prepack_decode, f32)
         w, b = self.weight_t, self.bias
         bptr = None if b is None else b.data_ptr()
@@ -130,7 +132,7 @@ class FastLinear(nn.Module):
                 pl = PreparedCall(_clib.fast().skinny, "skinny GEMM")
                 sizes = (lib.g16_skinny_workspace_bytes(M, N, K, ksplit),
                          lib.g16_skinny_counter_bytes(M, N, K, ksplit))
-                if self.prepack_decode and lib.g16_skinny_strips_route(M, N, K, f32):
+                if self.prepack_decode and lib.g16_skinny_strips_route(M, N, K, int(f32)):
                     pls = PreparedCall(_clib.fast().skinny_strips, "skinny GEMM (decode layout)")
             entry = (pl, ksplit, sizes, w.data_ptr(), bptr, pls)
             self._skinny[key] = entry
@@ -176,9 +178,12 @@ class FastLinear(nn.Module):
         return self._wd_ptr
 
     def _small_gemm(self, x: torch.Tensor, M: int) -> torch.Tensor | None:
-        # mm_t's GEMM call for a contiguous, aligned fp32 or fp16 x of M > 8 rows where the plan is one
-        # of the smaller tiles, whose calls are bound by host time: the same checks as supported() and
-        # mm_t, once, and no reshapes (64 x 4096 x 1024: 15.7 us per call through the general path).
+        # mm_t's GEMM call for a contiguous, aligned fp32 x of M > 8 rows where the plan is one of the
+        # smaller tiles, whose calls are bound by host time: the same checks as supported() and mm_t,
+        # once, and no reshapes (64 x 4096 x 1024: 15.7 us per call through the general path, 11.1
+        # here). fp16 x keeps the general path: with outlier rows its speculative launches compute
+        # tiles again until the host sees the miss, and a host further ahead of the device enqueues
+        # more of them (53 x 4608 x 2176: 18.1 us per call by the general path, 24.8 by this one).
         # None: not that case (the general path then decides).
         w, b, dev = self.weight_t, self.bias, x.device
         K, N = self.in_features, self.out_features
@@ -187,9 +192,6 @@ class FastLinear(nn.Module):
             return None
         if b is not None and not (b.dtype == torch.float32 and b.device == dev and b.is_contiguous() and b.numel() == N):
             return None
-        f32 = 1 if x.dtype == torch.float32 else 0
-        if not f32 and dev.index not in _spec_history:
-            return None  # mm_t enables the speculation history first
         kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, _direct = _gemm_route(_clib.load(), M, N, K, dev)
         if kind == "packed":
             return None
@@ -197,7 +199,7 @@ class FastLinear(nn.Module):
         out = torch.empty(*x.shape[:-1], N, device=dev, dtype=x.dtype)
         scratch = scratch_buffer(dev, stream, scratch_bytes) if scratch_bytes else None
         bufs = split_buffers(dev, stream, ws_bytes, cnt_bytes) if kind == "splitk" else (None, 0, None, 0)
-        _clib.check(_clib.fast().mm_t_gemm(x.data_ptr(), f32, w.data_ptr(), out.data_ptr(), 1 - f32,
+        _clib.check(_clib.fast().mm_t_gemm(x.data_ptr(), True, w.data_ptr(), out.data_ptr(), False,
                                            None if b is None else b.data_ptr(), ROW_SCALE_THRESHOLD, M, N, K,
                                            _sm_count(dev), None if scratch is None else scratch.data_ptr(),
                                            scratch_bytes, *bufs, stream), "GEMM")
@@ -212,37 +214,38 @@ class FastLinear(nn.Module):
         self._wd_ptr = 0
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        out_dtype = x.dtype if x.dtype in (torch.float32, torch.float16) else torch.float32
+        dt = x.dtype
+        f32 = dt == _F32
         if torch.is_grad_enabled() and x.requires_grad:
             return F.linear(x, self.weight_t.t().to(x.dtype), None if self.bias is None else self.bias.to(x.dtype))
         shape = x.shape
         # Fast path for small batches (generation): minimal Python per call (linear.py:49-64).
         # Unlike the reference, the weight's support is checked (once per layer and M), so a
         # FastLinear built directly with K or N not a multiple of 8 still takes the fallback.
-        if x.is_cuda and x.dtype in (torch.float32, torch.float16) and x.is_contiguous() and x.data_ptr() % 16 == 0:
+        if (f32 or dt == _F16) and x.is_cuda and x.is_contiguous() and x.data_ptr() % 16 == 0:
             K, N = self.in_features, self.out_features
             M = x.numel() // K if shape[-1] == K else -1
             if 0 < M <= SKINNY_MAX_M:
                 dev = x.device
-                f32 = 1 if x.dtype == torch.float32 else 0
                 pl, ksplit, sizes, wptr, bptr, pls = self._decode_entry(M, dev, f32)
                 if pl is not None:
                     stream = stream_handle(dev.index or 0)
-                    out = torch.empty(*shape[:-1], N, device=dev, dtype=x.dtype)
+                    out = torch.empty(*shape[:-1], N, device=dev, dtype=dt)
                     wd = 0
                     if pls is not None:
                         w = self.weight_t
                         wd = self._wd_ptr if self._wd_key == (wptr, tensor_version(w), w.device) else self._decode_weight()
                     if wd:
-                        pls(x.data_ptr(), f32, wd, out.data_ptr(), 1 - f32, bptr, M, N, K, stream)
+                        pls(x.data_ptr(), f32, wd, out.data_ptr(), not f32, bptr, M, N, K, stream)
                     else:
                         bufs = split_buffers(dev, stream, *sizes)
-                        pl(x.data_ptr(), f32, wptr, out.data_ptr(), 1 - f32, bptr, M, N, K, ksplit, *bufs, stream)
+                        pl(x.data_ptr(), f32, wptr, out.data_ptr(), not f32, bptr, M, N, K, ksplit, *bufs, stream)
                     return out
-            elif M > SKINNY_MAX_M:
+            elif f32 and M > SKINNY_MAX_M:
                 out = self._small_gemm(x, M)
                 if out is not None:
                     return out
+        out_dtype = dt if f32 or dt == _F16 else _F32
         x2 = x.reshape(-1, self.in_features)
         if x2.dtype not in (torch.float16, torch.float32):
             x2 = x2.float()

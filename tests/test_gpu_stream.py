@@ -145,7 +145,8 @@ def test_fast_linear_small_batches_are_mm_t(cuda, shape, K, N, dt, bias):
     fl = g.FastLinear.from_linear(nn.Linear(K, N, bias=bias).to(cuda))
     x = torch.randn(*shape, K, device=cuda).to(dt)
     want = g.mm_t(x.reshape(-1, K), fl.weight_t, fl.bias, dt).reshape(*shape, N)
-    assert fl._small_gemm(x, x.numel() // K) is not None
+    if dt == torch.float32:
+        assert fl._small_gemm(x, x.numel() // K) is not None
     y = fl(x)
     assert y.shape == want.shape and y.dtype == dt and torch.equal(y, want)
     strided = torch.randn(*shape, 2 * K, device=cuda).to(dt)[..., ::2]
@@ -155,5 +156,6 @@ def test_fast_linear_small_batches_are_mm_t(cuda, shape, K, N, dt, bias):
     assert torch.equal(fl(x), want)
     if bias:
         fl.bias = fl.bias.half()
-        assert fl._small_gemm(x, x.numel() // K) is None
+        if dt == torch.float32:
+            assert fl._small_gemm(x, x.numel() // K) is None
         assert torch.equal(fl(x), g.mm_t(x.reshape(-1, K), fl.weight_t, fl.bias.float(), dt).reshape(*shape, N))
