@@ -895,15 +895,16 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
         // applies before its MFMAs of that step. Later steps of the row are scaled as they are cast.
         //   M_j has little room: with ~100 instructions (address arithmetic mostly) it set the pace, 1570
         // shader cycles per step at 4096^3 against 1054 with packed A. So the loop is unrolled over the
-        // ring (every LDS address is an immediate) and the descriptors' ranges and the scalar offset,
-        // which the range check includes, replace per-step masks and pointers.
+        // ring (every LDS address is an immediate) and the descriptors' ranges and the scalar offset
+        // replace per-step masks and pointers.
         constexpr int NL = BM * BK * 4 / 16 / Cfg::THREADS;
         static_assert(NL == 4 && BM / Cfg::WAVES == 32 && Cfg::B_INSTR == 2 && NSTAGE == 4,
                       "4 loads of 8 rows and two DMA instructions per wavefront and step");
         const int dr0 = wave * 32 + (lane >> 3), dc = lane & 7;  // this lane's first row, its 4-value chunk
-        // X from this tile's first row on; loads past its last row give 0. A step past K reads what
-        // follows (the next row): its stage is never multiplied. Columns past K in the last step of a
-        // K that is no multiple of BK are masked by the lane's offset.
+        // X from this tile's first row on; loads past its last row give 0. Steps past K load the last
+        // step again (their stages are never multiplied), so that no scalar offset passes a one-row
+        // tile's range. Columns past K in the last step of a K that is no multiple of BK are masked by
+        // the lane's offset.
         const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<float*>(static_cast<const float*>(X) + static_cast<size_t>(m0) * K), 0,
             static_cast<int>(min(static_cast<long>(M - m0), static_cast<long>(BM)) * K * 4), kRawBufferDword3);
@@ -916,10 +917,11 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
         float4v xs[2][NL];
         int scaled = 0;  // 1: some row this wavefront stages has a factor < 1
         auto load_op = [&](int s, int l) __attribute__((always_inline)) {
-          const uint32_t last = s == nk - 1 ? 0xffffffffu : 0u;
+          const int sc = min(s, nk - 1);
+          const uint32_t last = sc == nk - 1 ? 0xffffffffu : 0u;
           return __builtin_bit_cast(
               float4v, __builtin_amdgcn_raw_buffer_load_b128(
-                           rx, static_cast<int>(((tail & last) | voff) + static_cast<uint32_t>(l * 32 * K)), s * (BK * 4), 0));
+                           rx, static_cast<int>(((tail & last) | voff) + static_cast<uint32_t>(l * 32 * K)), sc * (BK * 4), 0));
         };
         auto load_x = [&](auto hc, int s) __attribute__((always_inline)) {
 #pragma unroll
@@ -963,7 +965,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
             float4v v = __builtin_bit_cast(
                 float4v, __builtin_amdgcn_raw_buffer_load_b128(
                              rx, s * BK + c * 4 < K ? static_cast<int>((r * K + c * 4) * 4) : static_cast<int>(kOob),
-                             s * (BK * 4), 0));
+                             min(s, nk - 1) * (BK * 4), 0));
             float f = s_fac[r];
             v *= f;
             float rm = absmax4(0.f, v);
@@ -1001,8 +1003,8 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
           }
           if (__any(m > kHalfMax)) raise(s);
         };
-        // B's DMA, in step order. Packed: the step's 16 KB block is a scalar offset, the range ends with
-        // the last block, and the two instructions differ by 1 KB in memory as in LDS, which the
+        // B's DMA, in step order. Packed: the step's 16 KB block is a scalar offset (steps past K fetch the
+        // last block again), the range ends with the last block, and the two instructions differ by 1 KB in memory as in LDS, which the
         // instruction's offset adds to both. Row-major: a running pointer, the range ends with the
         // matrix (rows past K), and lanes past N are masked.
         const uint32_t bst = sB_lds + wave * Cfg::B_INSTR * 1024;
@@ -1027,7 +1029,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
                 "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
                 "buffer_load_dwordx4 %1, %2, %3 offen offset:1024 lds"
                 :
-                : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(bvo[0]), "s"(rbp), "s"(s * 16384)
+                : "s"(__builtin_amdgcn_readfirstlane(at)), "v"(bvo[0]), "s"(rbp), "s"(min(s, nk - 1) * 16384)
                 : "memory", "m0");
           } else {
             const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
@@ -1796,9 +1798,11 @@ bool direct_route(const Plan& p, int N, int K, int ksplit, int num_cus) {
   return p.tile == Tile::T256 && ksplit == 1 && K > 0 && K <= kDirectMaxK && N <= kDirectMaxN &&
          4L * p.ntm * p.ntn >= 3L * num_cus;
 }
-// Thresholds the direct launch takes: up to 2^15, so that every value of a row within the threshold
-// has a finite cast (it rescales only rows that leave fp16's range).
-constexpr int kDirectMaxTexp = 15;
+// Thresholds the direct launches take: up to 2^15, so that every value of a row within the threshold
+// has a finite cast (they rescale only rows that leave fp16's range), and from 2^2, so that a row's
+// factor 2^-e, e <= 128 - texp, and its inverse are normal numbers.
+constexpr int kDirectMinTexp = 2, kDirectMaxTexp = 15;
+bool direct_thresh(int texp) { return texp >= kDirectMinTexp && texp <= kDirectMaxTexp; }
 
 // fp32 activations also run as one direct launch on the 4-wavefront tiles with 64-deep K steps, where
 // the cast's launch costs more than streaming A at 4 bytes instead of 2: for up to 64 rows always; above,
@@ -2128,9 +2132,9 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   if (scratch == nullptr) return G16_E_NULL;
   if (!g16::aligned16(scratch)) return G16_E_ALIGN;
   if (scratch_bytes < g16_mm_t_scratch_bytes(M, N, K, num_cus)) return G16_E_WORKSPACE;
-  if (x_is_f32 && texp <= g16::kDirectMaxTexp && g16_mm_t_direct_route(M, N, K, num_cus) == 1)
+  if (x_is_f32 && g16::direct_thresh(texp) && g16_mm_t_direct_route(M, N, K, num_cus) == 1)
     return g16_mm_t_direct(static_cast<const float*>(x), w_t, 0, out, out_is_f16, bias, thresh, M, N, K, num_cus, stream);
-  if (x_is_f32 && texp <= g16::kDirectMaxTexp) {
+  if (x_is_f32 && g16::direct_thresh(texp)) {
     // one launch: the tiles stream x and cast it themselves (the scratch stays unused)
     const int ks = g16_hgemm_plan(M, N, K, num_cus);
     if (g16::stream_route(g16::choose_tile(M, N, K, num_cus), M, K, g16::ksplit_for(K, ks))) {
@@ -2170,7 +2174,7 @@ extern "C" int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, 
   if (M == 0 || N == 0) return G16_OK;
   if (out == nullptr || x == nullptr || w == nullptr) return G16_E_NULL;
   const int texp = g16::thresh_exponent(thresh);
-  if (texp == -1000 || texp > g16::kDirectMaxTexp || g16_mm_t_direct_route(M, N, K, num_cus) == 0) return G16_E_SHAPE;
+  if (!g16::direct_thresh(texp) || g16_mm_t_direct_route(M, N, K, num_cus) == 0) return G16_E_SHAPE;
   if (!g16::aligned16(x)) return G16_E_ALIGN;
   const g16::ResidentCast rc{x, 1, texp};
   return g16::gemm_launch(nullptr, w, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus, nullptr, 0, nullptr, 0,

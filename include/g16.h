@@ -167,8 +167,8 @@ int g16_mm_t_spec_paused(const uint16_t* w_t, void* stream);
  * x itself and casts it in registers on the way into LDS. `w` is w_t [K,N], or, with w_packed != 0,
  * its packed form (g16_pack_weight). A row whose values all fit fp16 is cast as it is; a row with a
  * larger value is scaled by a power of two from that value on (its sums so far are scaled with it),
- * by the rule of g16_rowscale_f32 for a threshold of at most 2^15 applied to the part of the row
- * read so far. Each value is so rounded to fp16 at least as finely as g16_rowscale_f32 rounds it; the
+ * by the rule of g16_rowscale_f32 for a threshold of 4 to 2^15 (others: G16_E_SHAPE) applied to the
+ * part of the row read so far. Each value is so rounded to fp16 at least as finely as g16_rowscale_f32 rounds it; the
  * results are the same bits unless a scaled value falls below fp16's normal range. */
 int g16_mm_t_direct_route(int M, int N, int K, int num_cus);
 int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,

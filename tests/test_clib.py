@@ -243,6 +243,7 @@ def test_direct_route_rule_and_refusals(lib):
     d = lib.g16_mm_t_direct
     assert d(A, A, 0, A, 0, None, 1024.0, 4096, 4096, 4096, 256, None) == -1
     assert d(A, A, 0, A, 0, None, 65536.0, 65536, 768, 768, 256, None) == -1    # threshold past 2^15
+    assert d(A, A, 0, A, 0, None, 2.0, 65536, 768, 768, 256, None) == -1        # threshold below 4
     assert d(A, A, 0, A, 0, None, 1000.0, 65536, 768, 768, 256, None) == -1     # not a power of two
     assert d(A + 4, A, 0, A, 0, None, 1024.0, 65536, 768, 768, 256, None) == -2
     assert d(A, A + 8, 1, A, 0, None, 1024.0, 65536, 768, 768, 256, None) == -2

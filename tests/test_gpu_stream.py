@@ -159,3 +159,29 @@ def test_fast_linear_small_batches_are_mm_t(cuda, shape, K, N, dt, bias):
         if dt == torch.float32:
             assert fl._small_gemm(x, x.numel() // K) is None
         assert torch.equal(fl(x), g.mm_t(x.reshape(-1, K), fl.weight_t, fl.bias.float(), dt).reshape(*shape, N))
+
+
+@pytest.mark.parametrize("thresh", [1.0, 2.0, 4.0, 1024.0, 2.0 ** 15])
+def test_gemm_call_takes_any_threshold(cuda, thresh):
+    # a row of 2^127 has the largest exponents: for thresholds below 4 a direct launch's factor would
+    # not be a normal number (two launches there); past 2^15 the scaled value itself is no fp16 number
+    from gtx16_fp16 import _clib
+
+    lib = _clib.load()
+    M, K, N = 64, 1024, 1024
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    x = randn((M, K), seed=11)
+    x[5, 100] = 2.0 ** 127
+    w = randn((K, N), seed=12, scale=0.02, dtype=torch.float16)
+    xd, wd = x.to(cuda), w.to(cuda)
+    out = torch.empty(M, N, device=cuda)
+    ks = lib.g16_hgemm_plan(M, N, K, cus)
+    bufs = [torch.zeros(max(16, n), dtype=torch.uint8, device=cuda)
+            for n in (lib.g16_mm_t_scratch_bytes(M, N, K, cus), lib.g16_hgemm_splitk_workspace_bytes(M, N, K, ks, cus),
+                      lib.g16_hgemm_splitk_counter_bytes(M, N, K, ks, cus))]
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    assert lib.g16_mm_t_gemm(xd.data_ptr(), 1, wd.data_ptr(), out.data_ptr(), 0, None, thresh, M, N, K, cus,
+                             *(v for b in bufs for v in (b.data_ptr(), b.numel())), st) == 0
+    ref = x.double() @ w.double()
+    err = (out.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert (err <= 2.0 ** -10).all(), err.max()  # fp16 rounding of the activations: 2^-11 per value
