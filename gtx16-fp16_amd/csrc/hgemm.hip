@@ -49,6 +49,10 @@
 //     tile with few columns (direct_route), through a ring of fp32 LDS stages on the 4-wavefront tiles
 //     (stream_route). A row is rescaled as soon as a value of it leaves fp16's range, its sums so far
 //     with it (exact), so no pass over the row has to come first and no slice waits for another.
+//   * Raw fp16 A (mm_t's GEMM path in one launch for fp16 activations on the unsplit 256x256 tile): an
+//     fp16 activation is its own cast, and its products' sums stay far inside fp32, so x is A as it
+//     is. Only an infinite value needs more: the rowscale cast turns its whole row into NaN, and so
+//     does the epilogue, which reads the rows of x again where a sum is infinite.
 //   * Speculative fp16 A (the 4-wavefront tiles with fp16 activations, mm_t's GEMM path in one
 //     launch): a row whose |max| does not exceed the threshold has scale 1, and its rowscale cast is
 //     the activation itself. So the GEMM streams x as A and tracks the largest |x| it multiplies
@@ -257,8 +261,9 @@ __device__ inline void phase_barrier() { asm volatile("s_barrier" ::: "memory");
 // A stages and rescales a row as soon as a value of it leaves fp16's range: the unsplit 256x256 tile
 // (through registers), and the 4-wavefront tiles with 64-deep K steps, split or not (through a ring of
 // fp32 stages in LDS; a slice rescales by what it has seen, and publishes its sums in units of 1).
+// RAW: A is the fp16 activations, row-major; rows that hold an infinity give NaN.
 template <class Cfg, bool OUT_F16, bool SPLITK, bool PACKED_A = false, bool PACKED_B = false, bool RESIDENT = false,
-          bool SPEC = false, bool DIRECT = false>
+          bool SPEC = false, bool DIRECT = false, bool RAW = false>
 __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
                                                          void* __restrict__ Cv, const float* __restrict__ bias,
                                                          const float* __restrict__ rscale, float* __restrict__ part,
@@ -276,6 +281,8 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
   static_assert(!DIRECT || (Cfg::WAVES == 8 && Cfg::BK == 32 && Cfg::MF16 && !SPLITK && !PACKED_A && !RESIDENT && !SPEC) ||
                     (STREAM && Cfg::BK == 64 && !Cfg::MF16 && NSTAGE == 4 && !PACKED_A && !PACKED_B && !RESIDENT && !SPEC),
                 "direct A: the unsplit 256x256 tile, the 4-wavefront tiles with 64-deep K steps");
+  static_assert(!RAW || (Cfg::WAVES == 8 && !SPLITK && !PACKED_A && !RESIDENT && !SPEC && !DIRECT),
+                "raw A: the unsplit 256-row tiles");
   constexpr int A_STAGES = RESIDENT ? kResidentSteps : (STREAM ? 2 : NSTAGE);
   __shared__ __attribute__((aligned(1024))) unsigned char sA[A_STAGES][Cfg::A_BYTES];
   __shared__ __attribute__((aligned(1024))) unsigned char sB[NSTAGE][Cfg::B_BYTES];
@@ -362,7 +369,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
         // whole 16 KB blocks; a 128-column tile streams one half of each: rows 0-127 of a block are
         // its first 8 KB (chunks q < 8), rows 128-255 the second, each already the 128-row stage
         // image (the row swizzle repeats every 8 rows). Step k0 adds k0/BK blocks (16 KB) either way.
-        static_assert((PACKED_A || DIRECT) && (Cfg::BN == 256 || Cfg::BN == 128), "packed weight: the 256-row tiles");
+        static_assert((PACKED_A || DIRECT || RAW) && (Cfg::BN == 256 || Cfg::BN == 128), "packed weight: the 256-row tiles");
         constexpr int kHalves = 256 / Cfg::BN;
         return __builtin_amdgcn_make_buffer_rsrc(
             const_cast<_Float16*>(B) + static_cast<size_t>(tn / kHalves) * ceil_div(K, BK) * 8192 + (tn % kHalves) * 4096, 0,
@@ -1422,6 +1429,33 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
     // well) for the store before it: 32 memory round trips in a row per wavefront, ~5.5 us of each
     // 256x256 tile's epilogue even with the stores taken out.
     constexpr int ERI = Cfg::WTM / 32, ERJ = Cfg::WTN / 32;
+    // raw A: bit b set where row lane / 8 + 8 b of this wavefront's rows holds an infinity. Finite fp16
+    // values cannot make an infinite sum (an infinite weight can), so x is looked at only where a sum is.
+    uint32_t inf_rows = 0;
+    if constexpr (RAW) {
+      static_assert(!RAW || ERI * 4 <= 32, "a bit per row and lane");
+      float am = 0.f;  // fmaxf drops the NaNs
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) am = fmaxf(am, fabsf(acc[i][j][r]));
+      if (__builtin_expect(__any(am == __uint_as_float(0x7f800000u)), 0)) {
+#pragma unroll 1
+        for (int r = 0; r < Cfg::WTM && m0 + wm0 + r < M; ++r) {
+          const u32x4* xr = reinterpret_cast<const u32x4*>(A + static_cast<size_t>(m0 + wm0 + r) * K);
+          bool inf = false;
+          for (int c = lane; c < K / 8; c += kWave) {
+            const u32x4 v = xr[c];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              inf = inf || (v[q] & 0x7fffu) == 0x7c00u || (v[q] & 0x7fff0000u) == 0x7c000000u;
+          }
+          if (__any(inf) && (lane >> 3) == (r & 7)) inf_rows |= 1u << (r >> 3);
+        }
+      }
+    }
     float erow[ERI][4];
     float4v ecol[ERJ];
 #pragma unroll
@@ -1439,6 +1473,8 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
           } else {
             erow[ri][q] = inv_factor(s_fac[grow - m0]);
           }
+        } else if constexpr (RAW) {
+          erow[ri][q] = (inf_rows >> (4 * ri + q)) & 1u ? __uint_as_float(0x7fc00000u) : 1.f;
         } else {
           erow[ri][q] = (RESIDENT || respec) ? s_scale[grow - m0]
                                              : (SPEC ? 1.f : (rscale != nullptr && grow < M ? rscale[grow] : 1.f));
@@ -1701,7 +1737,10 @@ using GemmFn = void (*)(const _Float16*, const _Float16*, void*, const float*, c
 
 template <bool OUT_F16>
 GemmFn<OUT_F16> gemm_fn(Tile t, bool splitk, bool packed, bool packed_b, bool resident = false, bool spec = false,
-                        bool direct = false) {
+                        bool direct = false, bool raw = false) {
+  if (raw)
+    return packed_b ? hgemm_kernel<Cfg256, OUT_F16, false, false, true, false, false, false, true>
+                    : hgemm_kernel<Cfg256, OUT_F16, false, false, false, false, false, false, true>;
   if (direct) {
     switch (t) {
       case Tile::T32: return splitk ? hgemm_kernel<Cfg32, OUT_F16, true, false, false, false, false, true> : hgemm_kernel<Cfg32, OUT_F16, false, false, false, false, false, true>;
@@ -1804,6 +1843,14 @@ bool direct_route(const Plan& p, int N, int K, int ksplit, int num_cus) {
 constexpr int kDirectMinTexp = 2, kDirectMaxTexp = 15;
 bool direct_thresh(int texp) { return texp >= kDirectMinTexp && texp <= kDirectMaxTexp; }
 
+// fp16 activations run as one raw launch (x is the GEMM's A as it is, no cast) where the plan is the
+// unsplit 256x256 tile: the cast it saves costs more than A's row-major DMA (64-byte pieces of 16 rows
+// instead of 1 KB runs) adds to the GEMM. Graph-timed, cast + packed GEMM -> raw (us, M x K x N, fp16
+// out): 8192 x 2048^2 72 -> 63 (61 prepacked), 16384 x 1024^2 48.9 -> 35.7, 65536 x 768 x 768 124 -> 90,
+// 65536 x 768 x 2048 257 -> 223, 4000 x 1000 x 5000 81 -> 75, 4096^3 118 -> 110. On 256x128 tiles, whose A stream weighs twice as much per
+// product, it does not: 2048 x 4096^2 cast + packed GEMM 79.6 us, raw 84.5; 1500 x 4096^2 75.1, 77.8.
+bool raw_route(const Plan& p, int K, int ksplit) { return p.tile == Tile::T256 && ksplit == 1 && K > 0; }
+
 // fp32 activations also run as one direct launch on the 4-wavefront tiles with 64-deep K steps, where
 // the cast's launch costs more than streaming A at 4 bytes instead of 2: for up to 64 rows always; above,
 // past K = 4096 (the cast reads such rows twice), and on short slices of split grids or of many rows.
@@ -1843,7 +1890,7 @@ int fp16_bits_at_most(int texp) {
 int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, const float* bias, const float* rscale,
                 int M, int N, int K, int ksplit, int num_cus, void* ws, size_t ws_bytes, uint32_t* counters_in,
                 size_t counter_bytes_in, void* stream, bool packed = false, bool packed_b = false,
-                const ResidentCast* rc = nullptr, const SpecA* sp = nullptr, bool direct = false) {
+                const ResidentCast* rc = nullptr, const SpecA* sp = nullptr, bool direct = false, bool raw = false) {
   if (M < 0 || N < 0 || K < 0 || K % 8 != 0 || N % 8 != 0 || K > kMaxK || N > kMaxN) return G16_E_SHAPE;
   if (M == 0 || N == 0) return G16_OK;
   if (ksplit < 1 || ksplit > 256) return G16_E_SPLIT;
@@ -1853,6 +1900,7 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   if (num_cus <= 0) num_cus = stream_cus(static_cast<hipStream_t>(stream));
   Plan p = choose_tile(M, N, K, num_cus);
   if (direct ? !direct_route(p, N, K, ks.ksplit, num_cus) && !stream_route(p, M, K, ks) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
+  if (raw && !raw_route(p, K, ks.ksplit)) return G16_E_SHAPE;
   const bool spec = sp != nullptr;
   if (spec && (!four_wave(p.tile) || packed ||
                ks.ksplit > kSpecMaxSplit || sp->texp < kSpecMinTexp))
@@ -1889,9 +1937,9 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   const int tbits = spec ? sp->tbits : 0;
   uint32_t* miss = spec ? sp->miss : nullptr;
   if (out_f16)
-    return launch(gemm_fn<true>(p.tile, sk, packed, packed_b, res, spec, direct), grid, block, s, a, b, C, bias, rscale, part,
+    return launch(gemm_fn<true>(p.tile, sk, packed, packed_b, res, spec, direct, raw), grid, block, s, a, b, C, bias, rscale, part,
                   counters, M, N, K, ks.kchunk, ks.ksplit, p.ntm, p.ntn, x, x_f32, texp, tbits, miss);
-  return launch(gemm_fn<false>(p.tile, sk, packed, packed_b, res, spec, direct), grid, block, s, a, b, C, bias, rscale, part,
+  return launch(gemm_fn<false>(p.tile, sk, packed, packed_b, res, spec, direct, raw), grid, block, s, a, b, C, bias, rscale, part,
                 counters, M, N, K, ks.kchunk, ks.ksplit, p.ntm, p.ntn, x, x_f32, texp, tbits, miss);
 }
 
@@ -2132,6 +2180,8 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   if (scratch == nullptr) return G16_E_NULL;
   if (!g16::aligned16(scratch)) return G16_E_ALIGN;
   if (scratch_bytes < g16_mm_t_scratch_bytes(M, N, K, num_cus)) return G16_E_WORKSPACE;
+  if (!x_is_f32 && g16_mm_t_raw_route(M, N, K, num_cus) == 1)
+    return g16_mm_t_raw(static_cast<const uint16_t*>(x), w_t, 0, out, out_is_f16, bias, M, N, K, num_cus, stream);
   if (x_is_f32 && g16::direct_thresh(texp) && g16_mm_t_direct_route(M, N, K, num_cus) == 1)
     return g16_mm_t_direct(static_cast<const float*>(x), w_t, 0, out, out_is_f16, bias, thresh, M, N, K, num_cus, stream);
   if (x_is_f32 && g16::direct_thresh(texp)) {
@@ -2161,6 +2211,21 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   const int ks = g16_hgemm_plan(M, N, K, num_cus);
   return g16::gemm_launch(y, w_t, out, out_is_f16 != 0, bias, s, M, N, K, ks, num_cus, workspace, workspace_bytes,
                           counters, counter_bytes, stream);
+}
+
+extern "C" int g16_mm_t_raw_route(int M, int N, int K, int num_cus) {
+  if (M <= 0 || N <= 0 || K <= 0 || num_cus <= 0) return 0;
+  return g16::raw_route(g16::choose_tile(M, N, K, num_cus), K, g16_hgemm_plan(M, N, K, num_cus)) ? 1 : 0;
+}
+
+extern "C" int g16_mm_t_raw(const uint16_t* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,
+                            const float* bias, int M, int N, int K, int num_cus, void* stream) {
+  if (M < 0 || N < 0 || K < 0 || K % 8 != 0 || N % 8 != 0 || num_cus <= 0) return G16_E_SHAPE;
+  if (M == 0 || N == 0) return G16_OK;
+  if (out == nullptr || x == nullptr || w == nullptr) return G16_E_NULL;
+  if (g16_mm_t_raw_route(M, N, K, num_cus) == 0) return G16_E_SHAPE;
+  return g16::gemm_launch(x, w, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus, nullptr, 0, nullptr, 0, stream,
+                          false, w_packed != 0, nullptr, nullptr, false, true);
 }
 
 extern "C" int g16_mm_t_direct_route(int M, int N, int K, int num_cus) {

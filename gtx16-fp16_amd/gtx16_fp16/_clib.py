@@ -42,6 +42,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "g16_mm_t_gemm": (_I, [_P, _I, _P, _P, _I, _P, _F, _I, _I, _I, _I, _P, _SZ, _P, _SZ, _P, _SZ, _P]),
     "g16_mm_t_spec_history": (_I, [_P]),
     "g16_mm_t_spec_paused": (_I, [_P, _P]),
+    "g16_mm_t_raw_route": (_I, [_I, _I, _I, _I]),
+    "g16_mm_t_raw": (_I, [_P, _P, _I, _P, _I, _P, _I, _I, _I, _I, _P]),
     "g16_mm_t_direct_route": (_I, [_I, _I, _I, _I]),
     "g16_mm_t_direct": (_I, [_P, _P, _I, _P, _I, _P, _F, _I, _I, _I, _I, _P]),
     "g16_packed_b_bytes": (_SZ, [_I, _I]),

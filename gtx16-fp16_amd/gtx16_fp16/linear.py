@@ -192,7 +192,7 @@ class FastLinear(nn.Module):
             return None
         if b is not None and not (b.dtype == torch.float32 and b.device == dev and b.is_contiguous() and b.numel() == N):
             return None
-        kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, _direct = _gemm_route(_clib.load(), M, N, K, dev)
+        kind, scratch_bytes, _ks, ws_bytes, cnt_bytes = _gemm_route(_clib.load(), M, N, K, dev)[:5]
         if kind == "packed":
             return None
         stream = stream_handle(dev.index or 0)

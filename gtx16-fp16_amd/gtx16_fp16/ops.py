@@ -94,23 +94,25 @@ _routes: dict[tuple[int, int, int, int], tuple] = {}
 
 
 def _gemm_route(lib, M: int, N: int, K: int, dev: torch.device) -> tuple:
-    """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes, direct) of the GEMM
-    path for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count; direct:
-    fp32 activations run as one launch that casts them itself (g16_mm_t_direct)."""
+    """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes, direct, raw) of the
+    GEMM path for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count; direct:
+    fp32 activations run as one launch that casts them itself (g16_mm_t_direct); raw: fp16
+    activations as one launch that needs no cast (g16_mm_t_raw)."""
     key = (M, N, K, dev.index or 0)
     r = _routes.get(key)
     if r is None:
         cus = _sm_count(dev)
         scratch = lib.g16_mm_t_scratch_bytes(M, N, K, cus)
         if lib.g16_hgemm_use_packed(M, N, K, cus):
-            r = ("packed", scratch, 1, 0, 0, lib.g16_mm_t_direct_route(M, N, K, cus) == 1)
+            r = ("packed", scratch, 1, 0, 0, lib.g16_mm_t_direct_route(M, N, K, cus) == 1,
+                 lib.g16_mm_t_raw_route(M, N, K, cus) == 1)
         else:
             ksplit = lib.g16_hgemm_plan(M, N, K, cus)
             if ksplit > 1:
                 r = ("splitk", scratch, ksplit, lib.g16_hgemm_splitk_workspace_bytes(M, N, K, ksplit, cus),
-                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False)
+                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False, False)
             else:
-                r = ("plain", scratch, 1, 0, 0, False)
+                r = ("plain", scratch, 1, 0, 0, False, False)
         _remember(key, r)
     return r
 
@@ -167,7 +169,8 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     by a power of two, cast to fp16, multiplied on the matrix cores with fp32 accumulation and
     scaled back; shapes with too few output tiles split K with a deterministic reduction. (Large fp32
     batches into at most 1024 columns scale only the rows that leave fp16's range, 65504: the GEMM
-    casts x itself, and every value is rounded at least as finely.)"""
+    casts x itself, and every value is rounded at least as finely. Large fp16 batches are multiplied
+    as they are: nothing is rounded.)"""
     if out_dtype not in (torch.float32, torch.float16):
         raise ValueError(f"out_dtype must be float32 or float16, got {out_dtype}")
     _check_operands(x2d, w_t, bias)
@@ -208,9 +211,9 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     if x2d.dtype == torch.float16 and dev.index not in _spec_history:
         if lib.g16_mm_t_spec_history(stream) == 0:
             _spec_history.add(dev.index)
-    kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct = _gemm_route(lib, M, N, K, dev)
+    kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct, raw = _gemm_route(lib, M, N, K, dev)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
-    if direct and x2d.dtype == torch.float32:
+    if direct if x2d.dtype == torch.float32 else raw:
         _direct(lib, x2d, w_t, 0, out, bptr, M, N, K, dev, stream)
         return out
     # no scratch where the GEMM casts its own rows into LDS (one launch, the unsplit small tile)
@@ -225,10 +228,14 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
 
 def _direct(lib, x2d: torch.Tensor, w: torch.Tensor, packed: int, out: torch.Tensor, bptr, M: int, N: int, K: int,
             dev: torch.device, stream: int) -> None:
-    # fp32 activations into few columns (N <= 1024): the GEMM reads and casts x itself, no scratch
-    _clib.check(lib.g16_mm_t_direct(x2d.data_ptr(), w.data_ptr(), packed, out.data_ptr(),
-                                    1 if out.dtype == torch.float16 else 0, bptr, ROW_SCALE_THRESHOLD, M, N, K,
-                                    _sm_count(dev), stream), "GEMM")
+    # the GEMM reads x itself, without scratch: fp32 activations into few columns (N <= 1024), cast on
+    # the way; fp16 activations on the 256x256 tile, as they are
+    tail = (M, N, K, _sm_count(dev), stream)
+    head = (x2d.data_ptr(), w.data_ptr(), packed, out.data_ptr(), 1 if out.dtype == torch.float16 else 0, bptr)
+    if x2d.dtype == torch.float32:
+        _clib.check(lib.g16_mm_t_direct(*head, ROW_SCALE_THRESHOLD, *tail), "GEMM")
+    else:
+        _clib.check(lib.g16_mm_t_raw(*head, *tail), "GEMM")
 
 
 def prepacked_route(M: int, N: int, K: int, device: torch.device) -> bool:
@@ -360,7 +367,7 @@ def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias:
     b = None if bias is None else bias.float().contiguous()
     x2d = _aligned(x2d)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
-    if _cast_source is None and x2d.dtype == torch.float32 and _gemm_route(lib, M, N, K, dev)[5]:
+    if _cast_source is None and _gemm_route(lib, M, N, K, dev)[5 if x2d.dtype == torch.float32 else 6]:
         _direct(lib, x2d, wp, 1, out, None if b is None else b.data_ptr(), M, N, K, dev, stream)
         return out
     _scratch, xp, rscale = _packed_cast(lib, x2d, M, K, dev, stream, _cast_source)

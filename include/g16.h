@@ -174,6 +174,15 @@ int g16_mm_t_direct_route(int M, int N, int K, int num_cus);
 int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,
                     const float* bias, float thresh, int M, int N, int K, int num_cus, void* stream);
 
+/* mm_t's GEMM path for fp16 activations in one launch and without scratch, where g16_mm_t_raw_route()
+ * is 1 (0 elsewhere; g16_mm_t_raw then returns G16_E_SHAPE): the GEMM multiplies x as it is, rounding
+ * nothing, where the rowscale cast would scale rows past the threshold. The results are the same bits
+ * unless a scaled value falls below fp16's normal range; a row that holds an infinity gives NaN, as
+ * after the cast. `w` as for g16_mm_t_direct. */
+int g16_mm_t_raw_route(int M, int N, int K, int num_cus);
+int g16_mm_t_raw(const uint16_t* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,
+                 const float* bias, int M, int N, int K, int num_cus, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Prepacked weight for the large GEMM (no counterpart kernel in the reference; it serves
  * FastLinear, src/gtx16_fp16/linear.py:12-76, whose fp16 weight_t [K,N] is fixed after from_linear,

@@ -232,6 +232,22 @@ def test_one_launch_route_needs_no_scratch(lib):
         assert lib.g16_mm_t_scratch_bytes(M, N, K, 256) > 0, (M, N, K)
 
 
+def test_raw_route_rule_and_refusals(lib):
+    # fp16 activations as they are: unsplit 256x256 tiles; elsewhere the entry point refuses before any launch
+    r, d, A = lib.g16_mm_t_raw_route, lib.g16_mm_t_raw, 0x1000
+    assert r(4096, 4096, 4096, 256) == 1 and r(65536, 768, 768, 256) == 1 and r(8192, 2048, 2048, 256) == 1
+    assert r(2048, 4096, 4096, 256) == 0 and r(777, 8192, 3072, 256) == 0 and r(64, 1024, 1024, 256) == 0
+    assert r(0, 768, 768, 256) == 0 and r(65536, 768, 768, 0) == 0 and r(65536, 768, 0, 256) == 0
+    assert d(A, A, 0, A, 0, None, 2048, 4096, 4096, 256, None) == -1
+    assert d(A, A, 0, A, 0, None, 65536, 768, 772, 256, None) == -1
+    assert d(A + 4, A, 0, A, 0, None, 65536, 768, 768, 256, None) == -2
+    assert d(A, A + 8, 1, A, 0, None, 65536, 768, 768, 256, None) == -2
+    assert d(None, A, 0, A, 0, None, 65536, 768, 768, 256, None) == -3
+    assert d(A, A, 0, A, 0, None, 0, 768, 768, 256, None) == 0
+    need = lib.g16_mm_t_scratch_bytes(65536, 768, 768, 256)
+    assert lib.g16_mm_t_gemm(A, 0, A, A, 0, None, 1024.0, 65536, 768, 768, 256, A, need - 1, None, 0, None, 0, None) == -4
+
+
 def test_direct_route_rule_and_refusals(lib):
     # fp32 activations cast by the GEMM itself: unsplit 256x256 tiles, N <= 1024, three quarters of the
     # CUs busy; where the rule says 0 the entry point refuses before any launch

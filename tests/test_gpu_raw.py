@@ -1,0 +1,70 @@
+"""The raw GEMM route (g16_mm_t_raw: fp16 activations multiplied as they are on the unsplit 256x256 tile)
+against the two-launch sequence (rowscale cast, packed GEMM) and fp64: ragged M, N and K (a last tile of
+one row, K tails of 8 and 24, one K step), one round of tiles and persistent grids, fp32 and fp16
+outputs, both weight layouts, rows past the threshold, infinities and NaN in x, an infinite weight."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+import oracle
+from _inputs import outlier_rows, randn
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(2304, 256, 4096), (49153, 8, 256), (16640, 1048, 768), (4000, 1000, 5000), (65536, 152, 264)]
+KINDS = ["within", "outliers", "special"]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
+@pytest.mark.parametrize("kind", KINDS)
+def test_raw_equals_the_two_launch_sequence(cuda, M, K, N, kind):
+    import gtx16_fp16 as g
+    from gtx16_fp16 import _clib, ops
+
+    lib = _clib.load()
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    if cus != 256:
+        pytest.skip(f"the shapes are for 256 CUs (this device has {cus})")
+    assert lib.g16_mm_t_raw_route(M, N, K, cus) == 1
+    x = randn((M, K), seed=M + K)
+    w = randn((K, N), seed=1, scale=0.02, dtype=torch.float16)
+    bias = randn((N,), seed=2, scale=0.02)
+    if kind == "outliers":
+        x = outlier_rows(x, 0.05, 2e3, 8e3, seed=3)
+    elif kind == "special":
+        for r, k, v in ((0, K - 1, "inf"), (255, 0, "-inf"), (256, K // 2, "nan"), (M - 1, K - 1, "-inf")):
+            x[r, k] = float(v)
+        w[K - 1, N - 3] = float("inf")  # an infinite sum that no infinite activation makes
+        w[0, 1] = 0.0
+    xd, wd, b = x.half().to(cuda), w.to(cuda), bias.to(cuda)
+    wp = ops.pack_weight(wd)
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    xp = torch.empty(lib.g16_packed_a_bytes(M, K) // 2, dtype=torch.float16, device=cuda)
+    s = torch.empty(M, device=cuda)
+    assert lib.g16_rowscale_pack_f16(xd.data_ptr(), xp.data_ptr(), s.data_ptr(), M, K, 1024.0, st) == 0
+    for odt, bits in ((torch.float32, torch.int32), (torch.float16, torch.int16)):
+        two = torch.empty(M, N, dtype=odt, device=cuda)
+        fn = lib.g16_hgemm_packed_ab_f16out if odt == torch.float16 else lib.g16_hgemm_packed_ab_f32out
+        assert fn(xp.data_ptr(), wp.data_ptr(), two.data_ptr(), b.data_ptr(), s.data_ptr(), M, N, K, st) == 0
+        outs = [g.mm_t(xd, wd, b, odt), ops.mm_t_prepacked(xd, wd, wp, b, odt), g.mm_t(xd, wd, b, odt)]
+        torch.cuda.synchronize()
+        y = outs[0]
+        for o in outs[1:]:
+            assert torch.equal(o.view(bits), y.view(bits))
+        assert torch.equal(torch.isnan(y), torch.isnan(two)) and torch.equal(torch.isinf(y), torch.isinf(two))
+        if kind == "within":
+            assert torch.equal(y.view(bits), two.view(bits))
+        if kind == "special":
+            assert torch.isnan(y[[0, 255, 256, M - 1]]).all() and torch.isinf(y[1, N - 3])
+            fin = torch.isfinite(two)
+            assert torch.equal(y[fin], two[fin])  # no finite row is scaled
+            continue
+        rows = list(range(64)) + [255, 256, M // 2, M - 1]
+        ref = xd[rows].double() @ wd.double() + b.double()
+        err, err2 = ((o[rows].double() - ref).norm(dim=1) / ref.norm(dim=1) for o in (y, two))
+        # exact products, fp32 sums, one rounding of an fp16 output (2^-11 per value)
+        assert (err <= (2.0 ** -10 if odt == torch.float16 else 1e-5)).all(), err.max()
+        assert (err <= err2 * 1.001 + 1e-7).all(), (err.max(), err2.max())
+        want = oracle.mm_t(xd[rows].cpu().numpy(), w.numpy(), bias.numpy(), str(odt).split(".")[1])
+        assert oracle.rel_err(y[rows].cpu().numpy(), want) <= 1e-3
