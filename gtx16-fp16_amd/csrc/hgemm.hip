@@ -1572,6 +1572,9 @@ struct Plan {
   int bm, bn;
   int ntm, ntn;
   int ks = 0;  // the split the tile was chosen with (the modelled choice below); 0: the planner's rule
+  // fp16 x without scratch runs raw (row-major x as A): a medium batch, like those on the 4-wavefront
+  // tiles, whose one-launch route needs no scratch either
+  bool raw_without_scratch = false;
 };
 
 // The 4-wavefront tiles (32x32x16 MFMA blocks, one barrier per K step): the ones the speculative
@@ -1723,6 +1726,16 @@ Plan choose_tile(int M, int N, int K, int num_cus) {
     } else {
       p.tile = Tile::T256; p.bm = 256; p.bn = 256;
     }
+  } else if (M >= 512 && N >= 256 && K > 1024 && 4L * ceil_div(M, 128) * ceil_div(N, 128) >= 5L * num_cus &&
+             static_cast<long>(ceil_div(M, 256)) * ceil_div(N, 128) <= num_cus) {
+    // 128x128 tiles would need 1.25 rounds or more and one round of 256x128 tiles holds the grid,
+    // padding rows and all (packed A; graph-timed, M x K x N, fp16 / fp32 x, 128x128 -> 256x128: 777 x
+    // 3072 x 8192 68.7 / 67.0 -> 57.0 / 57.9 us, 520 x 3072 x 10240 67.5 / 66.7 -> 57.0 / 57.9, 1000 x
+    // 1536 x 8192 46.2 / 48.8 -> 36.0 / 36.7, 1280 x 2048 x 4096 54.6 / 55.2 -> 42.7 / 44.2, 1280 x 3072
+    // x 4096 78.9 / 77.1 -> 57.9 / 59.2). At K = 1024 the cast takes most of the gain (777 x 8192: 30.0
+    // -> 27.2): 128x128 tiles there.
+    p.tile = Tile::T256N; p.bm = 256; p.bn = 128;
+    p.raw_without_scratch = true;
   } else {
     p.tile = Tile::T128; p.bm = 128; p.bn = 128;
   }
@@ -1738,6 +1751,7 @@ using GemmFn = void (*)(const _Float16*, const _Float16*, void*, const float*, c
 template <bool OUT_F16>
 GemmFn<OUT_F16> gemm_fn(Tile t, bool splitk, bool packed, bool packed_b, bool resident = false, bool spec = false,
                         bool direct = false, bool raw = false) {
+  if (raw && t == Tile::T256N) return hgemm_kernel<Cfg256n, OUT_F16, false, false, false, false, false, false, true>;
   if (raw)
     return packed_b ? hgemm_kernel<Cfg256, OUT_F16, false, false, true, false, false, false, true>
                     : hgemm_kernel<Cfg256, OUT_F16, false, false, false, false, false, false, true>;
@@ -1900,7 +1914,7 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   if (num_cus <= 0) num_cus = stream_cus(static_cast<hipStream_t>(stream));
   Plan p = choose_tile(M, N, K, num_cus);
   if (direct ? !direct_route(p, N, K, ks.ksplit, num_cus) && !stream_route(p, M, K, ks) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
-  if (raw && !raw_route(p, K, ks.ksplit)) return G16_E_SHAPE;
+  if (raw && !raw_route(p, K, ks.ksplit) && !(p.raw_without_scratch && ks.ksplit == 1 && !packed_b)) return G16_E_SHAPE;
   const bool spec = sp != nullptr;
   if (spec && (!four_wave(p.tile) || packed ||
                ks.ksplit > kSpecMaxSplit || sp->texp < kSpecMinTexp))
@@ -2177,9 +2191,14 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
     return g16::gemm_launch(nullptr, w_t, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus, nullptr, 0, nullptr,
                             0, stream, false, false, &rc);
   }
+  const bool has_scratch = scratch != nullptr && g16::aligned16(scratch) &&
+                           scratch_bytes >= g16_mm_t_scratch_bytes(M, N, K, num_cus);
+  if (!has_scratch && !x_is_f32 && texp >= g16::kSpecMinTexp && g16::choose_tile(M, N, K, num_cus).raw_without_scratch)
+    return g16::gemm_launch(static_cast<const uint16_t*>(x), w_t, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus,
+                            nullptr, 0, nullptr, 0, stream, false, false, nullptr, nullptr, false, true);
   if (scratch == nullptr) return G16_E_NULL;
   if (!g16::aligned16(scratch)) return G16_E_ALIGN;
-  if (scratch_bytes < g16_mm_t_scratch_bytes(M, N, K, num_cus)) return G16_E_WORKSPACE;
+  if (!has_scratch) return G16_E_WORKSPACE;
   if (!x_is_f32 && g16_mm_t_raw_route(M, N, K, num_cus) == 1)
     return g16_mm_t_raw(static_cast<const uint16_t*>(x), w_t, 0, out, out_is_f16, bias, M, N, K, num_cus, stream);
   if (x_is_f32 && g16::direct_thresh(texp) && g16_mm_t_direct_route(M, N, K, num_cus) == 1)

@@ -232,6 +232,23 @@ def test_one_launch_route_needs_no_scratch(lib):
         assert lib.g16_mm_t_scratch_bytes(M, N, K, 256) > 0, (M, N, K)
 
 
+def test_medium_batches_take_256x128_tiles_in_one_round(lib):
+    import ctypes
+
+    def tile(M, N, K):
+        r, c = ctypes.c_int(), ctypes.c_int()
+        assert lib.g16_hgemm_tile(M, N, K, 256, ctypes.byref(r), ctypes.byref(c)) == 0
+        return r.value, c.value, lib.g16_hgemm_plan(M, N, K, 256)
+
+    # where 128x128 tiles need 1.25 rounds and 256x128 tiles fit one, also with padding rows
+    for M, N, K in [(777, 8192, 3072), (520, 10240, 3072), (1280, 4096, 2048), (1000, 8192, 1032), (777, 6144, 3072)]:
+        assert tile(M, N, K) == (256, 128, 1), (M, N, K)
+        assert lib.g16_hgemm_use_packed(M, N, K, 256) == 1 and lib.g16_mm_t_raw_route(M, N, K, 256) == 0
+    assert tile(777, 8192, 1024) == (128, 128, 1)    # short K
+    assert tile(520, 8192 + 128, 3072) == (256, 128, 1) and tile(511, 14336, 3072)[:2] == (128, 128)
+    assert tile(1000, 4096, 3072) == (128, 128, 1)   # one round of 128x128 tiles
+
+
 def test_raw_route_rule_and_refusals(lib):
     # fp16 activations as they are: unsplit 256x256 tiles; elsewhere the entry point refuses before any launch
     r, d, A = lib.g16_mm_t_raw_route, lib.g16_mm_t_raw, 0x1000

@@ -68,3 +68,49 @@ def test_raw_equals_the_two_launch_sequence(cuda, M, K, N, kind):
         assert (err <= err2 * 1.001 + 1e-7).all(), (err.max(), err2.max())
         want = oracle.mm_t(xd[rows].cpu().numpy(), w.numpy(), bias.numpy(), str(odt).split(".")[1])
         assert oracle.rel_err(y[rows].cpu().numpy(), want) <= 1e-3
+
+
+@pytest.mark.parametrize("M,K,N", [(777, 1096, 8192), (513, 1048, 10248), (1280, 2048, 4096)])
+@pytest.mark.parametrize("kind", KINDS)
+def test_medium_batches_with_and_without_scratch(cuda, M, K, N, kind):
+    # 256x128 tiles in one round: mm_t and FastLinear cast and pack x, a C caller without scratch gets
+    # the raw launch; the two-launch sequence's bits where no row is scaled, NaN rows alike
+    import torch.nn as nn
+
+    import gtx16_fp16 as g
+    from gtx16_fp16 import _clib
+
+    lib = _clib.load()
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    if cus != 256:
+        pytest.skip(f"the shapes are for 256 CUs (this device has {cus})")
+    x = randn((M, K), seed=M + K)
+    if kind == "outliers":
+        x = outlier_rows(x, 0.05, 2e3, 8e3, seed=3)
+    elif kind == "special":
+        x[0, K - 1], x[M - 1, 0], x[5, 7] = float("inf"), -float("inf"), float("nan")
+    w, bias = randn((K, N), seed=1, scale=0.02, dtype=torch.float16), randn((N,), seed=2, scale=0.02)
+    wd, b = w.to(cuda), bias.to(cuda)
+    fl = g.FastLinear(K, N, device=cuda)
+    fl.weight_t, fl.bias = wd, b
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    for dt in (torch.float16, torch.float32):
+        xd = x.to(dt).to(cuda)
+        y = g.mm_t(xd, wd, b, dt)
+        assert torch.equal(fl(xd).nan_to_num(1.0), y.nan_to_num(1.0)) and fl._wp is None
+        fin = torch.isfinite(xd).all(1)
+        assert torch.isnan(y[~fin]).all() and torch.isfinite(y[fin]).all()
+        ref = xd[fin].double() @ wd.double() + b.double()
+        err = (y[fin].double() - ref).norm(dim=1) / ref.norm(dim=1)
+        # fp16 rounding of the activations and of an fp16 output: 2^-11 per value each
+        assert (err <= 2.0 ** -10).all(), err.max()
+        out = torch.empty_like(y)
+        rc = lib.g16_mm_t_gemm(xd.data_ptr(), int(dt == torch.float32), wd.data_ptr(), out.data_ptr(),
+                               int(dt == torch.float16), b.data_ptr(), 1024.0, M, N, K, cus, None, 0, None, 0, None, 0, st)
+        assert rc == (-3 if dt == torch.float32 else 0)  # fp32 x needs its scratch, as on other tiles
+        if rc == 0:
+            assert torch.equal(torch.isnan(out), torch.isnan(y))
+            err = (out[fin].double() - ref).norm(dim=1) / ref.norm(dim=1)
+            assert (err <= 2.0 ** -10).all(), err.max()
+            if kind != "outliers":
+                assert torch.equal(out[fin], y[fin])
