@@ -25,8 +25,7 @@
 //     strip, and the last arriver reads slices x M x width partial sums back through one CU.
 //     Up to N = 8192 the strips are 256 columns (half the slices of 512-column strips and a 4x
 //     smaller read-back; 128-column strips stream worse: 1 x 4096^2 in 8.58-8.62 us, against
-//     9.11-9.16 with 512 columns and 8.91-8.98 with 128), above that 512, except at M >= 7
-//     (strip_cols).
+//     9.11-9.16 with 512 columns and 8.91-8.98 with 128), above that 512 (strip_cols).
 #include <mutex>
 #include <type_traits>
 
@@ -579,12 +578,13 @@ template <int MM> struct SchedFor<MM, 512> {
 // last arriver's read-back (slices x M x strip width) dominates the exchange, which the narrow
 // strips cut 4x (1 x 4096^2: 9.16 -> 8.63 us; 6 x 4096^2: 14.87 -> 10.98); with many strips the
 // split is shallow already and the 1 KB rows stream slightly better (1 x 4096 x 11008: 16.77 us
-// with 512 columns, 16.90 with 256). M = 7 and 8 take 256 columns throughout: the matrix-core form
-// needs them, and gains more than the wide rows (fp32 x, 512-column FMA loop -> 256-column matrix
-// cores: 7 x 4096 x 11008 23.8 -> 21.9 us, 8 x 4096 x 11008 25.6 -> 22.1, 8 x 8192 x 9216 42.2 -> 37.7,
-// 7 x 512 x 9000 9.9 -> 7.7, 8 x 8192 x 28672 84.3 -> 82.3, 7 x 8192 x 28672 80.4 -> 81.5); M = 5 and 6
-// do not (5 x 8192 x 9216 34.5 vs 38.9, 6 x 4096 x 14336 24.6 vs 25.5).
-int strip_cols(int M, int N) { return N <= 8192 || M >= 7 ? 256 : 512; }
+// with 512 columns, 16.90 with 256; 8 x 4096 x 14336: 27.3 vs 31.9; 5 x 8192 x 9216 34.5 vs 38.9).
+// Counter areas are sized by it (g16_skinny_counter_bytes, the fixed 64 KiB of the no-allocation
+// form), so it depends on neither the activations' type nor the form that runs.
+int strip_cols(int M, int N) {
+  (void)M;
+  return N <= 8192 ? 256 : 512;
+}
 
 template <typename TX, int COLS>
 SkinnyFn<TX> skinny_fn_w(int M) {
@@ -605,11 +605,9 @@ SkinnyFn<TX> skinny_fn_w(int M) {
 // wavefront), fp32 activations: M = 8 4096 x 4096 (32) 12.69 vs 12.95, 11008 x 4096 (86) 20.50 vs
 // 25.52; M = 7 4096 x 8192 (64) 16.36 vs 17.29, 11008 x 4096 21.0 vs 23.5, but 4096 x 4096 12.4 vs
 // 11.3; M = 6 11008 x 4096 21.0 vs 22.2, but 4096 x 8192 16.7 vs 16.3; M = 5 11008 x 4096 21.5 vs
-// 21.8. fp16: M = 8 4096 x 4096 11.7 vs 12.6, 11008 x 4096 20.3 vs 24.0; M = 5 19.8 vs 20.8. With
-// one batch per wavefront and few slices (N > 8192) the FMA loop is the faster and more accurate one
-// at M = 8 too (7 x 1536 x 10240, 32 rows: 10.7 us against 11.9 on the matrix cores).
-bool use_mf(int M, int N, int cols, int rows_per_wave) {
-  return cols == 256 && M >= 5 && rows_per_wave >= (M == 8 && N <= 8192 ? kMfBatch : (M >= 7 ? 64 : 80));
+// 21.8. fp16: M = 8 4096 x 4096 11.7 vs 12.6, 11008 x 4096 20.3 vs 24.0; M = 5 19.8 vs 20.8.
+bool use_mf(int M, int cols, int rows_per_wave) {
+  return cols == 256 && M >= 5 && rows_per_wave >= (M == 8 ? kMfBatch : (M == 7 ? 64 : 80));
 }
 template <typename TX>
 SkinnyFn<TX> skinny_fn(int M, int cols, bool mf) {
@@ -681,7 +679,7 @@ int skinny_launch(const TX* A, const uint16_t* B, void* C, int c_f16, const floa
     part = static_cast<float*>(ws);
   }
   const dim3 grid(static_cast<unsigned>(nstrips) * static_cast<unsigned>(sp.ksplit)), block(kThreads);
-  return launch(skinny_fn<TX>(M, cols, use_mf(M, N, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
+  return launch(skinny_fn<TX>(M, cols, use_mf(M, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
                 reinterpret_cast<const _Float16*>(B), C, c_f16, bias, part, counters, N, K, sp.rows_per_wave, sp.ksplit,
                 nstrips);
 }

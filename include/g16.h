@@ -233,7 +233,7 @@ int g16_hgemm_tile(int M, int N, int K, int num_cus, int* rows, int* cols);
  * configuration skinny_config (src/gtx16_fp16/ops.py:45-51,78-84; src/gtx16_fp16/linear.py:49-64).
  * A is read with 16-byte alignment (A must be 16-byte aligned, like B).
  * The kernel streams B once with 16-byte loads; K is split over ksplit workgroups per strip of
- * g16_skinny_strip_cols(M, N) columns (256 up to N = 8192 and for M >= 7, else 512) and reduced
+ * g16_skinny_strip_cols(M, N) columns (256 up to N = 8192, 512 above) and reduced
  * deterministically (last arriving workgroup, slice order). C needs no zero-fill.
  * The split workspace (ksplit * M * N * 4 bytes) must stay below 2 GiB (G16_E_SPLIT otherwise).
  * g16_skinny_plan() returns the ksplit this library would choose for num_cus compute units; the

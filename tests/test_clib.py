@@ -287,6 +287,17 @@ def test_direct_route_rule_and_refusals(lib):
     assert lib.g16_mm_t_gemm(A, 1, A, A, 0, None, 1024.0, 65536, 768, 768, 256, A, need - 1, None, 0, None, 0, None) == -4
 
 
+def test_skinny_strips_fit_the_counter_areas_at_every_m(lib):
+    # one strip width for every M: a split launch's counters are 256 bytes per strip of 512 columns
+    # past N = 8192, so the fixed 64 KiB of the no-allocation form take N up to 131072 at M = 7 and 8
+    # too (7 x 70000 in two slices keeps its partial sums, 3.9 MB, inside that form's 4 MiB)
+    for M in range(1, 9):
+        for N, strips in ((8192, 32), (8200, 17), (11008, 22), (70000, 137), (74888, 147), (131072, 256)):
+            assert lib.g16_skinny_strip_cols(M, N) == (256 if N <= 8192 else 512)
+            assert lib.g16_skinny_counter_bytes(M, N, 4096, 2) == strips * 256 <= 64 * 1024
+    assert lib.g16_skinny_workspace_bytes(7, 74888, 4096, 2) <= 4 << 20
+
+
 def test_fast_extension_matches_the_c_entry_points(lib):
     # _g16fast forwards its arguments unchanged: the same rejected calls give the same statuses
     fast = _clib.fast()
