@@ -95,8 +95,8 @@ __device__ inline void fma_row(float (&acc)[MM][8], const float (&a)[MM], u32x4 
 }
 
 // Two fp16 parts of a finite x (|x| < 2^15 after the row scaling): hi is x rounded toward zero to
-// fp16, lo the rest rounded to nearest, so |x - hi - lo| <= 2^-21 |x| (<= 2^-25 where lo is
-// subnormal), and an fp16 x gives hi = x. Both parts carry x's sign: a part that would be zero for
+// fp16, lo the rest rounded to nearest, so |x - hi - lo| <= 2^-21 |x| (or 2^-25 where lo is
+// subnormal: 2^-39 of a row's largest |x|, which is >= 2^14), and an fp16 x gives hi = x. Both parts carry x's sign: a part that would be zero for
 // a nonzero x is the smallest subnormal (2^-24) with x's sign instead (an error of <= 2^-23,
 // negligible next to a row whose largest |x| is >= 2^14). An infinite weight times (hi, lo)
 // therefore gives the infinity the fp32 product gives, never inf - inf; x = +-0 gives (+-0, 0), and
@@ -111,9 +111,9 @@ __device__ inline void split_hi_lo(float x, _Float16& hi, _Float16& lo) {
   lo = __builtin_bit_cast(_Float16, hz ? (xz ? static_cast<uint16_t>(0u) : tiny) : ((lb & 0x7fffu) == 0 ? tiny : lb));
 }
 
-// MF (launched by use_mf: larger M on 256-column strips, enough K rows per wavefront): a wavefront
-// whose activations are all finite multiplies on the matrix cores (below); one with an inf or NaN
-// among them takes the fp32 FMA loop.
+// MF (launched by use_mf: larger M on 256-column strips, enough K rows per wavefront): the wavefront
+// multiplies on the matrix cores (below), with fp32 activations only if all of its are finite; one
+// with an inf or NaN among them takes the fp32 FMA loop.
 template <typename TX, int MM, class S, bool MF = false>
 __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__ A, const _Float16* __restrict__ B,
                                                           void* __restrict__ Cv, int c_f16, const float* __restrict__ bias,
@@ -209,14 +209,11 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
     constexpr bool XF16 = std::is_same_v<TX, _Float16>;
     // fp16 activations are their own A fragments: no scale, no lo parts (A rows 8-15 are 0 and their
     // sums, which an infinite weight makes NaN, are not used), and infinities and NaN multiply as in
-    // the FMA loop.
-    //   The activations are held kMfGroup batches at a time. Their row exponents only rise: a group
-    // with a larger |x| in row m scales the row's sums down to the new exponent (exact) and goes on in
-    // it, so the parts of every x are exact to 2^-38 of the row's largest |x| so far.
+    // the FMA loop. They are held kMfGroup batches at a time; fp32 ones are a single such group
+    // (use_mf), whose largest |x| per row gives the row's exponent.
     std::conditional_t<XF16, _Float16, float> xr[kMfGroup][8];
     float4v acc2[2][8];
-    constexpr int kNoExp = -1000;  // no nonzero activation in the row yet
-    int e = kNoExp;
+    int e = 0;
     if (rows_per_wave >= kMfBatch) {
       fma_loop = false;
 #pragma unroll
@@ -257,19 +254,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
           }
           amax = fmaxf(amax, __shfl_xor(amax, 16));
           amax = fmaxf(amax, __shfl_xor(amax, 32));
-          // amax * 2^-e in [2^14, 2^15)
-          const int en = amax > 0.f ? max(e, __builtin_amdgcn_frexp_expf(amax) - 15) : e;
-          if (g0 > 0 && __any(en != e)) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int d = __shfl(e - en, 4 * (g & 1) + i);
-#pragma unroll
-              for (int s = 0; s < 2; ++s)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc2[s][j][i] = __builtin_ldexpf(acc2[s][j][i], d);
-            }
-          }
-          e = en;
+          e = amax > 0.f ? __builtin_amdgcn_frexp_expf(amax) - 15 : 0;  // amax * 2^-e in [2^14, 2^15)
         }
 #pragma unroll
         for (int bt = 0; bt < kMfGroup; ++bt) {
@@ -599,25 +584,32 @@ SkinnyFn<TX> skinny_fn_w(int M) {
     default: return skinny_kernel<TX, 8, typename SchedFor<8, COLS>::type>;
   }
 }
-// The matrix-core form (skinny_kernel's MF) runs where it pays: 256-column strips and enough K rows
-// per wavefront to hide its work (permutes, hi/lo split) behind the weights' loads, more at smaller M.
-// Graph-timed against the FMA loop, weights rotated past the Infinity Cache, us (K x N, rows per
-// wavefront), fp32 activations: M = 8 4096 x 4096 (32) 12.69 vs 12.95, 11008 x 4096 (86) 20.50 vs
-// 25.52; M = 7 4096 x 8192 (64) 16.36 vs 17.29, 11008 x 4096 21.0 vs 23.5, but 4096 x 4096 12.4 vs
-// 11.3; M = 6 11008 x 4096 21.0 vs 22.2, but 4096 x 8192 16.7 vs 16.3; M = 5 11008 x 4096 21.5 vs
-// 21.8. fp16: M = 8 4096 x 4096 11.7 vs 12.6, 11008 x 4096 20.3 vs 24.0; M = 5 19.8 vs 20.8.
+// The matrix-core form (skinny_kernel's MF) runs on 256-column strips with enough K rows per wavefront
+// to hide its work (permutes, hi/lo split) behind the weights' loads. Graph-timed against the FMA
+// loop, weights rotated past the Infinity Cache, us (K x N, rows per wavefront):
+//   * fp32 activations: M = 8 and 32..128 rows. 4096 x 4096 (32) 12.69 vs 12.95, 11008 x 4096 (86)
+//     20.50 vs 25.52, 14336 x 4096 24.80 vs 29.29, 4096 x 8192 16.52 vs 19.18. Elsewhere the FMA loop
+//     keeps all 24 bits of x where the two fp16 parts keep 21; at M = 5 to 7 the parts would save
+//     at most 10 % (7 x 11008 x 4096 21.0 vs 23.5, 5 x 11008 x 4096 21.5 vs 21.8).
+//   * fp16 activations, which lose nothing: M = 8 from 32 rows (4096 x 4096 11.7 vs 12.6, 11008 x 4096
+//     20.3 vs 24.0), M = 7 from 64, M = 5 and 6 from 80 (5 x 11008 x 4096 19.8 vs 20.8).
+template <typename TX>
 bool use_mf(int M, int cols, int rows_per_wave) {
-  return cols == 256 && M >= 5 && rows_per_wave >= (M == 8 ? kMfBatch : (M == 7 ? 64 : 80));
+  if (cols != 256) return false;
+  if (std::is_same_v<TX, float>) return M == 8 && rows_per_wave >= kMfBatch && rows_per_wave <= kMfBatch * kMfGroup;
+  return M >= 5 && rows_per_wave >= (M == 8 ? kMfBatch : (M == 7 ? 64 : 80));
 }
 template <typename TX>
 SkinnyFn<TX> skinny_fn(int M, int cols, bool mf) {
   if (mf) {
-    switch (M) {
-      case 5: return skinny_kernel<TX, 5, typename SchedFor<5, 256>::type, true>;
-      case 6: return skinny_kernel<TX, 6, typename SchedFor<6, 256>::type, true>;
-      case 7: return skinny_kernel<TX, 7, typename SchedFor<7, 256>::type, true>;
-      default: return skinny_kernel<TX, 8, typename SchedFor<8, 256>::type, true>;
+    if constexpr (std::is_same_v<TX, _Float16>) {
+      switch (M) {
+        case 5: return skinny_kernel<TX, 5, typename SchedFor<5, 256>::type, true>;
+        case 6: return skinny_kernel<TX, 6, typename SchedFor<6, 256>::type, true>;
+        case 7: return skinny_kernel<TX, 7, typename SchedFor<7, 256>::type, true>;
+      }
     }
+    return skinny_kernel<TX, 8, typename SchedFor<8, 256>::type, true>;
   }
   return cols == 256 ? skinny_fn_w<TX, 256>(M) : skinny_fn_w<TX, 512>(M);
 }
@@ -679,7 +671,7 @@ int skinny_launch(const TX* A, const uint16_t* B, void* C, int c_f16, const floa
     part = static_cast<float*>(ws);
   }
   const dim3 grid(static_cast<unsigned>(nstrips) * static_cast<unsigned>(sp.ksplit)), block(kThreads);
-  return launch(skinny_fn<TX>(M, cols, use_mf(M, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
+  return launch(skinny_fn<TX>(M, cols, use_mf<TX>(M, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
                 reinterpret_cast<const _Float16*>(B), C, c_f16, bias, part, counters, N, K, sp.rows_per_wave, sp.ksplit,
                 nstrips);
 }

@@ -131,3 +131,31 @@ def test_skinny_matrix_core_groups(cuda, M, K, N, kind, dt):
     assert torch.equal(torch.isposinf(y), torch.isposinf(want)) and torch.equal(torch.isneginf(y), torch.isneginf(want))
     fin = torch.isfinite(want)
     assert (y.double()[fin] - want[fin]).norm() <= 1e-5 * want[fin].norm()
+
+
+# shapes whose wavefronts hold enough K rows for the matrix cores, and one on 512-column strips; fp32
+# activations take them at M = 8 with 32 to 128 rows only, which none of these is
+@pytest.mark.parametrize("M,K,N", [(5, 11008, 4096), (6, 14336, 4096), (7, 11008, 4096), (7, 4096, 11008), (8, 20480, 8192),
+                                   (8, 4104, 8712)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_skinny_multiplies_every_bit_of_the_activations(cuda, M, K, N, dt):
+    import gtx16_fp16 as g
+
+    w = randn((K, N), seed=N, scale=0.02, dtype=torch.float16)
+    x = randn((M, K), seed=K + M)
+    x[1] = 0.0
+    x[1, K // 3] = 1.0 + 2.0 ** -23       # one-hot, all 24 bits (fp16: rounds to 1)
+    x[2] = 0.0
+    x[2, 0], x[2, 7] = 3e4, 1e-3 / 3       # a large value that meets a zero weight, in one wavefront
+    w[0] = 0.0
+    x = x.to(dt)
+    y = g.mm_t(x.to(cuda), w.to(cuda)).cpu().double()
+    # a single product, rounded once to fp32 (2^-24) and added to zeros; the product itself is exact
+    for row, k in ((1, K // 3), (2, 7)):
+        want = x[row, k].double() * w[k].double()
+        assert ((y[row] - want).abs() <= 2.0 ** -24 * want.abs()).all(), (row, (y[row] - want).abs().max())
+    # every output: at most n roundings of 2^-24 each along its chain of sums, n < 512 here (the rows
+    # of a wavefront, two parts, eight wavefronts, the slices), on sum |x w|
+    x64, w64 = x.to(cuda).double(), w.to(cuda).double()
+    bound = (512 * 2.0 ** -24 * (x64.abs() @ w64.abs())).cpu()
+    assert ((y - (x64 @ w64).cpu()).abs() <= bound).all()
