@@ -238,9 +238,9 @@ __device__ inline uint32_t arrive_add_coherent(uint32_t* counter, uint32_t add) 
   __syncthreads();
   return s_val;
 }
-// Split counter of a speculative launch: the arrival count in the low kSpecShift bits, and bit
-// kSpecShift + z set by slice z if its A exceeded the threshold (each slice adds its own bit once,
-// so the fields never carry into each other).
+// Split counter of a speculative or direct launch: the arrival count in the low kSpecShift bits, and
+// bit kSpecShift + z set by slice z if its A exceeded the threshold (speculative) or made it rescale a
+// row (direct); each slice adds its own bit once, so the fields never carry into each other.
 constexpr int kSpecShift = 8;
 constexpr int kSpecMaxSplit = 32 - kSpecShift;
 
@@ -260,7 +260,12 @@ __device__ inline void phase_barrier() { asm volatile("s_barrier" ::: "memory");
 // DIRECT: A is unused; the kernel streams the fp32 activations X itself, casts them on the way into the
 // A stages and rescales a row as soon as a value of it leaves fp16's range: the unsplit 256x256 tile
 // (through registers), and the 4-wavefront tiles with 64-deep K steps, split or not (through a ring of
-// fp32 stages in LDS; a slice rescales by what it has seen, and publishes its sums in units of 1).
+// fp32 stages in LDS). A slice rescales by what it has seen. One that did publishes its rows' factors
+// beside its sums, in rscale[(tn * ksplit + z) * M + row] (which such a launch writes; it has no row
+// scales; one place per tile column tn, as 36 columns storing to one took 5 us at 11 x 2944 x 4608), and the
+// slice that arrives last brings every slice's sums to the row's smallest factor before it adds them,
+// so that no sum leaves the scaled units before the epilogue: partial sums past fp32's range that
+// cancel do not overflow.
 // RAW: A is the fp16 activations, row-major; rows that hold an infinity give NaN.
 template <class Cfg, bool OUT_F16, bool SPLITK, bool PACKED_A = false, bool PACKED_B = false, bool RESIDENT = false,
           bool SPEC = false, bool DIRECT = false, bool RAW = false>
@@ -706,7 +711,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
     //   Rescaling as on the 256x256 tile: a step with a value past fp16's range raises its row's
     // exponent, scales its values, and leaves the factor for the accumulators, which every wavefront
     // applies before its MFMAs of that step; the row's later steps are scaled as they are cast.
-    auto stream_loop = [&]() __attribute__((always_inline)) {
+    auto stream_loop = [&]() __attribute__((always_inline)) -> int {  // 1: this wavefront rescaled a row
       constexpr int RW = BM / 4;              // rows per wavefront
       constexpr int AI = RW / 4;              // its DMA instructions per step (4 rows of 256 bytes each)
       constexpr int H = RW / 8;               // 8-row groups: lane l casts 8 values of row 8 h + l / 8
@@ -861,7 +866,9 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
         step(std::integral_constant<int, 1>{}, it + 1);
       }
       if (it < nk) step(std::integral_constant<int, 0>{}, it);
+      return scaled;
     };
+    [[maybe_unused]] int rescaled = 0;  // direct A on the 4-wavefront tiles: stream_loop's result
     if constexpr (Cfg::WAVES == 8) {
       // Ping-pong schedule for two wavefronts per SIMD. Wavefronts 0-3 (group 0) and 4-7 (group 1)
       // land one of each on every SIMD. Each wavefront alternates a memory phase M_j (fragment reads
@@ -1163,7 +1170,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       }
       if (grp == 0) phase_barrier();  // every wavefront passes the same number of barriers
     } else {
-      if constexpr (STREAM) stream_loop();
+      if constexpr (STREAM) rescaled = stream_loop();
       else if constexpr (RESIDENT) kloop4(std::true_type{}, std::false_type{});
       else kloop4(std::false_type{}, std::false_type{});
     }
@@ -1259,19 +1266,6 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
     // 1 / factor: a power of two's exponent negated, infinity for a row's factor 0
     auto inv_factor = [](float f) { return __uint_as_float(f == 0.f ? 0x7f800000u : 0x7f000000u - __float_as_uint(f)); };
     // ---- split-K: publish this slice, let the last slice reduce ----
-    if constexpr (SPLITK && STREAM) {
-      // the slice's rows have factors of their own: its sums leave in units of 1
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4v f = *reinterpret_cast<const float4v*>(&s_fac[wm0 + 32 * i + 8 * q + 4 * fk]);
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[i][j][4 * q + r] *= inv_factor(f[r]);
-        }
-    }
     if constexpr (SPLITK) {
       constexpr uint32_t TILE_BYTES = BM * BN * 4;
       // Each wavefront stores its accumulators in its own register order: slot s of the wavefront is
@@ -1316,7 +1310,39 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
 #pragma unroll
         for (int s = 0; s < SLOTS; ++s) store_coherent4(slices, slot_off(z, s), piece(s));
       }
-      if constexpr (SPEC) {
+      [[maybe_unused]] uint32_t rejoin = 0;  // direct: bit z set if slice z rescaled a row
+      // rows past M have no place in rscale; their sums are not stored
+      [[maybe_unused]] float* const facs = const_cast<float*>(rscale) + static_cast<size_t>(tn) * ksplit * M + m0;
+      // the rows' smallest factors into s_fac, and what slice z's sums are multiplied by into
+      // s_join[z * BM + row] (the fp32 stages are free). Factor 0 of an infinite row: 0 * inf = NaN,
+      // which its sums are already.
+      float* const s_join = reinterpret_cast<float*>(&sX[0][0]);
+      [[maybe_unused]] auto join_factors = [&]() __attribute__((always_inline)) {
+        for (int i = tid; i < ksplit * BM; i += Cfg::THREADS) {
+          const int zz = i / BM, r = i % BM;
+          s_join[i] = ((rejoin >> zz) & 1u) != 0u && m0 + r < M ? load_coherent(facs + static_cast<size_t>(zz) * M + r) : 1.f;
+        }
+        __syncthreads();
+        if (tid < BM) {
+          float f = 1.f;
+          for (int z0 = 0; z0 < ksplit; z0 += 8) {
+#pragma unroll
+            for (int b = 0; b < 8; ++b) f = fminf(f, s_join[min(z0 + b, ksplit - 1) * BM + tid]);
+          }
+          s_fac[tid] = f;
+        }
+        __syncthreads();
+        for (int i = tid; i < ksplit * BM; i += Cfg::THREADS) s_join[i] = s_fac[i % BM] * inv_factor(s_join[i]);
+        __syncthreads();
+      };
+      if constexpr (STREAM) {
+        const int ev = __syncthreads_or(rescaled);
+        if (ev && tid < BM && m0 + tid < M) store_coherent(facs + static_cast<size_t>(z) * M + tid, s_fac[tid]);
+        const uint32_t total = arrive_add_coherent(counters + tile * kCounterStride,
+                                                   1u + (ev ? (1u << (kSpecShift + z)) : 0u));
+        if ((total & ((1u << kSpecShift) - 1u)) != static_cast<uint32_t>(ksplit)) return;
+        rejoin = total >> kSpecShift;
+      } else if constexpr (SPEC) {
         const uint32_t total = arrive_add_coherent(counters + tile * kCounterStride,
                                                    1u + (over ? (1u << (kSpecShift + z)) : 0u));
         if ((total & ((1u << kSpecShift) - 1u)) != static_cast<uint32_t>(ksplit)) return;
@@ -1374,6 +1400,18 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
 #pragma unroll
             for (int s = 0; s < SLOTS; ++s)
               v[b][s] = z0 + b < ksplit ? load_coherent4(slices, slot_off(z0 + b, s)) : float4v{0.f, 0.f, 0.f, 0.f};
+          if constexpr (STREAM) {
+            if (__builtin_expect(rejoin != 0u, 0)) {
+              if (z0 == 0) join_factors();  // their loads go along with the first slices'
+#pragma unroll
+              for (int b = 0; b < ZB; ++b)
+#pragma unroll
+                for (int s = 0; s < SLOTS; ++s)
+                  if (z0 + b < ksplit)
+                    v[b][s] *= *reinterpret_cast<const float4v*>(
+                        &s_join[(z0 + b) * BM + wm0 + 32 * (s / QV / TN) + 8 * (s % QV) + 4 * fk]);
+            }
+          }
 #pragma unroll
           for (int b = 0; b < ZB; ++b)
 #pragma unroll
@@ -1464,15 +1502,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
       for (int q = 0; q < 4; ++q) {
         const int grow = m0 + wm0 + 32 * ri + (lane >> 3) + 8 * q;
         if constexpr (DIRECT) {
-          if constexpr (SPLITK) {
-            // 1, but not a constant to the compiler: the other routes' scale, bias and fp16 cast are one
-            // fused instruction with one rounding, and without a multiply it would add, then cast
-            float one = 1.f;
-            asm volatile("" : "+v"(one));
-            erow[ri][q] = one;
-          } else {
-            erow[ri][q] = inv_factor(s_fac[grow - m0]);
-          }
+          erow[ri][q] = inv_factor(s_fac[grow - m0]);
         } else if constexpr (RAW) {
           erow[ri][q] = (inf_rows >> (4 * ri + q)) & 1u ? __uint_as_float(0x7fc00000u) : 1.f;
         } else {
@@ -1876,6 +1906,8 @@ bool raw_route(const Plan& p, int K, int ksplit) { return p.tile == Tile::T256 &
 // -> 18.2, 333 x 4096^2 (64x128) 37.5 -> 39.7.
 bool stream_route(const Plan& p, int M, int K, const KSplit& ks) {
   if (K <= 0) return false;
+  // split: a bit per slice in the counters, and the slices' row factors fit where the cast would be
+  if (ks.ksplit > kSpecMaxSplit || (ks.ksplit > 1 && 4L * ks.ksplit * p.ntn > 2L * K)) return false;
   if (p.tile == Tile::T32) return true;
   if (p.tile != Tile::T64 && p.tile != Tile::T64x64) return false;
   return M <= 64 || K > 4096 || (ks.kchunk <= 1024 && (ks.ksplit > 1 || M >= 512 || K <= 768));
@@ -2204,12 +2236,13 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
   if (x_is_f32 && g16::direct_thresh(texp) && g16_mm_t_direct_route(M, N, K, num_cus) == 1)
     return g16_mm_t_direct(static_cast<const float*>(x), w_t, 0, out, out_is_f16, bias, thresh, M, N, K, num_cus, stream);
   if (x_is_f32 && g16::direct_thresh(texp)) {
-    // one launch: the tiles stream x and cast it themselves (the scratch stays unused)
+    // one launch: the tiles stream x and cast it themselves
     const int ks = g16_hgemm_plan(M, N, K, num_cus);
     if (g16::stream_route(g16::choose_tile(M, N, K, num_cus), M, K, g16::ksplit_for(K, ks))) {
       if (!g16::aligned16(x)) return G16_E_ALIGN;
       const g16::ResidentCast rc{x, 1, texp};
-      return g16::gemm_launch(nullptr, w_t, out, out_is_f16 != 0, bias, nullptr, M, N, K, ks, num_cus, workspace,
+      auto* facs = static_cast<float*>(scratch);  // the slices' row factors, where the cast would be
+      return g16::gemm_launch(nullptr, w_t, out, out_is_f16 != 0, bias, facs, M, N, K, ks, num_cus, workspace,
                               workspace_bytes, counters, counter_bytes, stream, false, false, &rc, nullptr, true);
     }
   }

@@ -185,3 +185,31 @@ def test_gemm_call_takes_any_threshold(cuda, thresh):
     ref = x.double() @ w.double()
     err = (out.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)
     assert (err <= 2.0 ** -10).all(), err.max()  # fp16 rounding of the activations: 2^-11 per value
+
+
+# splits of 2 to 8 slices on each tile of the route
+@pytest.mark.parametrize("M,K,N,tile,ks", [r for r in ROUTES if r[4] > 1])
+def test_slices_past_fp32_range_cancel(cuda, M, K, N, tile, ks):
+    # partial sums near 1e40 in the first and the last slice cancel; what is left is finite, as it is
+    # where one pass over the row scales it (sums in scaled units until the epilogue)
+    import gtx16_fp16 as g
+
+    x = randn((M, K), seed=M + K)
+    w = randn((K, N), seed=1, scale=0.02, dtype=torch.float16)
+    x[:, :40] = x[:, K - 40:] = 0.0  # (the other rows do not meet the weights of 1)
+    rows = [0, M // 2, M - 1]
+    for i, r in enumerate(rows):
+        x[r] = 0.0
+        x[r, :40], x[r, K - 40:] = 3e38, -3e38
+        x[r, K // 2] = (-2.0) ** (127 - i)
+    w[:40] = w[K - 40:] = 1.0
+    for odt in (torch.float32, torch.float16):
+        y = g.mm_t(x.to(cuda), w.to(cuda), None, odt)
+        torch.cuda.synchronize()
+        ref = x.double() @ w.double()
+        if odt == torch.float16:
+            assert not torch.isnan(y[rows]).any()  # (past fp16's range)
+            y, ref = (torch.stack([t[r] for r in range(M) if r not in rows]) for t in (y, ref))
+        err = (y.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)
+        # fp16 rounding of the activations (and of an fp16 output): 2^-11 per value each
+        assert (err <= 2.0 ** -10).all(), err.max()
