@@ -249,6 +249,17 @@ constexpr int kSpecMaxSplit = 32 - kSpecShift;
 // compiler from moving LDS accesses across it.
 __device__ inline void phase_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
+// Largest |x| of m and 4 values, a NaN among them kept: the cast of direct A takes it over several rows
+// of a lane at once, and v_max_f32 and v_max3_f32, which drop a quiet NaN, lose the maximum itself to a
+// signaling one in any operand (measured), and with it another row's value past fp16's range.
+// v_maximum3_f32 costs the same. past_half() is true for a NaN too: the step's rows are then
+// looked at one by one.
+__device__ inline float absmax4(float m, float4v v) {
+  m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(v.x)), fabsf(v.y));
+  return __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, fabsf(v.z)), fabsf(v.w));
+}
+__device__ inline bool past_half(float m) { return !(m <= kHalfMax); }
+
 // RESIDENT: A is unused; the kernel casts X (fp32 when x_f32, else fp16; threshold 2^texp) itself
 // into resident LDS stages (the 32x128 tile, unsplit, K <= kResidentSteps * BK).
 // SPEC: A is the fp16 activations, streamed as they are; tbits is the largest fp16 bit pattern
@@ -745,10 +756,6 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
           v[h][1] = p[1];
         }
       };
-      auto absmax4 = [](float m, float4v x) __attribute__((always_inline)) {
-        m = fmaxf(fmaxf(m, fabsf(x.x)), fabsf(x.y));
-        return fmaxf(fmaxf(m, fabsf(x.z)), fabsf(x.w));
-      };
       auto cast_x = [&](int s) __attribute__((always_inline)) {
         if (__builtin_expect(__builtin_amdgcn_readfirstlane(scaled), 0)) {
 #pragma unroll
@@ -760,7 +767,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
         float m = 0.f;
 #pragma unroll
         for (int h = 0; h < H; ++h) m = absmax4(absmax4(m, v[h][0]), v[h][1]);
-        if (__builtin_expect(__any(m > kHalfMax), 0)) {
+        if (__builtin_expect(__any(past_half(m)), 0)) {
 #pragma unroll
           for (int h = 0; h < H; ++h) {
             const int r = crow + 8 * h;
@@ -941,10 +948,6 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
 #pragma unroll
           for (int l = 0; l < NL; ++l) xs[decltype(hc)::value][l] = load_op(s, l);
         };
-        auto absmax4 = [](float m, float4v v) __attribute__((always_inline)) {
-          m = fmaxf(fmaxf(m, fabsf(v.x)), fabsf(v.y));
-          return fmaxf(fmaxf(m, fabsf(v.z)), fabsf(v.w));
-        };
         auto write_op = [&](int st, int l, float4v v) __attribute__((always_inline)) {
           *reinterpret_cast<half4*>(wbase + st * Cfg::A_BYTES + l * 8 * (BK * 2)) = __builtin_convertvector(v, half4);
         };
@@ -1000,9 +1003,9 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
           s_evt[st][wave] = s;
           scaled = 1;
         };
-        // largest |x| of a load so far; asm, so that it stays in front of the register's next load
+        // absmax4 in asm, so that it stays in front of the register's next load
         auto absmax_asm = [](float& m, float4v v) __attribute__((always_inline)) {
-          asm volatile("v_max3_f32 %0, %0, |%1|, |%2|\n\tv_max3_f32 %0, %0, |%3|, |%4|"
+          asm volatile("v_maximum3_f32 %0, %0, |%1|, |%2|\n\tv_maximum3_f32 %0, %0, |%3|, |%4|"
                        : "+v"(m)
                        : "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w));
         };
@@ -1015,7 +1018,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
             m = absmax4(m, xs[H][l]);
             write_op(s % NSTAGE, l, xs[H][l]);
           }
-          if (__any(m > kHalfMax)) raise(s);
+          if (__any(past_half(m))) raise(s);
         };
         // B's DMA, in step order. Packed: the step's 16 KB block is a scalar offset (steps past K fetch the
         // last block again), the range ends with the last block, and the two instructions differ by 1 KB in memory as in LDS, which the
@@ -1102,8 +1105,8 @@ __global__ __launch_bounds__(Cfg::THREADS) void hgemm_kernel(const _Float16* __r
           __builtin_amdgcn_sched_barrier(0);
           phase_barrier();
           __builtin_amdgcn_sched_barrier(0);
-          if (__builtin_expect(__any((m > kHalfMax) | (evt == j)), 0)) {
-            if (__any(m > kHalfMax)) raise(j + D);
+          if (__builtin_expect(__any(past_half(m) | (evt == j)), 0)) {
+            if (__any(past_half(m))) raise(j + D);
             // rows whose exponent was raised at this step: their sums so far follow
             if (__any(evt == j)) {
               const float* const del = &s_delta[st][wm0 + 4 * (lane_id() >> 4)];

@@ -118,3 +118,32 @@ def test_direct_replays_in_a_graph(cuda):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager) and torch.equal(g.mm_t(x, w), eager)
+
+
+# the 256x256 tile and, in their own loop, the 4-wavefront ones
+@pytest.mark.parametrize("M,K,N", [(24600, 96, 520), (49153, 8, 256), (128, 1024, 1024), (1024, 264, 1024), (128, 6144, 8192)])
+@pytest.mark.parametrize("pos", range(4))
+def test_signaling_nan_beside_a_row_past_fp16_range(cuda, M, K, N, pos):
+    # rows 8 apart share a lane of the cast: a signaling NaN in one of them, at any place of its 4 values,
+    # leaves the others' exponents alone (a CPU copy keeps its bits)
+    import gtx16_fp16 as g
+
+    x = randn((M, K), seed=pos)
+    base = (K // 8 // 2) * 8  # a chunk of 4 values past the first K steps
+    huge, nan = [], []
+    for blk in range(4):  # rows 32 blk + {0, 8, 16, 24}: one NaN row after, between and before huge ones
+        rows = [32 * blk + 1 + 8 * i for i in range(4)]
+        for i, r in enumerate(rows):
+            if i == blk:
+                x[r].view(torch.int32)[base + pos] = 0x7F800001 + 0x1000 * pos
+                nan.append(r)
+            else:
+                x[r, base + (pos + i) % 4] = 1e5 * (i + 1)
+                huge.append(r)
+    assert torch.isnan(x[nan]).any(1).all()
+    w = randn((K, N), seed=1, scale=0.02, dtype=torch.float16)
+    y = g.mm_t(x.to(cuda), w.to(cuda)).cpu()
+    assert torch.isnan(y[nan]).all()
+    ref = x[huge].double() @ w.double()
+    err = (y[huge].double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert (err <= 2.0 ** -10).all(), err  # fp16 rounding of the activations: 2^-11 per value
