@@ -213,3 +213,25 @@ def test_slices_past_fp32_range_cancel(cuda, M, K, N, tile, ks):
         err = (y.cpu().double() - ref).norm(dim=1) / ref.norm(dim=1)
         # fp16 rounding of the activations (and of an fp16 output): 2^-11 per value each
         assert (err <= 2.0 ** -10).all(), err.max()
+
+
+# (M, K, N, slices, streamed): above 64 rows and past K = 4096 only 3 slices and more are streamed
+@pytest.mark.parametrize("M,K,N,ks,streamed", [
+    (333, 4104, 4096, 1, False), (700, 4352, 1024, 1, False), (128, 6144, 4096, 2, False), (160, 11008, 1536, 3, True),
+    (142, 8192, 1856, 5, True), (333, 4096, 4096, 1, False), (64, 4096, 11008, 2, True), (1024, 1024, 1024, 1, True)])
+def test_route_by_its_rounding(cuda, M, K, N, ks, streamed):
+    # a row with |max| 2000 is halved by the rowscale cast, and 3 * 2^-24 with it (to 2 * 2^-24, a tie to
+    # even); the streamed tiles scale only rows that leave fp16's range
+    import gtx16_fp16 as g
+    from gtx16_fp16 import _clib
+
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    if cus != 256:
+        pytest.skip(f"the route table is for 256 CUs (this device has {cus})")
+    assert _clib.load().g16_hgemm_plan(M, N, K, cus) == ks
+    x = torch.zeros(M, K)
+    x[M - 1, 0], x[M - 1, K - 1] = 2000.0, 3 * 2.0 ** -24
+    w = torch.zeros(K, N, dtype=torch.float16)
+    w[K - 1] = 1.0
+    y = g.mm_t(x.to(cuda), w.to(cuda)).cpu()
+    assert (y[M - 1] == (3 if streamed else 4) * 2.0 ** -24).all() and not y[:-1].any()
