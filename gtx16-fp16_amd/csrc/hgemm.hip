@@ -78,9 +78,13 @@ namespace g16 {
 namespace {
 
 constexpr int kGroupM = 8;
-// Direct A runs few tile columns (direct_route): with 8 tile rows to a group, a group of 3 columns is
-// not a divisor of an XCD's 32 workgroups, and rows of x are read again in the next round (65536 x
-// 3072 x 768: 377 us; 339 with 1 or 2 rows to a group, 348 with 4; packed A within 2 % either way).
+// Direct A runs few tile columns on 256x256 tiles (direct_route): with 8 tile rows to a group, a group of
+// 3 columns is not a divisor of an XCD's 32 workgroups, and rows of x are read again in the next round
+// (65536 x 3072 x 768: 377 us; 339 with 1 or 2 rows to a group, 348 with 4; packed A within 2 % either
+// way). On the 4-wavefront tiles it hardly matters unsplit (within 3 %), and the split grids of few
+// columns that run there gain more often than they lose: 250 x 6144 x 512 13.8 us, 16.1 with 8 rows, 188 x
+// 6784 x 2176 26.9, 29.9, 456 x 2000 x 392 11.4, 12.6, but 1079 x 8704 x 384 33.2, 28.6 and 80 x 6144 x
+// 2048 18.4, 17.3.
 constexpr int kDirectGroupM = 2;
 constexpr int kSplitAlign = 64;  // split-K slices start on a multiple of every tile's K step
 // The planner's rule (M <= 64) splits no K below this: two slices of 256 cost more than they save
@@ -1870,19 +1874,36 @@ bool resident_route(const Plan& p, int ksplit, int K) {
 // fp32 activations run as one direct launch (cast in registers on the way into the GEMM's A stages)
 // where the plan is the unsplit 256x256 tile, at most 4 tile columns read each row, the grid fills
 // three quarters of the CUs, and a tile row of x stays within a descriptor's range. It saves the cast
-// pass over x (6 bytes per value at ~6 TB/s), and costs the GEMM 32 KB of fp32 A per K step and CU
-// instead of 16 KB, and the cast's instructions, once per tile column. Event-timed on one box, cast +
-// packed GEMM -> direct (us, M x K x N, prepacked weight): 65536 x 768 x 768 134 -> 99, 65536 x 3072 x
-// 768 456 -> 349, 65536 x 256 x 256 52 -> 28, 65536 x 768 x 1024 158 -> 128, 16384 x 4096 x 1024 178 ->
-// 141; with more columns the gain ends: 65536 x 768 x 2048 261 -> 246, 65536 x 768 x 3072 364 -> 376,
-// 4096^3 117 -> 140. With 1 % of the rows past fp16's range: 65536 x 768 x 768 135 -> 113, 20000 x 768
-// x 768 47 -> 42, 20000 x 768 x 1280 (not taken) 73 -> 74; a half-empty grid has nothing to hide the
-// rescaling behind, 11000 x 768 x 768 (129 tiles, not taken) 34 -> 38 (29 without such rows).
+// pass over x (6 bytes per value at ~6 TB/s) and the GEMM's wait for it; it costs the GEMM 32 KB of
+// fp32 A per K step and CU instead of 16 KB, and the cast's instructions, once per tile column. So the
+// gain grows with the rows and the cost with the rounds of tiles: past K = 512, where the K loop is
+// most of the time, a round has to stand for enough rows. Graph-timed, cast + packed GEMM -> direct
+// (us, M x K x N, row-major weight, fp32 out; a prepacked weight and fp16 outputs differ by a few %):
+//   one round      16384 x 1024^2 60 -> 51, 16384 x 4096 x 1024 184 -> 145, 12300 x 768 x 1024 43.4 -> 41.0,
+//                  but 12300 x 2000 x 1024 83.9 -> 86.3
+//   whole rounds   65536 x 256 x 256 53 -> 35, 65536 x 768^2 140 -> 118, 65536 x 3072 x 768 472 -> 354,
+//                  65536 x 768 x 1024 166 -> 152, 65536 x 2000 x 1024 395 -> 338
+//   begun rounds   22000 x 384 x 1024 (2) 49.5 -> 45.1, 24000 x 768 x 1024 (2) 73.5 -> 71.3, 33000 x 2000
+//                  x 768 (2) 172 -> 168, but 20000 x 1024^2 (2) 80.0 -> 79.5, 22000 x 2000 x 1024 (2) 144
+//                  -> 162, 33000 x 2000 x 1024 (3) 220 -> 233, 50000 x 2000 x 904 (4) 342 -> 368
+//   ragged columns 65536 x 768 x 904 (4) 200 -> 209 where 648 is 170 -> 155 and 1024 169 -> 159: with four
+//                  columns and more than three rounds, rows of C that end inside a cache line weigh on
+//                  the epilogues of so few K steps (65536 x 384 x 904 156 -> 138, 65536 x 1536 x 904 327
+//                  -> 290 gain again, 40000 x 768 x 1000 in 3 rounds 148 -> 145)
+// More columns end the gain: 65536 x 768 x 2048 261 -> 246, 65536 x 768 x 3072 364 -> 376, 4096^3 117 ->
+// 140. With 1 % of the rows past fp16's range: 65536 x 768^2 135 -> 113, 20000 x 768^2 47 -> 42; a
+// half-empty grid has nothing to hide the rescaling behind, 11000 x 768^2 (129 tiles, not taken) 34 ->
+// 38 (29 without such rows).
 constexpr int kDirectMaxK = 1 << 20;
 constexpr int kDirectMaxN = 1024;
 bool direct_route(const Plan& p, int N, int K, int ksplit, int num_cus) {
-  return p.tile == Tile::T256 && ksplit == 1 && K > 0 && K <= kDirectMaxK && N <= kDirectMaxN &&
-         4L * p.ntm * p.ntn >= 3L * num_cus;
+  if (p.tile != Tile::T256 || ksplit != 1 || K <= 0 || K > kDirectMaxK || N > kDirectMaxN) return false;
+  const long tiles = static_cast<long>(p.ntm) * p.ntn, cus = num_cus;
+  if (4 * tiles < 3 * cus) return false;
+  if (K <= 512) return true;
+  const long rounds = (tiles + cus - 1) / cus, rows = 256L * p.ntm;  // 11008 or 14336 rows a round on 256 CUs
+  if (rows < (K <= 1024 ? 43 : 56) * cus * rounds) return false;
+  return !(K <= 1024 && N > 768 && N % 64 != 0 && rounds > 3);
 }
 // Thresholds the direct launches take: up to 2^15, so that every value of a row within the threshold
 // has a finite cast (they rescale only rows that leave fp16's range), and from 2^2, so that a row's

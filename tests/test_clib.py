@@ -273,6 +273,14 @@ def test_direct_route_rule_and_refusals(lib):
     assert r(65536, 3072, 768, 256) == 0 and r(4096, 4096, 4096, 256) == 0 and r(11000, 768, 768, 256) == 0
     assert r(64, 1024, 1024, 256) == 0 and r(0, 768, 768, 256) == 0 and r(65536, 768, 768, 0) == 0
     assert r(65536, 256, (1 << 20) + 8, 256) == 0 and r(65536, 256, 1 << 20, 256) == 1
+    # past K = 512 a round of tiles has to stand for 11008 rows, past K = 1024 for 14336 (256 CUs); short
+    # rows of C that end inside a cache line stay out past three rounds of four columns
+    for M, N, K, want in [(22000, 1024, 512, 1), (22000, 1024, 520, 1), (21760, 1024, 520, 0), (20000, 1024, 1024, 0),
+                          (22016, 1024, 1032, 0), (33000, 768, 2000, 1), (33000, 1024, 2000, 0), (22000, 1024, 2000, 0),
+                          (12300, 1024, 768, 1), (12300, 1024, 2000, 0), (16384, 1024, 4096, 1), (65536, 1024, 2000, 1),
+                          (50000, 904, 2000, 0), (65536, 904, 768, 0), (65536, 904, 512, 1), (65536, 904, 1032, 1),
+                          (65536, 768, 768, 1), (65536, 1024, 768, 1), (65536, 1016, 1024, 0), (49152, 1000, 768, 1)]:
+        assert r(M, N, K, 256) == want, (M, N, K)
     d = lib.g16_mm_t_direct
     assert d(A, A, 0, A, 0, None, 1024.0, 4096, 4096, 4096, 256, None) == -1
     assert d(A, A, 0, A, 0, None, 65536.0, 65536, 768, 768, 256, None) == -1    # threshold past 2^15
