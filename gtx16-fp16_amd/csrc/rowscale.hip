@@ -13,6 +13,8 @@
 // packed_offset in g16_common.hpp): every 256-row x 32-column block of y is one contiguous 16 KB
 // run, already in the order (and LDS swizzle) the GEMM's DMA writes into LDS, so that DMA reads
 // whole 1 KB runs instead of 64-byte pieces of 256 different rows.
+#include <algorithm>
+
 #include "rowscale_math.hpp"
 
 namespace g16 {
@@ -182,6 +184,21 @@ int rowscale_launch(const void* X, void* Y, float* S, int M, int K, float thresh
   if (!aligned16(X) || !aligned16(Y)) return G16_E_ALIGN;
   const int texp = thresh_exponent(thresh);
   if (texp == -1000) return G16_E_SHAPE;
+  // A launch holds less than 2^32 threads (past that its grid wraps): 2^23 rows, whole packed blocks, at a
+  // time.
+  constexpr int kMaxRows = 1 << 23;
+  if (M > kMaxRows) {
+    for (int r0 = 0; r0 < M;) {
+      const int n = std::min(kMaxRows, M - r0);
+      const size_t at = PACK ? static_cast<size_t>(r0 / kPackRows) * packed_ksteps(K) * (kPackRows * kPackK)
+                             : static_cast<size_t>(r0) * K;
+      const int st = rowscale_launch<TX, CH, PACK>(static_cast<const TX*>(X) + static_cast<size_t>(r0) * K,
+                                                   static_cast<_Float16*>(Y) + at, S + r0, n, K, thresh, stream);
+      if (st != G16_OK) return st;
+      r0 += n;
+    }
+    return G16_OK;
+  }
   constexpr int EPC = 16 / static_cast<int>(sizeof(TX));
   const int rows = PACK ? ceil_div(M, kPackRows) * kPackRows : M;
   // A workgroup per row: past K = 4096, where a wavefront would read its row twice, and for so few

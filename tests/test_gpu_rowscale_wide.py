@@ -48,3 +48,58 @@ def test_rowscale_wide_bitexact(cuda, M, K, dt):
     assert np.array_equal(np.isnan(gp), pn) and np.array_equal(gp.view(np.uint16)[~pn], pw.view(np.uint16)[~pn])
     for t in (s, sp):
         assert np.array_equal(t.cpu().numpy().view(np.uint32), S.astype(np.float32).view(np.uint32))
+
+
+def test_rowscale_of_more_rows_than_one_launch_holds(cuda):
+    # 2^24 + 3 rows of 4104 fp16 values (138 GB, cast onto themselves: each value is read before it is
+    # written): a workgroup of 256 threads per row is past the 2^32 threads of a launch
+    from gtx16_fp16 import _clib
+
+    M, K = (1 << 24) + 3, 4104
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info(cuda)[0] < 150 * 10 ** 9:
+        pytest.skip("needs 150 GB of free GPU memory")
+    x = torch.zeros(M, K, dtype=torch.float16, device=cuda)
+    s = torch.zeros(M, device=cuda)
+    rows = [0, (1 << 23) - 1, 1 << 23, (1 << 24) - 1, 1 << 24, M - 1]
+    for i, r in enumerate(rows):
+        x[r, K - 1 - i] = 2048.0 * (i + 1)
+    want, S, _ = oracle.rowscale(x[rows].cpu().numpy())
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    assert _clib.load().g16_rowscale_f16(x.data_ptr(), x.data_ptr(), s.data_ptr(), M, K, 1024.0, st) == 0
+    got, gs = x[rows].cpu().numpy(), s[rows].cpu().numpy()
+    ones = int((s == 1.0).sum())
+    del x, s
+    torch.cuda.empty_cache()
+    assert np.array_equal(got.view(np.uint16), want.view(np.uint16)) and np.array_equal(gs, S.astype(np.float32))
+    assert ones == M - len(rows)
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_rowscale_of_short_rows_past_one_launch(cuda, packed):
+    # 2^26 + 5 rows of 8: four rows to a workgroup, past the 2^32 threads as well
+    from gtx16_fp16 import _clib
+
+    lib = _clib.load()
+    M, K = (1 << 26) + 5, 8
+    if torch.cuda.mem_get_info(cuda)[0] < 8 * 10 ** 9:
+        pytest.skip("needs 8 GB of free GPU memory")
+    x = torch.zeros(M, K, dtype=torch.float16, device=cuda)
+    rows = [0, (1 << 23) - 1, 1 << 23, (1 << 26) - 1, 1 << 26, M - 1]
+    for i, r in enumerate(rows):
+        x[r, i] = 2048.0 * (i + 1)
+    want, S, _ = oracle.rowscale(x[rows].cpu().numpy())
+    s = torch.zeros(M, device=cuda)
+    y = torch.full((lib.g16_packed_a_bytes(M, K) // 2 if packed else M * K,), 7.0, dtype=torch.float16, device=cuda)
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    fn = lib.g16_rowscale_pack_f16 if packed else lib.g16_rowscale_f16
+    assert fn(x.data_ptr(), y.data_ptr(), s.data_ptr(), M, K, 1024.0, st) == 0
+    if packed:  # row r's 8 values, one chunk of its 256-row block (a single block of 32 columns wide)
+        blocks = y.view(-1, 16, 64, 8)
+        sw = [(r % 256 >> 1) & 3 for r in rows]
+        got = torch.stack([blocks[r // 256, r % 256 // 16, r % 16 * 4 + w] for r, w in zip(rows, sw)])
+    else:
+        got = y.view(M, K)[rows]
+    assert np.array_equal(got.cpu().numpy().view(np.uint16), want.view(np.uint16))
+    assert np.array_equal(s[rows].cpu().numpy(), S.astype(np.float32))
+    assert int((s == 1.0).sum()) == M - len(rows) and int((y != 0).sum()) == len(rows)
