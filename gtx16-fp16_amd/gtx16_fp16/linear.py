@@ -110,21 +110,28 @@ class FastLinear(nn.Module):
         layer's ``.weight`` (its shape, device or dtype) as they would on nn.Linear."""
         return self.weight_t.t()
 
+    def _operands_ok(self, w: torch.Tensor, b: torch.Tensor | None, dev: torch.device) -> bool:
+        # weight_t and bias as the kernels read them through their pointers (supported()'s checks of the
+        # weight, and an fp32 bias)
+        K, N = self.in_features, self.out_features
+        return (w.dtype == torch.float16 and w.device == dev and w.shape == (K, N) and w.is_contiguous()
+                and K % 8 == 0 and N % 8 == 0 and w.data_ptr() % 16 == 0 and _is_target(dev.index or 0)
+                and (b is None or (b.dtype == torch.float32 and b.device == dev and b.is_contiguous() and b.numel() == N)))
+
     def _decode_entry(self, M: int, dev: torch.device, f32: bool = True):
         key = (M, dev.index, self.prepack_decode, f32)
         w, b = self.weight_t, self.bias
         bptr = None if b is None else b.data_ptr()
         entry = self._skinny.get(key)
-        if entry is None or entry[3] != w.data_ptr() or entry[4] != bptr:
+        # half-precision calls are checked whole every time, as mm_t checks them: the pointers alone do not
+        # show a view or a tensor of another type or shape at the same address
+        if entry is None or entry[3] != w.data_ptr() or entry[4] != bptr or \
+                not (f32 or (entry[0] is not None) == self._operands_ok(w, b, dev)):
             # (re)validated whenever weight_t or bias is a different tensor, e.g. after .to() or
             # .half() (which turns the bias fp16: the kernel reads an fp32 bias)
             K, N = self.in_features, self.out_features
-            ok = (w.dtype == torch.float16 and w.is_contiguous() and w.device == dev and K % 8 == 0
-                  and N % 8 == 0 and w.data_ptr() % 16 == 0 and _is_target(dev.index or 0)
-                  and (b is None or (b.dtype == torch.float32 and b.device == dev and b.is_contiguous()
-                                     and b.numel() == N)))
             pl, ksplit, sizes, pls = None, 0, (0, 0), None
-            if ok:
+            if self._operands_ok(w, b, dev):
                 lib = _clib.load()
                 # the split kernel on weight_t always (also the decode layout's stand-in while its copy
                 # cannot be built: under graph capture)
@@ -187,10 +194,7 @@ class FastLinear(nn.Module):
         # None: not that case (the general path then decides).
         w, b, dev = self.weight_t, self.bias, x.device
         K, N = self.in_features, self.out_features
-        if not (w.dtype == torch.float16 and w.device == dev and w.shape == (K, N) and w.is_contiguous()
-                and K % 8 == 0 and N % 8 == 0 and w.data_ptr() % 16 == 0 and _is_target(dev.index or 0)):
-            return None
-        if b is not None and not (b.dtype == torch.float32 and b.device == dev and b.is_contiguous() and b.numel() == N):
+        if not self._operands_ok(w, b, dev):
             return None
         kind, scratch_bytes, _ks, ws_bytes, cnt_bytes = _gemm_route(_clib.load(), M, N, K, dev)[:5]
         if kind == "packed":
@@ -222,7 +226,7 @@ class FastLinear(nn.Module):
         # Fast path for small batches (generation): minimal Python per call (linear.py:49-64).
         # Unlike the reference, the weight's support is checked (once per layer and M), so a
         # FastLinear built directly with K or N not a multiple of 8 still takes the fallback.
-        if (f32 or dt == _F16) and x.is_cuda and x.is_contiguous() and x.data_ptr() % 16 == 0:
+        if (f32 or dt == _F16) and shape and x.is_cuda and x.is_contiguous() and x.data_ptr() % 16 == 0:
             K, N = self.in_features, self.out_features
             M = x.numel() // K if shape[-1] == K else -1
             if 0 < M <= SKINNY_MAX_M:

@@ -159,3 +159,32 @@ def test_skinny_multiplies_every_bit_of_the_activations(cuda, M, K, N, dt):
     x64, w64 = x.to(cuda).double(), w.to(cuda).double()
     bound = (512 * 2.0 ** -24 * (x64.abs() @ w64.abs())).cpu()
     assert ((y - (x64 @ w64).cpu()).abs() <= bound).all()
+
+
+def test_fast_linear_fp16_sees_other_operands_at_the_same_address(cuda):
+    # a bias or a weight replaced by a view of its memory: another type is used as what it is, another
+    # shape is refused, after calls that had the layer's own tensors
+    import gtx16_fp16 as g
+
+    torch.manual_seed(0)
+    K, N = 1024, 256
+    x = torch.randn(4, K, device=cuda).half()
+    fl = g.FastLinear.from_linear(nn.Linear(K, N).to(cuda))
+    first = fl(x)
+    bias = fl.bias.clone()
+    fl.bias = fl.bias.view(torch.float16)[:N]
+    fl.bias.copy_(torch.arange(N))
+    want = g.mm_t(x, fl.weight_t, fl.bias.float(), torch.float16)
+    assert torch.equal(fl(x), want) and torch.equal(fl(x), want)
+    fl.bias = bias
+    assert torch.equal(fl(x), first)
+    whole = fl.weight_t
+    fl.weight_t = whole[: K // 2]
+    with pytest.raises(RuntimeError):
+        fl(x)
+    fl.weight_t = whole
+    assert torch.equal(fl(x), first)
+    # a scalar is still a batch of one for a layer of one feature
+    one = g.FastLinear(1, 8, bias=False, device=cuda)
+    one.weight_t.fill_(2.0)
+    assert torch.equal(one(torch.tensor(3.0, dtype=torch.float16, device=cuda)), torch.full((8,), 6.0, device=cuda).half())
