@@ -8,9 +8,9 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _clib
+from . import _clib, ops
 from .kernels import SKINNY_MAX_M, PreparedCall, scratch_buffer, split_buffers, stream_handle
-from .ops import (ROW_SCALE_THRESHOLD, STRIPS_MAX_M, _gemm_route, _is_target, _sm_count, is_affected, mm_t,
+from .ops import (STRIPS_MAX_M, _gemm_route, _is_target, _sm_count, is_affected, mm_t,
                   mm_t_prepacked, pack_decode_weight, pack_weight, prepacked_route, skinny_strips, supported,
                   tensor_version)
 
@@ -204,7 +204,7 @@ class FastLinear(nn.Module):
         scratch = scratch_buffer(dev, stream, scratch_bytes) if scratch_bytes else None
         bufs = split_buffers(dev, stream, ws_bytes, cnt_bytes) if kind == "splitk" else (None, 0, None, 0)
         _clib.check(_clib.fast().mm_t_gemm(x.data_ptr(), True, w.data_ptr(), out.data_ptr(), False,
-                                           None if b is None else b.data_ptr(), ROW_SCALE_THRESHOLD, M, N, K,
+                                           None if b is None else b.data_ptr(), ops.ROW_SCALE_THRESHOLD, M, N, K,
                                            _sm_count(dev), None if scratch is None else scratch.data_ptr(),
                                            scratch_bytes, *bufs, stream), "GEMM")
         return out

@@ -213,7 +213,7 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
             _spec_history.add(dev.index)
     kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct, raw = _gemm_route(lib, M, N, K, dev)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
-    if direct if x2d.dtype == torch.float32 else raw:
+    if (direct and _direct_thresh()) if x2d.dtype == torch.float32 else raw:
         _direct(lib, x2d, w_t, 0, out, bptr, M, N, K, dev, stream)
         return out
     # no scratch where the GEMM casts its own rows into LDS (one launch, the unsplit small tile)
@@ -224,6 +224,11 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
                                   M, N, K, _sm_count(dev), None if scratch is None else scratch.data_ptr(),
                                   scratch_bytes, *bufs, stream), "GEMM")
     return out
+
+
+def _direct_thresh() -> bool:
+    # the thresholds g16_mm_t_direct takes; the two launches take any power of two
+    return 4.0 <= ROW_SCALE_THRESHOLD <= 32768.0
 
 
 def _direct(lib, x2d: torch.Tensor, w: torch.Tensor, packed: int, out: torch.Tensor, bptr, M: int, N: int, K: int,
@@ -367,7 +372,8 @@ def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias:
     b = None if bias is None else bias.float().contiguous()
     x2d = _aligned(x2d)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
-    if _cast_source is None and _gemm_route(lib, M, N, K, dev)[5 if x2d.dtype == torch.float32 else 6]:
+    direct, raw = _gemm_route(lib, M, N, K, dev)[5:]
+    if _cast_source is None and ((direct and _direct_thresh()) if x2d.dtype == torch.float32 else raw):
         _direct(lib, x2d, wp, 1, out, None if b is None else b.data_ptr(), M, N, K, dev, stream)
         return out
     _scratch, xp, rscale = _packed_cast(lib, x2d, M, K, dev, stream, _cast_source)

@@ -147,3 +147,27 @@ def test_signaling_nan_beside_a_row_past_fp16_range(cuda, M, K, N, pos):
     ref = x[huge].double() @ w.double()
     err = (y[huge].double() - ref).norm(dim=1) / ref.norm(dim=1)
     assert (err <= 2.0 ** -10).all(), err  # fp16 rounding of the activations: 2^-11 per value
+
+
+@pytest.mark.parametrize("thresh", [2.0, 1024.0, 2.0 ** 15])
+def test_a_changed_threshold_reaches_every_route(cuda, monkeypatch, thresh):
+    # ops.ROW_SCALE_THRESHOLD is read by each call: the direct route and the prepacked weight (two launches
+    # for thresholds the direct kernel does not take), the streamed tiles and FastLinear's short path
+    import torch.nn as nn
+
+    import gtx16_fp16 as g
+    from gtx16_fp16 import ops
+
+    monkeypatch.setattr(ops, "ROW_SCALE_THRESHOLD", thresh)
+    for M, K, N in ((24600, 96, 520), (64, 1024, 1024)):
+        fl = g.FastLinear.from_linear(nn.Linear(K, N, bias=False).to(cuda))
+        # 3 * 2^-24 rounds to 4 * 2^-24 wherever its row, whose largest value is 3, is halved (threshold 2,
+        # two launches) and is itself elsewhere
+        x = torch.zeros(M, K, device=cuda)
+        x[M - 1, 0], x[M - 1, K - 1] = 3.0, 3 * 2.0 ** -24
+        fl.weight_t.zero_()
+        fl.weight_t[K - 1] = 1.0
+        want = (4 if thresh == 2.0 else 3) * 2.0 ** -24
+        outs = [g.mm_t(x, fl.weight_t), fl(x), ops.mm_t_prepacked(x, fl.weight_t, ops.pack_weight(fl.weight_t))]
+        for y in outs:
+            assert (y[M - 1] == want).all() and not y[:-1].any()
