@@ -41,8 +41,11 @@ class FastLinear(nn.Module):
 
     Two more caches are opt-in, because each trades memory or a staleness risk for speed:
 
-    * ``share_cast = True``: large-batch layers called one after another with the same input tensor
-      (a transformer's Q, K and V projections) on one stream reuse the first call's rowscale cast.
+    * ``share_cast = True``: large-batch layers called one after another with the same fp32 input tensor
+      (a transformer's Q, K and V projections) on one stream reuse the first call's rowscale cast. It
+      pays from three layers on (three 768 x 768 layers of 65536 rows: 327 -> 314 us); a layer that
+      shares its input with no other is up to 20 % faster without it, because the GEMM then casts
+      the input itself.
       A cast is reused only while the input is the same live tensor with the same torch version
       counter; writes that bypass torch's counter (a custom kernel writing through ``data_ptr()``,
       ``x.data.copy_()``, a serving stack refilling the buffer in place) are not seen and would

@@ -350,12 +350,14 @@ def _packed_cast(lib, x2d: torch.Tensor, M: int, K: int, dev: torch.device, stre
 def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias: torch.Tensor | None = None,
                    out_dtype: torch.dtype = torch.float32, _cast_source: torch.Tensor | None = None) -> torch.Tensor:
     """mm_t for a weight that also has its prepacked form ``wp = pack_weight(w_t)``: same contract and
-    the same result bits as ``mm_t(x2d, w_t, bias, out_dtype)``. On the large-GEMM route the GEMM
+    (without a ``_cast_source``) the same result bits as ``mm_t(x2d, w_t, bias, out_dtype)``. On the large-GEMM route the GEMM
     reads ``wp`` instead of ``w_t`` (plain 16-byte LDS reads for both operands); elsewhere it is
     exactly mm_t. Check supported(x2d, w_t) first.
 
     ``_cast_source`` (used by FastLinear) names the tensor x2d was taken from: consecutive calls on
-    one stream with the same unmodified source share one rowscale cast of it."""
+    one stream with the same unmodified source share one rowscale cast of it (fp32; fp16 x needs none where
+    mm_t multiplies it as it is). Large fp32 batches into few columns then round as that cast does, rows
+    with |max| > 1024 scaled, where mm_t scales only rows that leave fp16's range."""
     if out_dtype not in (torch.float32, torch.float16):
         raise ValueError(f"out_dtype must be float32 or float16, got {out_dtype}")
     _check_operands(x2d, w_t, bias)
@@ -373,7 +375,11 @@ def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias:
     x2d = _aligned(x2d)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
     direct, raw = _gemm_route(lib, M, N, K, dev)[5:]
-    if _cast_source is None and ((direct and _direct_thresh()) if x2d.dtype == torch.float32 else raw):
+    # One launch that reads x itself; for fp32 x not where layers share a cast of it: three direct launches
+    # take 4 to 9 % longer than a cast and three packed GEMMs (65536 x 768^2 327 us, 314; 16384 x 4096 x 1024
+    # 421, 387), two as long, one 15 % less. Raw ones are no slower shared (8192 x 2048^2 172 us, 180;
+    # 4096^3 307, 309).
+    if (direct and _direct_thresh() and _cast_source is None) if x2d.dtype == torch.float32 else raw:
         _direct(lib, x2d, wp, 1, out, None if b is None else b.data_ptr(), M, N, K, dev, stream)
         return out
     _scratch, xp, rscale = _packed_cast(lib, x2d, M, K, dev, stream, _cast_source)

@@ -298,3 +298,24 @@ def test_no_prepacked_copy_is_built_under_graph_capture(ops, cuda):
         y = fl(x)
     torch.cuda.synchronize()
     assert fl._wp is not None and torch.equal(y, want)
+
+
+def test_shared_cast_leaves_fp16_products_uncast(ops, cuda):
+    # fp16 activations on the 256x256 tile are multiplied as they are with share_cast too: mm_t's bits (a
+    # cast would halve the row with |max| 2000 and round its 3 * 2^-24), and no cast is kept
+    import gtx16_fp16 as g
+
+    K, N = 768, 768
+    layers = _qkv(cuda)
+    x = torch.zeros(65536, K, dtype=torch.float16, device=cuda)
+    x[7, 0], x[7, K - 1] = 2000.0, 3 * 2.0 ** -24
+    x[8:] = torch.randn(1, K, device=cuda)
+    ops.release_cast_cache()
+    for fl in layers:
+        fl.weight_t[0] = 0.0
+        fl.weight_t[K - 1, :8] = 1.0
+        y = fl(x)
+        assert torch.equal(y, g.mm_t(x, fl.weight_t, fl.bias, torch.float16))
+        z = ops.mm_t_prepacked(x, fl.weight_t, ops.pack_weight(fl.weight_t), None, torch.float32, _cast_source=x)
+        assert torch.equal(z, g.mm_t(x, fl.weight_t)) and (z[7, :8] == 3 * 2.0 ** -24).all()
+    assert len(ops._cast_cache) == 0
