@@ -2203,8 +2203,8 @@ extern "C" int g16_mm_t_gemm(const void* x, int x_is_f32, const uint16_t* w_t, v
                              const float* bias, float thresh, int M, int N, int K, int num_cus, void* scratch,
                              size_t scratch_bytes, void* workspace, size_t workspace_bytes, uint32_t* counters,
                              size_t counter_bytes, void* stream) {
-  // mm_t's GEMM path in one call: the same two launches, and the same result bits, as the
-  // separate rowscale and GEMM entry points on the route g16_hgemm_use_packed / g16_hgemm_plan pick
+  // mm_t's GEMM path in one call: one launch on the routes the header lists, else the two launches of
+  // the separate rowscale and GEMM entry points on the route g16_hgemm_use_packed / g16_hgemm_plan pick
   if (M < 0 || N < 0 || K < 0 || K % 8 != 0 || N % 8 != 0 || K > g16::kMaxK || N > g16::kMaxN || num_cus <= 0)
     return G16_E_SHAPE;
   if (M == 0 || N == 0) return G16_OK;

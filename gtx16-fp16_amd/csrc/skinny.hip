@@ -2,7 +2,8 @@
 //
 // Semantics (reference: src/gtx16_fp16/kernels.py:153-219, ops.py:45-51,78-84): fp32 math on the
 // unquantised activations (fp32 or fp16 used as is), fp16 weights widened to fp32, bias added once,
-// fp32 output, or an fp16 one rounded once from it as it is stored.
+// fp32 output, or an fp16 one rounded once from it as it is stored. (One form of M = 8 takes fp32
+// activations as two fp16 parts, within 2^-21 of them: use_mf.)
 //
 // The path is HBM-bound for small M (arithmetic intensity <= 8 flop/byte): B is streamed exactly
 // once and the design follows from B's layout ([K,N], N contiguous):

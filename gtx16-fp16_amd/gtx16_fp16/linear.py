@@ -25,12 +25,14 @@ class FastLinear(nn.Module):
     fp16 (nearest-even); ``bias`` stays fp32. Those two buffers are the whole state_dict.
 
     Which kernel a call reaches depends on its row count M (all leading dimensions flattened):
-    M <= 8 goes to the skinny GEMV, which multiplies the activations exactly as given (fp32 or fp16)
-    in fp32 arithmetic; M > 8 goes to the MFMA GEMM, which first rounds each activation row to fp16
-    after dividing it by a power of two when its largest magnitude exceeds 1024, accumulates in
-    fp32, and multiplies the power of two back in. fp32 and fp16 inputs give outputs of their own
-    dtype; any other input dtype is computed as fp32 and returns fp32. Inputs that need autograd,
-    and shapes the kernels cannot take, are computed by ``F.linear`` instead.
+    M <= 8 goes to the skinny GEMV, which multiplies the activations as given (fp32 or fp16) in fp32
+    arithmetic (some M = 8 shapes on the matrix cores, fp32 activations there to 2^-21); M > 8 goes
+    to the MFMA GEMM, which rounds each activation to fp16 after dividing its row by a power of two
+    when the row's largest magnitude exceeds 1024 (65504, fp16's range, where the GEMM reads the
+    activations itself; large fp16 batches are not rounded at all), accumulates in fp32, and
+    multiplies the power of two back in (mm_t says which shapes). fp32 and fp16 inputs give outputs of
+    their own dtype; any other input dtype is computed as fp32 and returns fp32. Inputs that need
+    autograd, and shapes the kernels cannot take, are computed by ``F.linear`` instead.
 
     On the tile-packed GEMM route (large M) the layer also builds, on first use, a copy of its
     weight in the GEMM's packed layout and keeps it outside the state_dict; it is rebuilt whenever

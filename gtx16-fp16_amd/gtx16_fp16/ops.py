@@ -165,12 +165,14 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     """out[M,N] = x2d[M,K] @ w_t[K,N] + bias[N]  (ops.py:65-108).
 
     x2d fp16 or fp32; w_t fp16; bias fp32 (or None); out fp32 or fp16. Check supported() first.
-    M <= 8: fp32 math on the unquantised x (skinny path). M > 8: rows with |max| > 1024 are scaled
-    by a power of two, cast to fp16, multiplied on the matrix cores with fp32 accumulation and
-    scaled back; shapes with too few output tiles split K with a deterministic reduction. (Large fp32
-    batches into at most 1024 columns scale only the rows that leave fp16's range, 65504: the GEMM
-    casts x itself, and every value is rounded at least as finely. Large fp16 batches are multiplied
-    as they are: nothing is rounded.)"""
+    M <= 8: fp32 math on the unquantised x (skinny path); only at M = 8, N <= 8192 and 32 to 128 rows
+    of K per wavefront is an fp32 x multiplied as two fp16 parts, which keep it to 2^-21. M > 8: rows
+    with |max| > 1024 are scaled by a power of two, cast to fp16, multiplied on the matrix cores with
+    fp32 accumulation and scaled back; shapes with too few output tiles split K with a deterministic
+    reduction. Where one launch reads x itself, values are rounded at least as finely: large fp32
+    batches into at most 1024 columns, and fp32 batches on the small tiles (9 to 64 rows, and more
+    where it is the faster form), scale only rows that leave fp16's range, 65504; large fp16 batches
+    (256x256 tiles) are multiplied as they are and nothing is rounded."""
     if out_dtype not in (torch.float32, torch.float16):
         raise ValueError(f"out_dtype must be float32 or float16, got {out_dtype}")
     _check_operands(x2d, w_t, bias)
@@ -202,9 +204,10 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     # GEMM path: fp16 inputs, with per-row power-of-two scaling for rows that would overflow. One
     # library call runs the rowscale cast into `scratch` and the GEMM on the planned route: the
     # tile-packed 256-row tiles for large outputs, split-K where the tiles leave CUs idle, else the
-    # plain tiles (the cast, scales and GEMM of ops.py:86-108); on the unsplit 32x128 tile with
-    # K <= 1280 the GEMM casts fp32 rows into LDS, and fp16 x on the 32-, 64- and 128-row tiles is
-    # streamed as it is (a row within the threshold is its own cast): one launch in both cases.
+    # plain tiles (the cast, scales and GEMM of ops.py:86-108). One launch instead where the GEMM casts
+    # fp32 rows itself (into LDS at once on the unsplit 32x128 tile with K <= 1280, step by step on the
+    # other small tiles) or streams fp16 x as it is (32-, 64- and 128-row tiles: a row within the
+    # threshold is its own cast).
     # The speculation history lets a weight whose fp16 call needed a tile computed again take the
     # two-launch route for a while; it is enabled once per device (a small pinned allocation,
     # retried on a later call if this one is being captured into a graph).
@@ -350,8 +353,8 @@ def _packed_cast(lib, x2d: torch.Tensor, M: int, K: int, dev: torch.device, stre
 def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias: torch.Tensor | None = None,
                    out_dtype: torch.dtype = torch.float32, _cast_source: torch.Tensor | None = None) -> torch.Tensor:
     """mm_t for a weight that also has its prepacked form ``wp = pack_weight(w_t)``: same contract and
-    (without a ``_cast_source``) the same result bits as ``mm_t(x2d, w_t, bias, out_dtype)``. On the large-GEMM route the GEMM
-    reads ``wp`` instead of ``w_t`` (plain 16-byte LDS reads for both operands); elsewhere it is
+    (without a ``_cast_source``) the same result bits as ``mm_t(x2d, w_t, bias, out_dtype)``. On the
+    large-GEMM route the GEMM reads ``wp`` instead of ``w_t`` (plain 16-byte LDS reads for both operands); elsewhere it is
     exactly mm_t. Check supported(x2d, w_t) first.
 
     ``_cast_source`` (used by FastLinear) names the tensor x2d was taken from: consecutive calls on

@@ -120,27 +120,38 @@ int g16_hgemm_packed_f16out(const uint16_t* Ap, const uint16_t* B, uint16_t* C, 
 int g16_hgemm_use_packed(int M, int N, int K, int num_cus);
 
 /* ---------------------------------------------------------------------------------------------
- * mm_t's GEMM path (src/gtx16_fp16/ops.py:86-108) in one call: the rowscale cast of x (fp32 when
- * x_is_f32, else fp16) into `scratch`, then the GEMM on the route this library plans for num_cus
- * compute units -- the tile-packed route where g16_hgemm_use_packed() is 1, else split-K with
- * ksplit = g16_hgemm_plan() when that is > 1, else the plain GEMM. The same result bits as the
- * separate entry points (rowscale, then GEMM); one call instead of two on a path whose small
- * shapes are bound by host and launch time. No counterpart kernel in the reference.
- *   One launch for fp16 x where the plan is a 4-wavefront tile (32x128, 64x128, 64x64 or
- *   128x128, split or not) and thresh >= 2^-8: the GEMM streams x itself as A, since a row within
- *   the threshold is its own cast, and computes a tile again, with A rescaled in registers by the
- *   rows' exponents, only where some |x| of it exceeds the threshold or is NaN (split tiles: the
- *   last slice to arrive recomputes every slice). Same result bits; no scratch is used. A weight whose call had
- *   a tile computed again takes the other route below for its next 63 calls when the scratch the
- *   caller passed allows it (a per-device history in pinned host memory, keyed by w_t, once
- *   g16_mm_t_spec_history has enabled it).
- *   One launch for fp32 x where the plan is the unsplit 32x128 tile and K <= 1280: the GEMM's
- *   workgroups cast their own rows of x into LDS (the rowscale arithmetic, the same bits) and no
- *   rowscale launch runs; g16_mm_t_scratch_bytes() is then 0 and scratch may be NULL (x must be
- *   16-byte aligned). Elsewhere the call makes the two launches.
+ * mm_t's GEMM path (src/gtx16_fp16/ops.py:86-108) in one call; one call instead of two on a path
+ * whose small shapes are bound by host and launch time. No counterpart kernel in the reference.
+ *   In general it is two launches: the rowscale cast of x (fp32 when x_is_f32, else fp16) into
+ *   `scratch`, then the GEMM on the route this library plans for num_cus compute units -- the
+ *   tile-packed route where g16_hgemm_use_packed() is 1, else split-K with ksplit =
+ *   g16_hgemm_plan() when that is > 1, else the plain GEMM -- with the result bits of those entry
+ *   points. Where a plan allows it, it is one launch; (a) and (b) give the same bits, (c) to (e) round
+ *   each value of x at least as finely and so give the same bits unless a value that the cast scales
+ *   falls below fp16's normal range in it:
+ *   (a) fp16 x where the plan is a 4-wavefront tile (32x128, 64x128, 64x64 or 128x128, split or not)
+ *   and thresh >= 2^-8: the GEMM streams x itself as A, since a row within the threshold is its own
+ *   cast, and computes a tile again, with A rescaled in registers by the rows' exponents, only where
+ *   some |x| of it exceeds the threshold or is NaN (split tiles: the last slice to arrive recomputes
+ *   every slice). No scratch is used. A weight whose call had a tile computed again takes the two
+ *   launches for its next 63 calls when the scratch the caller passed allows it (a per-device history
+ *   in pinned host memory, keyed by w_t, once g16_mm_t_spec_history has enabled it).
+ *   (b) fp32 x where the plan is the unsplit 32x128 tile and K <= 1280: the GEMM's workgroups cast
+ *   their own rows of x into LDS (the rowscale arithmetic); g16_mm_t_scratch_bytes() is then 0.
+ *   (c) fp32 x, thresh 4 to 2^15, on the 32x128 tile and, where streaming x is measured to be
+ *   faster than casting it, the 64x128 and 64x64 tiles, split or not: as g16_mm_t_direct, each K
+ *   slice scaling by the part of the row it holds; slices are added in the row's largest scale.
+ *   (d) fp32 x, thresh 4 to 2^15, where g16_mm_t_direct_route() is 1: g16_mm_t_direct.
+ *   (e) fp16 x where g16_mm_t_raw_route() is 1: g16_mm_t_raw (thresh is then not used); and, for
+ *   thresh >= 2^-8, the unsplit 256x128 tiles of one round of medium batches (512 rows and more)
+ *   when `scratch` is NULL, misaligned or too small. With their scratch these take the two
+ *   launches, which are faster: there the rounding of rows past the threshold depends on it.
+ *   fp32 x must be 16-byte aligned, fp16 x as the GEMM entry points need it.
  *   scratch: at least g16_mm_t_scratch_bytes(M, N, K, num_cus) bytes, 16-byte aligned (the fp16
- *   cast and the row scales; it must stay allocated until the GEMM has run). It may be NULL on the
- *   one-launch routes above (fp16 x then always takes the one launch).
+ *   cast and the row scales, or (c)'s scales; it must stay allocated until the GEMM has run). It may
+ *   be NULL in (a), which then always takes the one launch, in (b), and in (e)'s medium batches;
+ *   elsewhere it is asked for even if the one launch does not write it (G16_E_NULL, G16_E_ALIGN,
+ *   G16_E_WORKSPACE).
  *   workspace / counters: as g16_hgemm_splitk needs them for that ksplit (unused otherwise, then
  *   NULL/0 is fine). thresh: as for the rowscale entry points.
  */
@@ -168,8 +179,9 @@ int g16_mm_t_spec_paused(const uint16_t* w_t, void* stream);
  * its packed form (g16_pack_weight). A row whose values all fit fp16 is cast as it is; a row with a
  * larger value is scaled by a power of two from that value on (its sums so far are scaled with it),
  * by the rule of g16_rowscale_f32 for a threshold of 4 to 2^15 (others: G16_E_SHAPE) applied to the
- * part of the row read so far. Each value is so rounded to fp16 at least as finely as g16_rowscale_f32 rounds it; the
- * results are the same bits unless a scaled value falls below fp16's normal range. */
+ * part of the row read so far. Each value is so rounded to fp16 at least as finely as
+ * g16_rowscale_f32 rounds it; the results are the same bits unless a scaled value falls below
+ * fp16's normal range. */
 int g16_mm_t_direct_route(int M, int N, int K, int num_cus);
 int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,
                     const float* bias, float thresh, int M, int N, int K, int num_cus, void* stream);
@@ -231,6 +243,8 @@ int g16_hgemm_tile(int M, int N, int K, int num_cus, int* rows, int* cols);
  * UNQUANTISED activations (fp32 or fp16), fp32 output.
  * Replaces skinny_f32in / skinny_f16in (src/gtx16_fp16/kernels.py:212-219) and its launch
  * configuration skinny_config (src/gtx16_fp16/ops.py:45-51,78-84; src/gtx16_fp16/linear.py:49-64).
+ * fp32 activations at M = 8, N <= 8192 and 32 to 128 K rows per wavefront are multiplied on the matrix
+ * cores as two fp16 parts of the row-scaled value, within 2^-21 of it; all others keep all their bits.
  * A is read with 16-byte alignment (A must be 16-byte aligned, like B).
  * The kernel streams B once with 16-byte loads; K is split over ksplit workgroups per strip of
  * g16_skinny_strip_cols(M, N) columns (256 up to N = 8192, 512 above) and reduced

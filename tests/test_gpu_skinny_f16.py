@@ -101,9 +101,9 @@ def test_fast_linear_fp16_decode(cuda, M, decode_copy):
         assert torch.equal(out, y) and torch.equal(fl(x), y)
 
 
-# (M, K, N): the matrix-core form at every M it serves, past one group of 128 K rows per wavefront
-# (activations grouped, row exponents raised between groups), ragged last batches, both activation
-# types; 512 x 9000 has too few rows per wavefront for it
+# (M, K, N): what fp16 activations take on the matrix cores (6 x 14336 x 4096: 112 rows per wavefront),
+# and shapes on 512-column strips or with short wavefronts, where they and fp32 ones take the FMA loop;
+# rising values, infinities and NaN
 @pytest.mark.parametrize("M,K,N", [(8, 8192, 9216), (7, 7000, 8200), (7, 4096, 11008), (6, 14336, 4096), (5, 11008, 520),
                                    (8, 4104, 8712), (7, 512, 9000)])
 @pytest.mark.parametrize("kind", ["plain", "rising", "inf"])

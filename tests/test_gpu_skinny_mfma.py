@@ -2,8 +2,9 @@
 
 mm_t with M = 8 and N <= 8192 runs the split skinny kernel; where each wavefront gets 32..128 K rows
 its multiplies run as v_mfma_f32_16x16x32_f16 on an fp16 hi/lo split of the row-scaled activations
-(reference semantics: fp32 math on the unquantised activations, kernels.py:160-219). The shapes below
-take that form (checked from the plan); the bar is the skinny bar of every other skinny test, and
+(reference semantics: fp32 math on the unquantised activations, kernels.py:160-219); fp16 activations
+take the matrix cores unsplit, from M = 5 on and on longer wavefronts too (test_gpu_skinny_f16.py).
+The shapes below take that form (checked from the plan); the bar is the skinny bar of every other skinny test, and
 infinities and NaNs must land where the oracle's fp64 products put them.
 """
 from __future__ import annotations
@@ -50,7 +51,8 @@ def _rows_per_wave(lib, cuda, M, N, K):
 
 
 def _takes_matrix_cores(lib, cuda, M, N, K):
-    # use_mf in skinny.hip: M = 8, 256-column strips (N <= 8192), 32..128 K rows per wavefront
+    # use_mf in skinny.hip, both activation types: M = 8, 256-column strips (N <= 8192), 32..128 K rows per
+    # wavefront
     rpw, _ = _rows_per_wave(lib, cuda, M, N, K)
     return M == 8 and lib.g16_skinny_strip_cols(M, N) == 256 and 32 <= rpw <= 128
 
