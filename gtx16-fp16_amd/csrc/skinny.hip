@@ -115,9 +115,10 @@ __device__ inline void split_hi_lo(float x, _Float16& hi, _Float16& lo) {
 // MF (launched by use_mf: larger M on 256-column strips, enough K rows per wavefront): the wavefront
 // multiplies on the matrix cores (below), with fp32 activations only if all of its are finite; one
 // with an inf or NaN among them takes the fp32 FMA loop.
-template <typename TX, int MM, class S, bool MF = false>
+//   C16: the output is fp16. (As an argument it slowed the fp32 form: 7 x 4096 x 11008 24.8 us, 24.0.)
+template <typename TX, int MM, class S, bool C16, bool MF = false>
 __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__ A, const _Float16* __restrict__ B,
-                                                          void* __restrict__ Cv, int c_f16, const float* __restrict__ bias,
+                                                          void* __restrict__ Cv, const float* __restrict__ bias,
                                                           float* __restrict__ part, uint32_t* __restrict__ counters,
                                                           int N, int K, int rows_per_wave, int ksplit, int nstrips) {
   constexpr int kStripCols = S::cols, kLanesPerRow = S::lanes_per_row, kRowsPerLoad = S::rows_per_load;
@@ -222,7 +223,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc2[s][j] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
-      for (int g0 = 0; g0 < nb; g0 += kMfGroup) {
+      for (int g0 = 0; g0 < (XF16 ? nb : 1); g0 += kMfGroup) {
         // The group's first weights stream while its activations come in (a wavefront that falls
         // back to the FMA loop drops them). Rows past the wavefront's range (and rows am >= M) are 0.
         load_batch(k0 + kMfBatch * g0);
@@ -373,7 +374,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
 
   // an fp16 output is the fp32 sum rounded once, as a cast of an fp32 output would
   auto put = [&](size_t i, float v) {
-    if (c_f16) static_cast<_Float16*>(Cv)[i] = static_cast<_Float16>(v);
+    if constexpr (C16) static_cast<_Float16*>(Cv)[i] = static_cast<_Float16>(v);
     else static_cast<float*>(Cv)[i] = v;
   };
 
@@ -465,7 +466,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
     const size_t o = static_cast<size_t>(group_row(i)) * N + c;
     if constexpr (kGW == 4) {
       if (bias != nullptr) v += float4v{bias[c], bias[c + 1], bias[c + 2], bias[c + 3]};
-      if (c_f16) *reinterpret_cast<half4*>(static_cast<_Float16*>(Cv) + o) = __builtin_convertvector(v, half4);
+      if constexpr (C16) *reinterpret_cast<half4*>(static_cast<_Float16*>(Cv) + o) = __builtin_convertvector(v, half4);
       else *reinterpret_cast<float4v*>(static_cast<float*>(Cv) + o) = v;
     } else {
       put(o, v + (bias != nullptr ? bias[c] : 0.f));
@@ -540,7 +541,7 @@ Split split_for(int K, int ksplit) {
 }
 
 template <typename TX>
-using SkinnyFn = void (*)(const TX*, const _Float16*, void*, int, const float*, float*, uint32_t*, int, int, int, int, int);
+using SkinnyFn = void (*)(const TX*, const _Float16*, void*, const float*, float*, uint32_t*, int, int, int, int, int);
 
 // The schedule of each M and strip width: graph-timed sweeps on MI355X of 2-16 loads per batch,
 // with and without the issue barrier, over M = 1..8 and K x N in {4096^2, 1024 x 3072,
@@ -572,17 +573,17 @@ int strip_cols(int M, int N) {
   return N <= 8192 ? 256 : 512;
 }
 
-template <typename TX, int COLS>
+template <typename TX, int COLS, bool C16>
 SkinnyFn<TX> skinny_fn_w(int M) {
   switch (M) {
-    case 1: return skinny_kernel<TX, 1, typename SchedFor<1, COLS>::type>;
-    case 2: return skinny_kernel<TX, 2, typename SchedFor<2, COLS>::type>;
-    case 3: return skinny_kernel<TX, 3, typename SchedFor<3, COLS>::type>;
-    case 4: return skinny_kernel<TX, 4, typename SchedFor<4, COLS>::type>;
-    case 5: return skinny_kernel<TX, 5, typename SchedFor<5, COLS>::type>;
-    case 6: return skinny_kernel<TX, 6, typename SchedFor<6, COLS>::type>;
-    case 7: return skinny_kernel<TX, 7, typename SchedFor<7, COLS>::type>;
-    default: return skinny_kernel<TX, 8, typename SchedFor<8, COLS>::type>;
+    case 1: return skinny_kernel<TX, 1, typename SchedFor<1, COLS>::type, C16>;
+    case 2: return skinny_kernel<TX, 2, typename SchedFor<2, COLS>::type, C16>;
+    case 3: return skinny_kernel<TX, 3, typename SchedFor<3, COLS>::type, C16>;
+    case 4: return skinny_kernel<TX, 4, typename SchedFor<4, COLS>::type, C16>;
+    case 5: return skinny_kernel<TX, 5, typename SchedFor<5, COLS>::type, C16>;
+    case 6: return skinny_kernel<TX, 6, typename SchedFor<6, COLS>::type, C16>;
+    case 7: return skinny_kernel<TX, 7, typename SchedFor<7, COLS>::type, C16>;
+    default: return skinny_kernel<TX, 8, typename SchedFor<8, COLS>::type, C16>;
   }
 }
 // The matrix-core form (skinny_kernel's MF) runs on 256-column strips with enough K rows per wavefront
@@ -600,19 +601,19 @@ bool use_mf(int M, int cols, int rows_per_wave) {
   if (std::is_same_v<TX, float>) return M == 8 && rows_per_wave >= kMfBatch && rows_per_wave <= kMfBatch * kMfGroup;
   return M >= 5 && rows_per_wave >= (M == 8 ? kMfBatch : (M == 7 ? 64 : 80));
 }
-template <typename TX>
+template <typename TX, bool C16>
 SkinnyFn<TX> skinny_fn(int M, int cols, bool mf) {
   if (mf) {
     if constexpr (std::is_same_v<TX, _Float16>) {
       switch (M) {
-        case 5: return skinny_kernel<TX, 5, typename SchedFor<5, 256>::type, true>;
-        case 6: return skinny_kernel<TX, 6, typename SchedFor<6, 256>::type, true>;
-        case 7: return skinny_kernel<TX, 7, typename SchedFor<7, 256>::type, true>;
+        case 5: return skinny_kernel<TX, 5, typename SchedFor<5, 256>::type, C16, true>;
+        case 6: return skinny_kernel<TX, 6, typename SchedFor<6, 256>::type, C16, true>;
+        case 7: return skinny_kernel<TX, 7, typename SchedFor<7, 256>::type, C16, true>;
       }
     }
-    return skinny_kernel<TX, 8, typename SchedFor<8, 256>::type, true>;
+    return skinny_kernel<TX, 8, typename SchedFor<8, 256>::type, C16, true>;
   }
-  return cols == 256 ? skinny_fn_w<TX, 256>(M) : skinny_fn_w<TX, 512>(M);
+  return cols == 256 ? skinny_fn_w<TX, 256, C16>(M) : skinny_fn_w<TX, 512, C16>(M);
 }
 
 size_t workspace_bytes(int M, int N, int ksplit) {
@@ -672,9 +673,10 @@ int skinny_launch(const TX* A, const uint16_t* B, void* C, int c_f16, const floa
     part = static_cast<float*>(ws);
   }
   const dim3 grid(static_cast<unsigned>(nstrips) * static_cast<unsigned>(sp.ksplit)), block(kThreads);
-  return launch(skinny_fn<TX>(M, cols, use_mf<TX>(M, cols, sp.rows_per_wave)), grid, block, static_cast<hipStream_t>(stream), A,
-                reinterpret_cast<const _Float16*>(B), C, c_f16, bias, part, counters, N, K, sp.rows_per_wave, sp.ksplit,
-                nstrips);
+  const bool mf = use_mf<TX>(M, cols, sp.rows_per_wave);
+  const auto fn = c_f16 != 0 ? skinny_fn<TX, true>(M, cols, mf) : skinny_fn<TX, false>(M, cols, mf);
+  return launch(fn, grid, block, static_cast<hipStream_t>(stream), A, reinterpret_cast<const _Float16*>(B), C, bias, part,
+                counters, N, K, sp.rows_per_wave, sp.ksplit, nstrips);
 }
 
 __global__ void clear_words(uint32_t* p, int n) {
