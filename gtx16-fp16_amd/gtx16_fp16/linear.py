@@ -267,11 +267,14 @@ class FastLinear(nn.Module):
             M = x2.shape[0]
             b = self.bias
             wp = None
-            # the 256x128 tiles run no faster on a prepacked weight (777 x 3072 x 8192: 59.5 us, mm_t 57.0;
-            # fp32 x 61.7, 58.0): it serves them only where it lets layers share one cast
+            # On 256x128 tiles a prepacked weight gains where the batch has more rows than the layer columns, up
+            # to 6 % (8241 x 896 x 744 fp16 33.1 -> 31.9 us, 2339 x 5760 x 2056 105.0 -> 100.6, 3291 x 4256 x 1304
+            # 88.7 -> 83.4), and loses below, up to 4 % (777 x 3072 x 8192 57.0 -> 59.5, 2086 x 3728 x 3072 76.7 ->
+            # 79.4): there it serves them only where it lets layers share one cast.
             if self.prepack_weight and M > SKINNY_MAX_M and \
                     prepacked_route(M, self.out_features, self.in_features, x2.device) and \
-                    (self.share_cast or _gemm_route(_clib.load(), M, self.out_features, self.in_features, x2.device)[6]):
+                    (M >= self.out_features or self.share_cast
+                     or _gemm_route(_clib.load(), M, self.out_features, self.in_features, x2.device)[6]):
                 wp = self._packed_weight()
             if wp is not None:
                 y = mm_t_prepacked(x2, self.weight_t, wp, b, odt, _cast_source=x if self.share_cast else None)

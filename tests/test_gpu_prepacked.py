@@ -319,3 +319,20 @@ def test_shared_cast_leaves_fp16_products_uncast(ops, cuda):
         z = ops.mm_t_prepacked(x, fl.weight_t, ops.pack_weight(fl.weight_t), None, torch.float32, _cast_source=x)
         assert torch.equal(z, g.mm_t(x, fl.weight_t)) and (z[7, :8] == 3 * 2.0 ** -24).all()
     assert len(ops._cast_cache) == 0
+
+
+# (M, K, N, prepacked): 256x128 tiles take the copy from as many rows as columns on, 256x256 ones always
+@pytest.mark.parametrize("M,K,N,prepacked", [(2474, 392, 2368, True), (2061, 672, 2656, False), (8241, 896, 744, True),
+                                             (777, 1096, 8192, False), (4096, 264, 4096, True), (2304, 264, 4096, True)])
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+def test_layers_build_the_copy_where_it_gains(ops, cuda, M, K, N, prepacked, dt):
+    import gtx16_fp16 as g
+
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the shapes are for 256 CUs")
+    assert ops.prepacked_route(M, N, K, cuda)
+    torch.manual_seed(0)
+    fl = g.FastLinear.from_linear(nn.Linear(K, N).to(cuda))
+    x = torch.randn(M, K, device=cuda).to(dt)
+    assert torch.equal(fl(x), g.mm_t(x, fl.weight_t, fl.bias, dt))
+    assert (fl._wp is not None) == prepacked
