@@ -11,7 +11,7 @@ import torch.nn.functional as F
 from . import _clib, ops
 from .kernels import SKINNY_MAX_M, PreparedCall, scratch_buffer, split_buffers, stream_handle
 from .ops import (STRIPS_MAX_M, _gemm_route, _is_target, _sm_count, is_affected, mm_t,
-                  mm_t_prepacked, pack_decode_weight, pack_weight, prepacked_route, skinny_strips, supported,
+                  mm_t_prepacked, pack_decode_weight, pack_weight, skinny_strips, supported,
                   tensor_version)
 
 _F32, _F16 = torch.float32, torch.float16  # forward's type checks cost more with the attribute lookups
@@ -199,10 +199,11 @@ class FastLinear(nn.Module):
         # None: not that case (the general path then decides).
         w, b, dev = self.weight_t, self.bias, x.device
         K, N = self.in_features, self.out_features
-        if not self._operands_ok(w, b, dev):
+        if K % 8 or N % 8:
             return None
+        # the route before the operands: on a packed one this look-up comes on top of the general path's work
         kind, scratch_bytes, _ks, ws_bytes, cnt_bytes = _gemm_route(_clib.load(), M, N, K, dev)[:5]
-        if kind == "packed":
+        if kind == "packed" or not self._operands_ok(w, b, dev):
             return None
         stream = stream_handle(dev.index or 0)
         out = torch.empty(*x.shape[:-1], N, device=dev, dtype=x.dtype)
@@ -271,11 +272,10 @@ class FastLinear(nn.Module):
             # to 6 % (8241 x 896 x 744 fp16 33.1 -> 31.9 us, 2339 x 5760 x 2056 105.0 -> 100.6, 3291 x 4256 x 1304
             # 88.7 -> 83.4), and loses below, up to 4 % (777 x 3072 x 8192 57.0 -> 59.5, 2086 x 3728 x 3072 76.7 ->
             # 79.4): there it serves them only where it lets layers share one cast.
-            if self.prepack_weight and M > SKINNY_MAX_M and \
-                    prepacked_route(M, self.out_features, self.in_features, x2.device) and \
-                    (M >= self.out_features or self.share_cast
-                     or _gemm_route(_clib.load(), M, self.out_features, self.in_features, x2.device)[6]):
-                wp = self._packed_weight()
+            if self.prepack_weight and M > SKINNY_MAX_M:
+                raw, prepacked = _gemm_route(_clib.load(), M, self.out_features, self.in_features, x2.device)[6:]
+                if prepacked and (raw or M >= self.out_features or self.share_cast):
+                    wp = self._packed_weight()
             if wp is not None:
                 y = mm_t_prepacked(x2, self.weight_t, wp, b, odt, _cast_source=x if self.share_cast else None)
             elif (self.prepack_decode and M <= STRIPS_MAX_M and x2.device == self.weight_t.device
@@ -288,7 +288,11 @@ class FastLinear(nn.Module):
                 y = skinny_strips(x2, self._wd, b)
             else:
                 y = mm_t(x2, self.weight_t, self.bias, odt)
-        return y.reshape(*shape[:-1], self.out_features).to(out_dtype)
+        if y.dtype != out_dtype:
+            y = y.to(out_dtype)
+        if len(shape) == 2 and shape[1] == self.in_features and y.shape[1] == self.out_features:
+            return y
+        return y.reshape(*shape[:-1], self.out_features)
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, bias={self.bias is not None}"

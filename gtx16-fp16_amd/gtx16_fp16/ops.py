@@ -94,10 +94,11 @@ _routes: dict[tuple[int, int, int, int], tuple] = {}
 
 
 def _gemm_route(lib, M: int, N: int, K: int, dev: torch.device) -> tuple:
-    """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes, direct, raw) of the
-    GEMM path for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count; direct:
-    fp32 activations run as one launch that casts them itself (g16_mm_t_direct); raw: fp16
-    activations as one launch that needs no cast (g16_mm_t_raw)."""
+    """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes, direct, raw, prepacked)
+    of the GEMM path for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count;
+    direct: fp32 activations run as one launch that casts them itself (g16_mm_t_direct); raw: fp16
+    activations as one launch that needs no cast (g16_mm_t_raw); prepacked: a prepacked weight serves
+    it (prepacked_route)."""
     key = (M, N, K, dev.index or 0)
     r = _routes.get(key)
     if r is None:
@@ -105,14 +106,14 @@ def _gemm_route(lib, M: int, N: int, K: int, dev: torch.device) -> tuple:
         scratch = lib.g16_mm_t_scratch_bytes(M, N, K, cus)
         if lib.g16_hgemm_use_packed(M, N, K, cus):
             r = ("packed", scratch, 1, 0, 0, lib.g16_mm_t_direct_route(M, N, K, cus) == 1,
-                 lib.g16_mm_t_raw_route(M, N, K, cus) == 1)
+                 lib.g16_mm_t_raw_route(M, N, K, cus) == 1, lib.g16_hgemm_use_packed_b(M, N, K, cus) == 1)
         else:
             ksplit = lib.g16_hgemm_plan(M, N, K, cus)
             if ksplit > 1:
                 r = ("splitk", scratch, ksplit, lib.g16_hgemm_splitk_workspace_bytes(M, N, K, ksplit, cus),
-                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False, False)
+                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False, False, False)
             else:
-                r = ("plain", scratch, 1, 0, 0, False, False)
+                r = ("plain", scratch, 1, 0, 0, False, False, False)
         _remember(key, r)
     return r
 
@@ -214,7 +215,7 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     if x2d.dtype == torch.float16 and dev.index not in _spec_history:
         if lib.g16_mm_t_spec_history(stream) == 0:
             _spec_history.add(dev.index)
-    kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct, raw = _gemm_route(lib, M, N, K, dev)
+    kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct, raw, _pb = _gemm_route(lib, M, N, K, dev)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
     if (direct and _direct_thresh()) if x2d.dtype == torch.float32 else raw:
         _direct(lib, x2d, w_t, 0, out, bptr, M, N, K, dev, stream)
@@ -247,10 +248,9 @@ def _direct(lib, x2d: torch.Tensor, w: torch.Tensor, packed: int, out: torch.Ten
 
 
 def prepacked_route(M: int, N: int, K: int, device: torch.device) -> bool:
-    """True where mm_t takes the tile-packed route on the 256x256 tile, the one a prepacked weight
-    serves."""
-    return _gemm_route(_clib.load(), M, N, K, device)[0] == "packed" and \
-        _clib.load().g16_hgemm_use_packed_b(M, N, K, _sm_count(device)) == 1
+    """True where mm_t takes the tile-packed route on the 256x256 or 256x128 tile, the ones a prepacked
+    weight serves."""
+    return _gemm_route(_clib.load(), M, N, K, device)[7]
 
 
 def pack_weight(w_t: torch.Tensor) -> torch.Tensor:
@@ -367,9 +367,12 @@ def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias:
     M, K = x2d.shape
     N = w_t.shape[1]
     dev = x2d.device
-    if M <= SKINNY_MAX_M or not prepacked_route(M, N, K, dev):
-        return mm_t(x2d, w_t, bias, out_dtype)
     lib = _clib.load()
+    if M <= SKINNY_MAX_M:
+        return mm_t(x2d, w_t, bias, out_dtype)
+    direct, raw, prepacked = _gemm_route(lib, M, N, K, dev)[5:]
+    if not prepacked:
+        return mm_t(x2d, w_t, bias, out_dtype)
     if wp.dtype != torch.float16 or wp.device != dev or not wp.is_contiguous() or \
             wp.numel() * 2 < lib.g16_packed_b_bytes(K, N) or wp.data_ptr() % 16 != 0:
         raise ValueError("wp is not a packed weight for this w_t (use pack_weight(w_t))")
@@ -377,7 +380,6 @@ def mm_t_prepacked(x2d: torch.Tensor, w_t: torch.Tensor, wp: torch.Tensor, bias:
     b = None if bias is None else bias.float().contiguous()
     x2d = _aligned(x2d)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
-    direct, raw = _gemm_route(lib, M, N, K, dev)[5:]
     # One launch that reads x itself; for fp32 x not where layers share a cast of it: three direct launches
     # take 4 to 9 % longer than a cast and three packed GEMMs (65536 x 768^2 327 us, 314; 16384 x 4096 x 1024
     # 421, 387), two as long, one 15 % less. Raw ones are no slower shared (8192 x 2048^2 172 us, 180;
