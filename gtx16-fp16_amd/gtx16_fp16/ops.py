@@ -186,6 +186,7 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     bptr = None if b is None else b.data_ptr()
 
     x2d = _aligned(x2d)
+    f32 = x2d.dtype == torch.float32
     if M <= SKINNY_MAX_M:  # memory-bound path, fp32 math
         out = torch.empty(M, N, device=dev, dtype=out_dtype)
         key = (-M, N, K, dev.index or 0)
@@ -197,8 +198,8 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
             _remember(key, plan)
         ksplit = plan[0]
         bufs = split_buffers(dev, stream, plan[1], plan[2])
-        _clib.check(_clib.fast().skinny(x2d.data_ptr(), 1 if x2d.dtype == torch.float32 else 0, w_t.data_ptr(),
-                                        out.data_ptr(), 1 if out_dtype == torch.float16 else 0, bptr, M, N, K, ksplit,
+        _clib.check(_clib.fast().skinny(x2d.data_ptr(), f32, w_t.data_ptr(),
+                                        out.data_ptr(), out_dtype == torch.float16, bptr, M, N, K, ksplit,
                                         *bufs, stream), "skinny GEMM")
         return out
 
@@ -212,19 +213,19 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     # The speculation history lets a weight whose fp16 call needed a tile computed again take the
     # two-launch route for a while; it is enabled once per device (a small pinned allocation,
     # retried on a later call if this one is being captured into a graph).
-    if x2d.dtype == torch.float16 and dev.index not in _spec_history:
+    if not f32 and dev.index not in _spec_history:
         if lib.g16_mm_t_spec_history(stream) == 0:
             _spec_history.add(dev.index)
     kind, scratch_bytes, _ks, ws_bytes, cnt_bytes, direct, raw, _pb = _gemm_route(lib, M, N, K, dev)
     out = torch.empty(M, N, device=dev, dtype=out_dtype)
-    if (direct and _direct_thresh()) if x2d.dtype == torch.float32 else raw:
+    if (direct and _direct_thresh()) if f32 else raw:
         _direct(lib, x2d, w_t, 0, out, bptr, M, N, K, dev, stream)
         return out
     # no scratch where the GEMM casts its own rows into LDS (one launch, the unsplit small tile)
     scratch = scratch_buffer(dev, stream, scratch_bytes) if scratch_bytes else None
     bufs = split_buffers(dev, stream, ws_bytes, cnt_bytes) if kind == "splitk" else (None, 0, None, 0)
-    _clib.check(_clib.fast().mm_t_gemm(x2d.data_ptr(), 1 if x2d.dtype == torch.float32 else 0, w_t.data_ptr(),
-                                  out.data_ptr(), 1 if out_dtype == torch.float16 else 0, bptr, ROW_SCALE_THRESHOLD,
+    _clib.check(_clib.fast().mm_t_gemm(x2d.data_ptr(), f32, w_t.data_ptr(),
+                                  out.data_ptr(), out_dtype == torch.float16, bptr, ROW_SCALE_THRESHOLD,
                                   M, N, K, _sm_count(dev), None if scratch is None else scratch.data_ptr(),
                                   scratch_bytes, *bufs, stream), "GEMM")
     return out
