@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kThreads) void skinny_kernel(const TX* __restrict__
 
   // Matrix-core form (MF): one v_mfma_f32_16x16x32_f16 computes 16 A rows x 16 columns x 32 K
   // rows. Its A rows 0-7 are the fp16 hi parts of the (row-scaled) activations, rows 8-15 their lo
-  // parts (split_hi_lo), so C[m] + C[m + 8] is the fp32-accurate product for m < 8: the products
+  // parts (split_hi_lo), so C[m] + C[m + 8] is the product for m < 8, each x to 2^-21: the products
   // of fp16 parts are exact, and the fp32 FMAs per weight and row become ~100 VALU instructions per
   // 32 rows. Each row m is scaled by 2^-e_m (exact) so its largest |x| over the wavefront's rows
   // lies in [2^14, 2^15), and the partial sum is scaled back by 2^e_m.
