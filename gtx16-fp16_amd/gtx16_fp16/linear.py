@@ -141,11 +141,13 @@ class FastLinear(nn.Module):
                 # the split kernel on weight_t always (also the decode layout's stand-in while its copy
                 # cannot be built: under graph capture)
                 ksplit = lib.g16_skinny_plan(M, N, K, _sm_count(dev))
-                pl = PreparedCall(_clib.fast().skinny, "skinny GEMM")
+                # (fp32 calls have entry points of their own, without the two type arguments)
+                pl = PreparedCall(_clib.fast().skinny_f32in if f32 else _clib.fast().skinny, "skinny GEMM")
                 sizes = (lib.g16_skinny_workspace_bytes(M, N, K, ksplit),
                          lib.g16_skinny_counter_bytes(M, N, K, ksplit))
                 if self.prepack_decode and lib.g16_skinny_strips_route(M, N, K, int(f32)):
-                    pls = PreparedCall(_clib.fast().skinny_strips, "skinny GEMM (decode layout)")
+                    pls = PreparedCall(_clib.fast().skinny_strips_f32in if f32 else _clib.fast().skinny_strips,
+                                       "skinny GEMM (decode layout)")
             entry = (pl, ksplit, sizes, w.data_ptr(), bptr, pls)
             self._skinny[key] = entry
         return entry
@@ -246,10 +248,16 @@ class FastLinear(nn.Module):
                         w = self.weight_t
                         wd = self._wd_ptr if self._wd_key == (wptr, tensor_version(w), w.device) else self._decode_weight()
                     if wd:
-                        pls(x.data_ptr(), f32, wd, out.data_ptr(), not f32, bptr, M, N, K, stream)
+                        if f32:
+                            pls(x.data_ptr(), wd, out.data_ptr(), bptr, M, N, K, stream)
+                        else:
+                            pls(x.data_ptr(), False, wd, out.data_ptr(), True, bptr, M, N, K, stream)
                     else:
                         bufs = split_buffers(dev, stream, *sizes)
-                        pl(x.data_ptr(), f32, wptr, out.data_ptr(), not f32, bptr, M, N, K, ksplit, *bufs, stream)
+                        if f32:
+                            pl(x.data_ptr(), wptr, out.data_ptr(), bptr, M, N, K, ksplit, *bufs, stream)
+                        else:
+                            pl(x.data_ptr(), False, wptr, out.data_ptr(), True, bptr, M, N, K, ksplit, *bufs, stream)
                     return out
             elif f32 and M > SKINNY_MAX_M:
                 out = self._small_gemm(x, M)
