@@ -1921,7 +1921,8 @@ bool raw_route(const Plan& p, int K, int ksplit) { return p.tile == Tile::T256 &
 
 // fp32 activations also run as one direct launch on the 4-wavefront tiles with 64-deep K steps, where
 // the cast's launch (2 to 7 us) costs more than streaming A at 4 bytes instead of 2: for up to 64 rows
-// always; above, on short slices of split grids or of many rows, and past K = 4096 in 3 slices or more.
+// always; above, on short slices of split grids or of many rows, and past K = 4096 in 3 slices or more
+// or into at most 6 tile columns (which read x again).
 // Graph-timed, rotated operands, cast + GEMM -> direct (us, M x K x N): 32x128 tiles 64 x 4096 x 1024
 // 12.6 -> 11.2, 16 x 4096^2 17.1 -> 14.6, 40 x 11008 x 5120 39.3 -> 36.1, 9 x 14336 x 512 17.4 -> 17.2;
 // 64x128 tiles 64 x 4096 x 11008 30.6 -> 30.8, 33 x 2048 x 14336 22.5 -> 20.6; 64x64 tiles 256 x 4096
@@ -1929,7 +1930,10 @@ bool raw_route(const Plan& p, int K, int ksplit) { return p.tile == Tile::T256 &
 // more 160 x 11008 x 1536 32.5 -> 31.8, 250 x 6144 x 512 17.6 -> 13.8, 1005 x 6560 x 264 29.9 -> 24.2,
 // 142 x 8192 x 1856 28.7 -> 25.9 (over 59 such shapes 0.93 to 1.30 times, 1.11 in the mean); 2 slices
 // 128 x 6144 x 4096 29.9 -> 32.8, 700 x 6144 x 512 27.9 -> 30.2, but 128 x 6144 x 8192 40.6 -> 39.2;
-// unsplit 333 x 4104 x 4096 37.8 -> 41.4, 339 x 9984 x 3712 66.2 -> 86.9, 700 x 4352 x 1024 28.8 -> 33.1.
+// unsplit 333 x 4104 x 4096 37.8 -> 41.4, 339 x 9984 x 3712 66.2 -> 86.9, 700 x 4352 x 1024 28.8 -> 33.1;
+// up to 6 columns 4451 x 6344 x 288 88.5 -> 65.2, 3193 x 6600 x 432 86.5 -> 69.7, 2274 x 7128 x 704 73.9 ->
+// 68.2, 2527 x 6232 x 264 (2 slices) 54.6 -> 39.8, but 2508 x 4184 x 296 40.2 -> 42.3 (29 shapes 0.95 to 1.41
+// times, 1.14 in the mean), 7 columns 1554 x 5320 x 432 43.1 -> 51.2, 1939 x 6496 x 392 53.3 -> 50.7.
 // Not taken below either: 256 x 1024^2 11.3 -> 11.3 (11.4 -> 12.3 with a row past fp16's range), 256 x
 // 2048 x 4096 16.5 -> 18.2, 333 x 4096^2 (64x128) 36.0 -> 39.7.
 bool stream_route(const Plan& p, int M, int K, const KSplit& ks) {
@@ -1938,7 +1942,7 @@ bool stream_route(const Plan& p, int M, int K, const KSplit& ks) {
   if (ks.ksplit > kSpecMaxSplit || (ks.ksplit > 1 && 4L * ks.ksplit * p.ntn > 2L * K)) return false;
   if (p.tile == Tile::T32) return true;
   if (p.tile != Tile::T64 && p.tile != Tile::T64x64) return false;
-  return M <= 64 || (K > 4096 && ks.ksplit >= 3) || (ks.kchunk <= 1024 && (ks.ksplit > 1 || M >= 512 || K <= 768));
+  return M <= 64 || (K > 4096 && (ks.ksplit >= 3 || p.ntn <= 6)) || (ks.kchunk <= 1024 && (ks.ksplit > 1 || M >= 512 || K <= 768));
 }
 
 // A speculative launch (mm_t's GEMM path in one launch for fp16 x on the 4-wavefront tiles): log2

@@ -215,10 +215,12 @@ def test_slices_past_fp32_range_cancel(cuda, M, K, N, tile, ks):
         assert (err <= 2.0 ** -10).all(), err.max()
 
 
-# (M, K, N, slices, streamed): above 64 rows and past K = 4096 only 3 slices and more are streamed
+# (M, K, N, slices, streamed): above 64 rows and past K = 4096 only 3 slices and more, or up to 6 tile
+# columns, are streamed
 @pytest.mark.parametrize("M,K,N,ks,streamed", [
     (333, 4104, 4096, 1, False), (700, 4352, 1024, 1, False), (128, 6144, 4096, 2, False), (160, 11008, 1536, 3, True),
-    (142, 8192, 1856, 5, True), (333, 4096, 4096, 1, False), (64, 4096, 11008, 2, True), (1024, 1024, 1024, 1, True)])
+    (142, 8192, 1856, 5, True), (333, 4096, 4096, 1, False), (64, 4096, 11008, 2, True), (1024, 1024, 1024, 1, True),
+    (3193, 6600, 432, 1, True), (2318, 6304, 264, 1, True), (2527, 6232, 264, 2, True), (1554, 5320, 432, 1, False)])
 def test_route_by_its_rounding(cuda, M, K, N, ks, streamed):
     # a row with |max| 2000 is halved by the rowscale cast, and 3 * 2^-24 with it (to 2 * 2^-24, a tie to
     # even); the streamed tiles scale only rows that leave fp16's range
