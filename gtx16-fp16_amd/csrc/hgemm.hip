@@ -1896,11 +1896,15 @@ bool resident_route(const Plan& p, int ksplit, int K) {
 // 38 (29 without such rows).
 constexpr int kDirectMaxK = 1 << 20;
 constexpr int kDirectMaxN = 1024;
+// What the direct kernel takes (a caller of g16_mm_t_direct may have it run there), and where it gains.
+bool direct_able(const Plan& p, int N, int K, int ksplit, int num_cus) {
+  return p.tile == Tile::T256 && ksplit == 1 && K > 0 && K <= kDirectMaxK && N <= kDirectMaxN &&
+         4L * p.ntm * p.ntn >= 3L * num_cus;
+}
 bool direct_route(const Plan& p, int N, int K, int ksplit, int num_cus) {
-  if (p.tile != Tile::T256 || ksplit != 1 || K <= 0 || K > kDirectMaxK || N > kDirectMaxN) return false;
-  const long tiles = static_cast<long>(p.ntm) * p.ntn, cus = num_cus;
-  if (4 * tiles < 3 * cus) return false;
+  if (!direct_able(p, N, K, ksplit, num_cus)) return false;
   if (K <= 512) return true;
+  const long tiles = static_cast<long>(p.ntm) * p.ntn, cus = num_cus;
   const long rounds = (tiles + cus - 1) / cus, rows = 256L * p.ntm;  // 11008 or 14336 rows a round on 256 CUs
   if (rows < (K <= 1024 ? 43 : 56) * cus * rounds) return false;
   return !(K <= 1024 && N > 768 && N % 64 != 0 && rounds > 3);
@@ -1914,10 +1918,18 @@ bool direct_thresh(int texp) { return texp >= kDirectMinTexp && texp <= kDirectM
 // fp16 activations run as one raw launch (x is the GEMM's A as it is, no cast) where the plan is the
 // unsplit 256x256 tile: the cast it saves costs more than A's row-major DMA (64-byte pieces of 16 rows
 // instead of 1 KB runs) adds to the GEMM. Graph-timed, cast + packed GEMM -> raw (us, M x K x N, fp16
-// out): 8192 x 2048^2 72 -> 63 (61 prepacked), 16384 x 1024^2 48.9 -> 35.7, 65536 x 768 x 768 124 -> 90,
-// 65536 x 768 x 2048 257 -> 223, 4000 x 1000 x 5000 81 -> 75, 4096^3 118 -> 110. On 256x128 tiles, whose A stream weighs twice as much per
-// product, it does not: 2048 x 4096^2 cast + packed GEMM 79.6 us, raw 84.5; 1500 x 4096^2 75.1, 77.8.
-bool raw_route(const Plan& p, int K, int ksplit) { return p.tile == Tile::T256 && ksplit == 1 && K > 0; }
+// out): 8192 x 2048^2 74 -> 64, 16384 x 1024^2 48.9 -> 35.7, 65536 x 768 x 2048 257 -> 223, 4096^3 118 -> 110,
+// 4096 x 4128 x 4096 120 -> 120. On 256x128 tiles, whose A stream weighs twice as much per product, it does
+// not: 2048 x 4096^2 cast + packed GEMM 79.6 us, raw 84.5; 1500 x 4096^2 75.1, 77.8.
+//   Rows of x that are no whole number of those pieces (K % 32 != 0) straddle cache lines, once per tile
+// column that reads them: up to 4 columns raw still gains at every K (16384 x 4104 x 1024 1.22 times,
+// 24952 x 6200 x 736 1.05), up to 20 to K ~ 1000 (4000 x 1000 x 5000 82 -> 76, 5000 x 1304 x 4096 0.98 to 1.03, 5000
+// x 2056 x 4096 0.94, 8192 x 6200 x 2048 0.96), beyond to K ~ 500 (2048 x 520 x 8192 1.01, 1138 x 776 x 12208
+// 0.98, 4329 x 3560 x 7088 199 -> 251; 3000 x 1000 x 8192 would gain, 1.09).
+bool raw_able(const Plan& p, int K, int ksplit) { return p.tile == Tile::T256 && ksplit == 1 && K > 0; }
+bool raw_route(const Plan& p, int K, int ksplit) {
+  return raw_able(p, K, ksplit) && (K % 32 == 0 || p.ntn <= 4 || K <= (p.ntn <= 20 ? 1048 : 520));
+}
 
 // fp32 activations also run as one direct launch on the 4-wavefront tiles with 64-deep K steps, where
 // the cast's launch (2 to 7 us) costs more than streaming A at 4 bytes instead of 2: for up to 64 rows
@@ -1977,8 +1989,8 @@ int gemm_launch(const uint16_t* A, const uint16_t* B, void* C, bool out_f16, con
   const KSplit ks = ksplit_for(K, ksplit);
   if (num_cus <= 0) num_cus = stream_cus(static_cast<hipStream_t>(stream));
   Plan p = choose_tile(M, N, K, num_cus);
-  if (direct ? !direct_route(p, N, K, ks.ksplit, num_cus) && !stream_route(p, M, K, ks) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
-  if (raw && !raw_route(p, K, ks.ksplit) && !(p.raw_without_scratch && ks.ksplit == 1 && !packed_b)) return G16_E_SHAPE;
+  if (direct ? !direct_able(p, N, K, ks.ksplit, num_cus) && !stream_route(p, M, K, ks) : (rc != nullptr && !resident_route(p, ks.ksplit, K))) return G16_E_SHAPE;
+  if (raw && !raw_able(p, K, ks.ksplit) && !(p.raw_without_scratch && ks.ksplit == 1 && !packed_b)) return G16_E_SHAPE;
   const bool spec = sp != nullptr;
   if (spec && (!four_wave(p.tile) || packed ||
                ks.ksplit > kSpecMaxSplit || sp->texp < kSpecMinTexp))
@@ -2307,7 +2319,7 @@ extern "C" int g16_mm_t_raw(const uint16_t* x, const uint16_t* w, int w_packed, 
   if (M < 0 || N < 0 || K < 0 || K % 8 != 0 || N % 8 != 0 || num_cus <= 0) return G16_E_SHAPE;
   if (M == 0 || N == 0) return G16_OK;
   if (out == nullptr || x == nullptr || w == nullptr) return G16_E_NULL;
-  if (g16_mm_t_raw_route(M, N, K, num_cus) == 0) return G16_E_SHAPE;
+  if (!g16::raw_able(g16::choose_tile(M, N, K, num_cus), K, g16_hgemm_plan(M, N, K, num_cus))) return G16_E_SHAPE;
   return g16::gemm_launch(x, w, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus, nullptr, 0, nullptr, 0, stream,
                           false, w_packed != 0, nullptr, nullptr, false, true);
 }
@@ -2323,7 +2335,9 @@ extern "C" int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, 
   if (M == 0 || N == 0) return G16_OK;
   if (out == nullptr || x == nullptr || w == nullptr) return G16_E_NULL;
   const int texp = g16::thresh_exponent(thresh);
-  if (!g16::direct_thresh(texp) || g16_mm_t_direct_route(M, N, K, num_cus) == 0) return G16_E_SHAPE;
+  if (!g16::direct_thresh(texp) ||
+      !g16::direct_able(g16::choose_tile(M, N, K, num_cus), N, K, g16_hgemm_plan(M, N, K, num_cus), num_cus))
+    return G16_E_SHAPE;
   if (!g16::aligned16(x)) return G16_E_ALIGN;
   const g16::ResidentCast rc{x, 1, texp};
   return g16::gemm_launch(nullptr, w, out, out_is_f16 != 0, bias, nullptr, M, N, K, 1, num_cus, nullptr, 0, nullptr, 0,

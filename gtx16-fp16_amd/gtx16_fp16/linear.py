@@ -281,8 +281,8 @@ class FastLinear(nn.Module):
             # 88.7 -> 83.4), and loses below, up to 4 % (777 x 3072 x 8192 57.0 -> 59.5, 2086 x 3728 x 3072 76.7 ->
             # 79.4): there it serves them only where it lets layers share one cast.
             if self.prepack_weight and M > SKINNY_MAX_M:
-                raw, prepacked = _gemm_route(_clib.load(), M, self.out_features, self.in_features, x2.device)[6:]
-                if prepacked and (raw or M >= self.out_features or self.share_cast):
+                cols = _gemm_route(_clib.load(), M, self.out_features, self.in_features, x2.device)[7]
+                if cols == 256 or (cols and (M >= self.out_features or self.share_cast)):
                     wp = self._packed_weight()
             if wp is not None:
                 y = mm_t_prepacked(x2, self.weight_t, wp, b, odt, _cast_source=x if self.share_cast else None)

@@ -5,6 +5,7 @@ the kernels behind it are the gfx950 ones of libg16.so.
 """
 from __future__ import annotations
 
+import ctypes
 import weakref
 
 import torch
@@ -97,23 +98,26 @@ def _gemm_route(lib, M: int, N: int, K: int, dev: torch.device) -> tuple:
     """(route, scratch bytes, ksplit, split workspace bytes, split counter bytes, direct, raw, prepacked)
     of the GEMM path for this shape: the plan g16_mm_t_gemm follows for the same compute-unit count;
     direct: fp32 activations run as one launch that casts them itself (g16_mm_t_direct); raw: fp16
-    activations as one launch that needs no cast (g16_mm_t_raw); prepacked: a prepacked weight serves
-    it (prepacked_route)."""
+    activations as one launch that needs no cast (g16_mm_t_raw); prepacked: the columns of the tile a
+    prepacked weight serves (prepacked_route), 256 or 128, else 0."""
     key = (M, N, K, dev.index or 0)
     r = _routes.get(key)
     if r is None:
         cus = _sm_count(dev)
         scratch = lib.g16_mm_t_scratch_bytes(M, N, K, cus)
         if lib.g16_hgemm_use_packed(M, N, K, cus):
+            rows, cols = ctypes.c_int(0), ctypes.c_int(0)
+            _clib.check(lib.g16_hgemm_tile(M, N, K, cus, ctypes.byref(rows), ctypes.byref(cols)), "GEMM plan")
+            pb = cols.value if lib.g16_hgemm_use_packed_b(M, N, K, cus) == 1 else 0
             r = ("packed", scratch, 1, 0, 0, lib.g16_mm_t_direct_route(M, N, K, cus) == 1,
-                 lib.g16_mm_t_raw_route(M, N, K, cus) == 1, lib.g16_hgemm_use_packed_b(M, N, K, cus) == 1)
+                 lib.g16_mm_t_raw_route(M, N, K, cus) == 1, pb)
         else:
             ksplit = lib.g16_hgemm_plan(M, N, K, cus)
             if ksplit > 1:
                 r = ("splitk", scratch, ksplit, lib.g16_hgemm_splitk_workspace_bytes(M, N, K, ksplit, cus),
-                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False, False, False)
+                     lib.g16_hgemm_splitk_counter_bytes(M, N, K, ksplit, cus), False, False, 0)
             else:
-                r = ("plain", scratch, 1, 0, 0, False, False, False)
+                r = ("plain", scratch, 1, 0, 0, False, False, 0)
         _remember(key, r)
     return r
 
@@ -173,7 +177,7 @@ def mm_t(x2d: torch.Tensor, w_t: torch.Tensor, bias: torch.Tensor | None = None,
     reduction. Where one launch reads x itself, values are rounded at least as finely: large fp32
     batches into at most 1024 columns, and fp32 batches on the small tiles (9 to 64 rows, and more
     where it is the faster form), scale only rows that leave fp16's range, 65504; large fp16 batches
-    (256x256 tiles) are multiplied as they are and nothing is rounded."""
+    (most on 256x256 tiles) are multiplied as they are and nothing is rounded."""
     if out_dtype not in (torch.float32, torch.float16):
         raise ValueError(f"out_dtype must be float32 or float16, got {out_dtype}")
     _check_operands(x2d, w_t, bias)
@@ -251,7 +255,7 @@ def _direct(lib, x2d: torch.Tensor, w: torch.Tensor, packed: int, out: torch.Ten
 def prepacked_route(M: int, N: int, K: int, device: torch.device) -> bool:
     """True where mm_t takes the tile-packed route on the 256x256 or 256x128 tile, the ones a prepacked
     weight serves."""
-    return _gemm_route(_clib.load(), M, N, K, device)[7]
+    return _gemm_route(_clib.load(), M, N, K, device)[7] != 0
 
 
 def pack_weight(w_t: torch.Tensor) -> torch.Tensor:

@@ -173,9 +173,10 @@ int g16_mm_t_spec_history(void* stream);
  * reference. */
 int g16_mm_t_spec_paused(const uint16_t* w_t, void* stream);
 
-/* mm_t's GEMM path for fp32 activations in one launch and without scratch, where
- * g16_mm_t_direct_route() is 1 (0 elsewhere; g16_mm_t_direct then returns G16_E_SHAPE): the GEMM reads
- * x itself and casts it in registers on the way into LDS. `w` is w_t [K,N], or, with w_packed != 0,
+/* mm_t's GEMM path for fp32 activations in one launch and without scratch, where the plan is the
+ * unsplit 256x256 tile with N <= 1024, K <= 2^20 and tiles for three quarters of num_cus (elsewhere
+ * G16_E_SHAPE); g16_mm_t_direct_route() is 1 where it is measured to be the faster form, which is
+ * where g16_mm_t_gemm uses it, else 0: the GEMM reads x itself and casts it in registers on the way into LDS. `w` is w_t [K,N], or, with w_packed != 0,
  * its packed form (g16_pack_weight). A row whose values all fit fp16 is cast as it is; a row with a
  * larger value is scaled by a power of two from that value on (its sums so far are scaled with it),
  * by the rule of g16_rowscale_f32 for a threshold of 4 to 2^15 (others: G16_E_SHAPE) applied to the
@@ -186,8 +187,9 @@ int g16_mm_t_direct_route(int M, int N, int K, int num_cus);
 int g16_mm_t_direct(const float* x, const uint16_t* w, int w_packed, void* out, int out_is_f16,
                     const float* bias, float thresh, int M, int N, int K, int num_cus, void* stream);
 
-/* mm_t's GEMM path for fp16 activations in one launch and without scratch, where g16_mm_t_raw_route()
- * is 1 (0 elsewhere; g16_mm_t_raw then returns G16_E_SHAPE): the GEMM multiplies x as it is, rounding
+/* mm_t's GEMM path for fp16 activations in one launch and without scratch, where the plan is the
+ * unsplit 256x256 tile (elsewhere G16_E_SHAPE); g16_mm_t_raw_route() is 1 where it is measured to be
+ * the faster form, which is where g16_mm_t_gemm uses it, else 0: the GEMM multiplies x as it is, rounding
  * nothing, where the rowscale cast would scale rows past the threshold. The results are the same bits
  * unless a scaled value falls below fp16's normal range; a row that holds an infinity gives NaN, as
  * after the cast. `w` as for g16_mm_t_direct. */

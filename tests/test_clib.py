@@ -255,6 +255,13 @@ def test_raw_route_rule_and_refusals(lib):
     assert r(4096, 4096, 4096, 256) == 1 and r(65536, 768, 768, 256) == 1 and r(8192, 2048, 2048, 256) == 1
     assert r(2048, 4096, 4096, 256) == 0 and r(777, 8192, 3072, 256) == 0 and r(64, 1024, 1024, 256) == 0
     assert r(0, 768, 768, 256) == 0 and r(65536, 768, 768, 0) == 0 and r(65536, 768, 0, 256) == 0
+    # rows that are no whole 64-byte pieces: up to 4 tile columns at any K, up to 20 to K = 1048, else 520
+    for M, N, K, want in [(4096, 4096, 4104, 0), (4096, 4096, 4128, 1), (7314, 1208, 10184, 0), (13921, 952, 8280, 1),
+                          (5000, 4096, 1048, 1), (5000, 4096, 1304, 0), (4000, 5000, 1000, 1), (2048, 8192, 520, 1),
+                          (2048, 8192, 552, 0), (2048, 8192, 544, 1), (16384, 1024, 4104, 1)]:
+        assert r(M, N, K, 256) == want, (M, N, K)
+    # (taken where the rule says 0 as well: this call fails for its alignment, not for its shape)
+    assert d(A + 4, A, 0, A, 0, None, 4096, 4096, 4104, 256, None) == -2
     assert d(A, A, 0, A, 0, None, 2048, 4096, 4096, 256, None) == -1
     assert d(A, A, 0, A, 0, None, 65536, 768, 772, 256, None) == -1
     assert d(A + 4, A, 0, A, 0, None, 65536, 768, 768, 256, None) == -2
@@ -282,6 +289,8 @@ def test_direct_route_rule_and_refusals(lib):
                           (65536, 768, 768, 1), (65536, 1024, 768, 1), (65536, 1016, 1024, 0), (49152, 1000, 768, 1)]:
         assert r(M, N, K, 256) == want, (M, N, K)
     d = lib.g16_mm_t_direct
+    # (taken where the rule says 0 as well: this call fails for its alignment, not for its shape)
+    assert d(A + 4, A, 0, A, 0, None, 1024.0, 22000, 1024, 2000, 256, None) == -2
     assert d(A, A, 0, A, 0, None, 1024.0, 4096, 4096, 4096, 256, None) == -1
     assert d(A, A, 0, A, 0, None, 65536.0, 65536, 768, 768, 256, None) == -1    # threshold past 2^15
     assert d(A, A, 0, A, 0, None, 2.0, 65536, 768, 768, 256, None) == -1        # threshold below 4

@@ -114,3 +114,32 @@ def test_medium_batches_with_and_without_scratch(cuda, M, K, N, kind):
             assert (err <= 2.0 ** -10).all(), err.max()
             if kind != "outliers":
                 assert torch.equal(out[fin], y[fin])
+
+
+@pytest.mark.parametrize("M,K,N,raw", [(4096, 4104, 4096, False), (4096, 4128, 4096, True), (5000, 1048, 4096, True),
+                                       (16384, 4104, 1024, True)])
+@pytest.mark.parametrize("share", [False, True])
+def test_raw_route_by_its_rounding(cuda, M, K, N, raw, share):
+    # a row with |max| 2000 is halved by the rowscale cast, and 3 * 2^-24 with it (to 2 * 2^-24, a tie to
+    # even); the raw launch rounds nothing. mm_t, the layer on its prepacked weight and, on every such
+    # shape, the raw entry point itself
+    import torch.nn as nn
+
+    import gtx16_fp16 as g
+    from gtx16_fp16 import _clib
+
+    if torch.cuda.get_device_properties(cuda).multi_processor_count != 256:
+        pytest.skip("the shapes are for 256 CUs")
+    x = torch.zeros(M, K, dtype=torch.float16, device=cuda)
+    x[M - 1, 0], x[M - 1, K - 1] = 2000.0, 3 * 2.0 ** -24
+    fl = g.FastLinear.from_linear(nn.Linear(K, N, bias=False).to(cuda))
+    fl.share_cast = share
+    fl.weight_t.zero_()
+    fl.weight_t[K - 1] = 1.0
+    for y in (g.mm_t(x, fl.weight_t), fl(x)):
+        assert (y[M - 1] == (3 if raw else 4) * 2.0 ** -24).all() and not y[:-1].any()
+    assert fl._wp is not None
+    y = torch.full((M, N), 7.0, device=cuda)
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    assert _clib.load().g16_mm_t_raw(x.data_ptr(), fl.weight_t.data_ptr(), 0, y.data_ptr(), 0, None, M, N, K, 256, st) == 0
+    assert (y[M - 1] == 3 * 2.0 ** -24).all() and not y[:-1].any()
