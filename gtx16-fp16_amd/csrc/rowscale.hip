@@ -7,7 +7,8 @@
 // Layout: one 64-lane wavefront per row, 4 rows per 256-thread workgroup. Each lane keeps up to
 // CH 16-byte chunks of its row in registers, so the row is read from HBM once: max-reduce across
 // the wavefront (no LDS, no barrier), then scale, convert and store from the registers. Longer rows
-// (K > 4096), and the rows of small batches, get a workgroup each.
+// (K > 4096, but not large packed batches a little past that), and the rows of small batches, get a
+// workgroup each.
 //
 // Output layouts: row-major y[M,K], or the tile-packed layout the 256x256 GEMM streams (see
 // packed_offset in g16_common.hpp): every 256-row x 32-column block of y is one contiguous 16 KB
@@ -45,7 +46,8 @@ __device__ inline _Float16* out_at(_Float16* Y, int row, int K, int idx, int nks
   }
 }
 
-template <typename TX, int CH, bool PACK>
+// LONG: rows of more than 64 * CH chunks, whose remainder streams twice (the second read hits L2).
+template <typename TX, int CH, bool PACK, bool LONG = false>
 __global__ __launch_bounds__(256) void rowscale_kernel(const TX* __restrict__ X, _Float16* __restrict__ Y,
                                                        float* __restrict__ S, int M, int K, int texp) {
   constexpr int EPC = 16 / static_cast<int>(sizeof(TX));  // elements per 16-byte chunk
@@ -78,6 +80,9 @@ __global__ __launch_bounds__(256) void rowscale_kernel(const TX* __restrict__ X,
   }
 #pragma unroll
   for (int c = 0; c < CH; ++c) amax = chunk_absmax(amax, buf[c], TX{});
+  if constexpr (LONG) {
+    for (int idx = lane + CH * kWave; idx < nch; idx += kWave) amax = chunk_absmax(amax, xr[idx], TX{});
+  }
 #pragma unroll
   for (int off = kWave / 2; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
 
@@ -89,6 +94,10 @@ __global__ __launch_bounds__(256) void rowscale_kernel(const TX* __restrict__ X,
   for (int c = 0; c < CH; ++c) {
     const int idx = lane + c * kWave;
     if (idx < nch) store_scaled(out_at<TX, PACK>(Y, row, K, idx, nks), buf[c], e, TX{});
+  }
+  if constexpr (LONG) {
+    for (int idx = lane + CH * kWave; idx < nch; idx += kWave)
+      store_scaled(out_at<TX, PACK>(Y, row, K, idx, nks), xr[idx], e, TX{});
   }
   if (lane == 0) S[row] = sc;
 }
@@ -206,6 +215,13 @@ int rowscale_launch(const void* X, void* Y, float* S, int M, int K, float thresh
   // fp32): 80 x 2048 3.06 -> 2.58, 333 x 4096 4.39 -> 3.86, 80 x 11008 16.9 -> 3.6, 777 x 8192 14.8 -> 8.3,
   // 8192 x 8192 99 -> 74 (fp16 62 -> 42; packed 103 -> 89 and 71 -> 52); with more short rows the
   // wavefronts are the faster ones (2048 x 256 3.0 vs 3.3, 8192 x 1024 10.6 vs 11.5).
+  // Packed rows a little past K = 4096 in large batches keep a wavefront each, which reads little of a row
+  // twice (4096 rows packed, wavefront and workgroup per row, us: fp16 K = 4104 14.1, 18.0, 5120 19.5, 20.6,
+  // 6144 22.8, 23.6, 7168 27.1, 26.9; but 20000 x 5120 97, 93. fp32 20000 x 4104 98, 105, 20000 x 5120 132,
+  // 137, 2048 x 4608 12.3, 13.1, 4096 x 6144 32.4, 30.1). Row-major ones gain from the workgroup at once.
+  if (PACK && K > kWave * CH * EPC && (EPC == 8 ? M >= 4096 && K <= 6400 : M >= 2048 && K <= 5120))
+    return launch(rowscale_kernel<TX, CH, PACK, PACK>, dim3(ceil_div(rows, kRowsPerBlock)), dim3(256),
+                  static_cast<hipStream_t>(stream), static_cast<const TX*>(X), static_cast<_Float16*>(Y), S, M, K, texp);
   if (K > kWave * CH * EPC || M <= kWideMaxM) {
     auto fn = K > kWave * CH * EPC ? rowscale_wide_kernel<TX, CH, PACK> : rowscale_wide_kernel<TX, CH / 4, PACK>;
     return launch(fn, dim3(rows), dim3(256), static_cast<hipStream_t>(stream), static_cast<const TX*>(X),

@@ -103,3 +103,33 @@ def test_rowscale_of_short_rows_past_one_launch(cuda, packed):
     assert np.array_equal(got.cpu().numpy().view(np.uint16), want.view(np.uint16))
     assert np.array_equal(s[rows].cpu().numpy(), S.astype(np.float32))
     assert int((s == 1.0).sum()) == M - len(rows) and int((y != 0).sum()) == len(rows)
+
+
+@pytest.mark.parametrize("M,K,dt", [(2048, 4104, torch.float32), (2053, 5120, torch.float32), (2053, 5128, torch.float32),
+                                    (4096, 4104, torch.float16), (4100, 6400, torch.float16), (4100, 6408, torch.float16)])
+def test_packed_rows_a_little_past_4096(cuda, M, K, dt):
+    # a wavefront per row with a remainder past its registers, and a workgroup per row just beyond the rule:
+    # bit-exact against the oracle on a few rows, and the packed bytes those of the row-major cast
+    from gtx16_fp16 import _clib
+
+    lib = _clib.load()
+    x = randn((M, K), seed=M + K)
+    x[5] *= 5000.0 if dt == torch.float32 else 500.0
+    x[7, K - 1], x[M - 1, 4100] = 6e4, 3e4  # a row's only large value, past the registers
+    x[9] = 0.0
+    x = x.to(dt)
+    xd = x.to(cuda)
+    st = torch.cuda.current_stream(cuda).cuda_stream
+    name = "f32" if dt == torch.float32 else "f16"
+    y = torch.empty(M, K, dtype=torch.float16, device=cuda)
+    s, sp = torch.empty(M, device=cuda), torch.empty(M, device=cuda)
+    yp = torch.full((lib.g16_packed_a_bytes(M, K) // 2,), 7.0, dtype=torch.float16, device=cuda)
+    assert getattr(lib, f"g16_rowscale_{name}")(xd.data_ptr(), y.data_ptr(), s.data_ptr(), M, K, 1024.0, st) == 0
+    assert getattr(lib, f"g16_rowscale_pack_{name}")(xd.data_ptr(), yp.data_ptr(), sp.data_ptr(), M, K, 1024.0, st) == 0
+    torch.cuda.synchronize()
+    rows = [0, 5, 7, 9, 255, 256, M - 1]
+    want, S, _ = oracle.rowscale(x[rows].numpy())
+    assert np.array_equal(y[rows].cpu().numpy().view(np.uint16), want.view(np.uint16))
+    assert np.array_equal(sp[rows].cpu().numpy(), S.astype(np.float32)) and torch.equal(s, sp)
+    pw = pack_a(y.cpu().numpy()).reshape(-1)
+    assert np.array_equal(yp.cpu().numpy().view(np.uint16), pw.view(np.uint16))
